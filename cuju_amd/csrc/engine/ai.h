@@ -29,7 +29,7 @@ HD float ClampVelocity(float v) {
 }
 
 // Gets the point at `self` clamped into the angular sector from `first` to `second`.
-HDN Vec3 GetClamped2D(const Vec3 &self, const Vec3 &first, const Vec3 &second) {
+HDN Vec3 GetClamped2D(Vec3 self, Vec3 first, Vec3 second) {
     int dir = SignSide(second.Angle2D(first));
     float a1 = self.Angle2D(first), a2 = self.Angle2D(second);
     if (SignSide(a1) != dir || SignSide(a2) == dir) return fabsf(a1) < fabsf(a2) ? first : second;
@@ -55,7 +55,8 @@ HD bool NeedDefendingMovement(int side, const Vec3 &pos, const Vec3 &target) {
 // GRF: a player missing from the mental image gets the image's first entry.
 // The first entry of player `p` is found eight entries at a time: a batch's player numbers load
 // together, and the lowest matching index wins.
-HDN PlayerImage MentalPlayerImage(const World &w, int k, int p) {
+HDN PlayerImage MentalPlayerImage(GlobalRef<const World> world, int k, int p) {
+    const World &w = world;
     const MentalImage &mi = w.match.mentalImages[k];
     const int age = (int)(w.match.actualTimeMs - (uint64_t)mi.timeStampMs);
     const int count = mi.players.count;
@@ -79,7 +80,8 @@ HDN PlayerImage MentalPlayerImage(const World &w, int k, int p) {
     }
     return count > 0 ? MentalImageEntry(w, mi, 0) : mi.players[0];
 }
-HDN float PlayerAverageVelocity(const World &w, int p, float periodS) {
+HDN float PlayerAverageVelocity(GlobalRef<const World> world, int p, float periodS) {
+    const World &w = world;
     const auto &hist = w.match.players[p].base.positionHistoryPerSecond;
     unsigned n = hist.count;
     if (n == 0) return 0;
@@ -200,7 +202,9 @@ HD Vec3 PullTowardMicro(const Vec3 &pos, const Vec3 &unpulled, const Placement &
 // Player p's place by a placement: its static (or dynamic) formation position squeezed toward
 // the midfield line, mapped into the block (y mirrored for the side), then pulled toward the x, y
 // and micro foci.
-HDN Vec3 PlaceInFormation(const World &w, const Ctx &c, int p, const Placement &r, bool dynamic) {
+HDN Vec3 PlaceInFormation(GlobalRef<const World> world, LocalRef<const Ctx> context, int p, const Placement &r, bool dynamic) {
+    const World &w = world;
+    const Ctx &c = context;
     const int side = TeamDynamicSide(w, w.playerTeamID[p]);
     Vec3 pos = dynamic ? w.match.players[p].dynamicFormationEntry.position : Formation(w, c, p).position;
     if (r.midFocusStrength > 0.0f) pos.v[0] = StretchTowardMidfield(pos.v[0], r.midFocus, r.midFocusStrength);
@@ -221,7 +225,8 @@ struct FormationHistory {
     Vec3 ball[4];
     float possessionSide;
 };
-HDN FormationHistory FormationHistoryOf(const World &w, int p) {
+HDN FormationHistory FormationHistoryOf(GlobalRef<const World> world, int p) {
+    const World &w = world;
     const Vec3 focal = Sp(w, w.match.designatedPossessionPlayer).position;
     const float urgency = 1.0f - NormalizedClamp((focal - Sp(w, p).position).Length(), 2.0f, 30.0f);
     const unsigned durations[4] = {TruncToUint32(3500 * (1.0f - urgency * 0.7f)), TruncToUint32(4000 * (1.0f - urgency * 0.5f)),
@@ -316,7 +321,9 @@ HD void TeamMicroFocus(const RoleTactics &t, float share, int side, float ballX,
 // (stronger attacking), the micro focus around the play (the 3 s ball average attacking; the 2 s
 // average halfway to the designated player defending), and a midfield focus from the tactics
 // (70%) and the ball (30%). Clamped to the pitch.
-HDN Vec3 TeamAdaptedFormationPosition(const World &w, const Ctx &c, int p, bool dynamic, const FormationHistory &history) {
+HDN Vec3 TeamAdaptedFormationPosition(GlobalRef<const World> world, LocalRef<const Ctx> context, int p, bool dynamic, const FormationHistory &history) {
+    const World &w = world;
+    const Ctx &c = context;
     const int side = TeamDynamicSide(w, w.playerTeamID[p]);
     const TeamAI &ai = TeamByID(w, w.playerTeamID[p]).ai;
     const MatchState &m = w.match;
@@ -348,7 +355,8 @@ HD Vec3 TeamAdaptedFormationPosition(const World &w, const Ctx &c, int p, bool d
 }
 
 // Pulls a position in front of the trap line back into a 4 m band around it.
-HDN void TeamApplyOffsideTrap(const World &w, int teamID, Vec3 &pos) {
+HDN void TeamApplyOffsideTrap(GlobalRef<const World> world, int teamID, Vec3 &pos) {
+    const World &w = world;
     const int side = TeamDynamicSide(w, teamID);
     const float trap = TeamByID(w, teamID).ai.offsideTrapX;
     const float half = 2.0f;

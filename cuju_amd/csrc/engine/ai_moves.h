@@ -11,46 +11,78 @@
 namespace eng {
 
 struct AIBase {
-    World &w;
-    const Ctx &c;
+    GlobalRef<World> world;
+    LocalRef<const Ctx> context;
     const int p;
-    MatchState &m;
-    Player &ps;
-    AIControllerState *eliza;  // null under a gamer
-    PlayerControllerState &ctl;
+    GlobalPointer<AIControllerState> elizaState;  // null under a gamer
+    GlobalRef<PlayerControllerState> controller;
     const int teamID, oppID, side;  // `side`: the sign of x of the own goal
     int k = 0;                      // mental image
-    CommandQueue &q;
+    GlobalRef<CommandQueue> queue;
 
-    HD AIBase(World &world, const Ctx &ctx, int player, CommandQueue &queue, PlayerControllerState &controller,
-              AIControllerState *e)
-        : w(world),
-          c(ctx),
+    HD AIBase(World &w, const Ctx &c, int player, CommandQueue &q, PlayerControllerState &ctl, AIControllerState *e)
+        : world(w),
+          context(c),
           p(player),
-          m(world.match),
-          ps(world.match.players[player]),
-          eliza(e),
-          ctl(controller),
-          teamID(world.playerTeamID[player]),
-          oppID(1 - world.playerTeamID[player]),
-          side(TeamDynamicSide(world, world.playerTeamID[player])),
-          q(queue) {}
+          elizaState(e),
+          controller(ctl),
+          teamID(w.playerTeamID[player]),
+          oppID(1 - w.playerTeamID[player]),
+          side(TeamDynamicSide(w, w.playerTeamID[player])),
+          queue(q) {}
 
-    HD Vec3 Pos(int o) const { return Sp(w, o).position; }
-    HD Vec3 Mov(int o) const { return Sp(w, o).movement; }
-    HD Vec3 Dir(int o) const { return Sp(w, o).directionVec; }
+    HD Vec3 Pos(int o) const {
+        World &w = world;
+        return Sp(w, o).position;
+    }
+    HD Vec3 Mov(int o) const {
+        World &w = world;
+        return Sp(w, o).movement;
+    }
+    HD Vec3 Dir(int o) const {
+        World &w = world;
+        return Sp(w, o).directionVec;
+    }
     HD Vec3 Pos() const { return Pos(p); }
     HD Vec3 Mov() const { return Mov(p); }
     HD Vec3 Dir() const { return Dir(p); }
-    HD float FloatVelocity() const { return PlayerFloatVelocity(w, p); }
-    HD float Stat(int s) const { return GetStatistic(w, c, p, s); }
-    HD int StaticRole(int o) const { return Formation(w, c, o).role; }
-    HD int DynamicRole() const { return ps.dynamicFormationEntry.role; }
-    HD const Team &Own() const { return TeamByID(w, teamID); }
-    HD const Team &Opp() const { return TeamByID(w, oppID); }
+    HD float FloatVelocity() const {
+        World &w = world;
+        return PlayerFloatVelocity(w, p);
+    }
+    HD float Stat(int s) const {
+        World &w = world;
+        const Ctx &c = context;
+        return GetStatistic(w, c, p, s);
+    }
+    HD int StaticRole(int o) const {
+        World &w = world;
+        const Ctx &c = context;
+        return Formation(w, c, o).role;
+    }
+    HD int DynamicRole() const {
+        World &w = world;
+        Player &ps = w.match.players[p];
+        return ps.dynamicFormationEntry.role;
+    }
+    HD const Team &Own() const {
+        World &w = world;
+        return TeamByID(w, teamID);
+    }
+    HD const Team &Opp() const {
+        World &w = world;
+        return TeamByID(w, oppID);
+    }
     HD const TeamAI &AI() const { return Own().ai; }
-    HD Vec3 MentalBall(int ms) const { return MentalBallPrediction(w, k, ms); }
-    HD Vec3 BallAt(int ms) const { return BallPredict(m.ball, ms); }
+    HD Vec3 MentalBall(int ms) const {
+        World &w = world;
+        return MentalBallPrediction(w, k, ms);
+    }
+    HD Vec3 BallAt(int ms) const {
+        World &w = world;
+        MatchState &m = w.match;
+        return BallPredict(m.ball, ms);
+    }
 
     // How likely the player is to win a duel for the ball with the opponents' designated player
     // (both 0.1 s ahead): 1 when the opponent stands between it and the ball seen 100 ms ahead
@@ -69,6 +101,9 @@ struct AIBase {
     // least 0.4 m from where it is), held to the offside trap. Returns its distance from the
     // opponent in `reach`.
     HD Vec3 ShootingPoint(int o, const Vec3 &goal, float &reach) const {
+        World &w = world;
+        const Ctx &c = context;
+        MatchState &m = w.match;
         const PlayerImage oi = MentalPlayerImage(w, MentalImageIndex(w, PlayerControllerReactionTime(w, c, p)), o);
         const Vec3 op = oi.position + oi.movement * 0.5f;
         const float range = o == m.designatedPossessionPlayer ? 24.0f : 8.0f;
@@ -87,6 +122,9 @@ struct AIBase {
     // for outfield players: to within the opponent's reach of its shooting point less a 4 m
     // buffer, then goalside by 70% of however far the player (0.14 s ahead) is beyond that reach.
     HDN void AddDefensiveComponent(Vec3 &desired, float bias, int forcedOpp = -1) const {
+        World &w = world;
+        MatchState &m = w.match;
+        Player &ps = w.match.players[p];
         const int o = forcedOpp < 0 ? ps.manMarking : forcedOpp;
         if (!(m.inPlay && !m.inSetPiece && StaticRole(p) != kRoleGoalkeeper)) return;
         if (o < 0) return;
@@ -107,6 +145,7 @@ struct AIBase {
     // where the perpendicular bisector of the player and the opponent crosses it (within the
     // line), plus a tenth of a sprint second and `distance` toward goal and its movement 0.14 s on.
     HDN Vec3 GetDefendPosition(int o, float distance = 0.0f) const {
+        World &w = world;
         const PlayerImage oi = MentalPlayerImage(w, k, o);
         const Vec3 goal = Vec3(kPitchHalfLength * side, 0, 0);
         const Vec3 op = oi.position;
@@ -128,6 +167,8 @@ struct AIBase {
     // threshold in 400 ms, free, in its penalty box in 160 ms (compared in double), and not a
     // teammate's kick (a back pass).
     HD bool BallSaveable() const {
+        World &w = world;
+        MatchState &m = w.match;
         if (GetDistance(BallAt(400), Pos()) > kBallDistanceOptimizeThreshold + 10.0f) return false;
         if (m.lastTouchTeamID == teamID && MatchLastTouchPlayer(w) != p && m.lastTouchTeamIDs[kTouchKicked] == teamID) return false;
         if (m.ballRetainer >= 0) return false;
@@ -136,6 +177,7 @@ struct AIBase {
     }
     // A goalkeeper's deflection (only those that pick the ball up, on request) of a saveable ball.
     HDN void KeeperDeflectCommand(bool onlyPickup) {
+        CommandQueue &q = queue;
         if (StaticRole(p) != kRoleGoalkeeper || !BallSaveable()) return;
         PlayerCommand cmd = DefaultPlayerCommand();
         cmd.desiredFunctionType = kFnDeflect;
@@ -145,6 +187,10 @@ struct AIBase {
     // Waiting at a set piece: standing, facing on; looking at the ball, or, for the retainer,
     // along its input.
     HDN void SetPieceCommand() {
+        World &w = world;
+        MatchState &m = w.match;
+        PlayerControllerState &ctl = controller;
+        CommandQueue &q = queue;
         PlayerCommand cmd = DefaultPlayerCommand();
         cmd.useDesiredMovement = true;
         cmd.useDesiredLookAt = true;
@@ -155,10 +201,15 @@ struct AIBase {
     }
     // ---- touch commands: each a guard, then a command from the input ----
     // The ball free and near (within the optimization threshold of where it will be in 200 ms).
-    HD bool BallFreeAndNear() const { return !(GetDistance(BallAt(200), Pos()) > kBallDistanceOptimizeThreshold) && m.ballRetainer < 0; }
+    HD bool BallFreeAndNear() const {
+        World &w = world;
+        MatchState &m = w.match;
+        return !(GetDistance(BallAt(200), Pos()) > kBallDistanceOptimizeThreshold) && m.ballRetainer < 0;
+    }
     // A command of `fn` along the input (snapped to 8 directions with no bias when `snap`), at the
     // input's speed; an idle input turns to the opponents' goal on request.
     HD PlayerCommand InputCommand(int fn, bool snap, bool idleTurnToGoal) const {
+        PlayerControllerState &ctl = controller;
         PlayerCommand cmd = DefaultPlayerCommand();
         cmd.desiredFunctionType = fn;
         cmd.useDesiredMovement = true;
@@ -175,6 +226,11 @@ struct AIBase {
     // body direction, walking.
     HDN void BallControlCommand(bool idleTurnToGoal = false, bool knockOn = false, bool stickyRun = false,
                                 bool keepBodyDirection = false) {
+        World &w = world;
+        MatchState &m = w.match;
+        Player &ps = w.match.players[p];
+        PlayerControllerState &ctl = controller;
+        CommandQueue &q = queue;
         if (!BallFreeAndNear()) return;
         if (!ps.hasPossession && !AllowLastDitchOf(w, p)) {
             const float strictnessInverse = 3.0f;
@@ -208,6 +264,11 @@ struct AIBase {
     // opponents need 400 ms more, do not hold it and are half likely to lose the duel. An AI
     // goalkeeper traps facing upfield, standing.
     HDN void TrapCommand(bool idleTurnToGoal = false, bool knockOn = false) {
+        World &w = world;
+        MatchState &m = w.match;
+        Player &ps = w.match.players[p];
+        PlayerControllerState &ctl = controller;
+        CommandQueue &q = queue;
         if (m.ball.momentum.Get2D().Length() < 2.0f || !BallFreeAndNear() || ctl.hasPossession) return;
         if (!(m.designatedPossessionPlayer == p ||
               (Own().designatedTeamPossessionPlayer == p && ps.timeToBallOptimisticMs < 1000 && ctl.oppTimeNeededToGetToBall > 400 &&
@@ -227,6 +288,8 @@ struct AIBase {
     // Interference when the team is not best placed: by any means (loosely), or strictly when at
     // least 20% likely to win the duel.
     HDN void InterfereCommand(bool byAnyMeans) {
+        PlayerControllerState &ctl = controller;
+        CommandQueue &q = queue;
         if (!BallFreeAndNear() || ctl.teamHasBestPossession) return;
         if (!byAnyMeans && CouldWinABallDuelLikeliness() < 0.2f) return;
         PlayerCommand cmd = InputCommand(kFnInterfere, false, false);
@@ -239,6 +302,10 @@ struct AIBase {
     // needing more than 260 ms to it), or 0.6 to 1.8 m from it while their player winds up a shot.
     // It sprints at the ball, led by the opponent's movement.
     HDN void SlidingCommand() {
+        World &w = world;
+        MatchState &m = w.match;
+        PlayerControllerState &ctl = controller;
+        CommandQueue &q = queue;
         if (HumanGamerCount(Own()) != 0 || m.ballRetainer >= 0 || CouldWinABallDuelLikeliness() < 0.7f) return;
         if (!(!ctl.teamHasBestPossession && ctl.possessionAmount < 0.6f && m.designatedPossessionPlayer != p && ctl.oppTeamHasPossession))
             return;
@@ -267,6 +334,8 @@ struct AIBase {
     // held up to 8 m/s above it and eased 10% toward (90% up to) the nearest velocity category.
     // Returns the player's time to the ball.
     HDN unsigned BallControlMovement(float desiredVel, Vec3 &bestDir, float &bestVel, Vec3 &bestLookAt) const {
+        World &w = world;
+        Player &ps = w.match.players[p];
         ENG_SCOPE(47);
         const Vec3 toBall = MentalBall((int)(250 + kDefaultTouchOffsetMs)).Get2D() - Pos();
         const float dist = toBall.Length();
@@ -341,8 +410,11 @@ struct AIBase {
     // time); a point off the pitch, or one reached while the ball comes toward the player or far
     // earlier than its time to the ball, ends the scan. Returns the chosen time (the span's end
     // without one), with the direction, speed and look-at of the chase.
-    HDN unsigned ToBallMovement(const Vec3 &desiredDir, float desiredVel, Vec3 &bestDir, float &bestVel, Vec3 &bestLookAt,
+    HDN unsigned ToBallMovement(Vec3 desiredDir, float desiredVel, Vec3 &bestDir, float &bestVel, Vec3 &bestLookAt,
                                 float haste) const {
+        World &w = world;
+        const Ctx &c = context;
+        Player &ps = w.match.players[p];
         ENG_SCOPE(39);
         const Vec3 pp = Pos();
         const float maxVel = GetMaximumVelocity(*c.sd, p);
@@ -415,6 +487,7 @@ struct AIBase {
     // 40 ms (half a metre ahead of it), fully when slow, 30% less (to the 0.5, then the 0.7) at a
     // sprint.
     HD Vec3 InputLook(const Vec3 &manualDir) const {
+        PlayerControllerState &ctl = controller;
         const float slow =
             1.0f - libm::powf(NormalizedClamp(MinF(ctl.inputVelocityFloat, FloatVelocity()), kIdleDribbleSwitch, kSprintVelocity), 0.5f) *
                        0.3f;
@@ -427,6 +500,9 @@ struct AIBase {
     // designated player with its team holding the ball (possession over 0.5 after a recent touch
     // of its own or with the opponents off it, over 0.99, or its own best possession).
     HD bool GoesForBall(bool forceMagnet) const {
+        World &w = world;
+        MatchState &m = w.match;
+        PlayerControllerState &ctl = controller;
         const int teamDesignated = Own().designatedTeamPossessionPlayer;
         const float poss = ctl.possessionAmount;
         return forceMagnet || m.designatedPossessionPlayer == p ||
@@ -440,6 +516,9 @@ struct AIBase {
     // magnet of agreement or a recent switch, by possession and less toward the own half; all of
     // it when forced.
     HD float ChaseOverride(const Vec3 &chaseDir, const Vec3 &manualDir, float ownHalf, bool forceMagnet) const {
+        World &w = world;
+        Player &ps = w.match.players[p];
+        PlayerControllerState &ctl = controller;
         float agree = 1.0f - Clamp(fabsf(chaseDir.Angle2D(manualDir)) / PI, 0.0f, 1.0f);
         agree = agree * 0.5f + 0.5f;
         float bias = 0.0f;
@@ -457,6 +536,8 @@ struct AIBase {
     // (30% of a recent switch, less toward the own half) toward shadowing the opponent (near it:
     // its movement) or hunting it (further: a point 30% of the way from it to the goal).
     HD float ShadowOpponent(float ownHalf, Vec3 &autoDir, float &autoVel, Vec3 &autoLook) const {
+        World &w = world;
+        PlayerControllerState &ctl = controller;
         const int lookMs = 40;
         const PlayerImage oi = MentalPlayerImage(w, k, ctl.opponentPlayer);
         const Vec3 op = oi.position + oi.movement * 0.14f + oi.directionVector * 0.6f;
@@ -488,6 +569,11 @@ struct AIBase {
     // going for the ball (a retainer keeps its input), or the shadowing of the opponent on the
     // ball. Below the idle-dribble switch the player faces where it looks.
     HDN void MovementCommand(bool forceMagnet, bool extraHaste) {
+        World &w = world;
+        MatchState &m = w.match;
+        Player &ps = w.match.players[p];
+        PlayerControllerState &ctl = controller;
+        CommandQueue &q = queue;
         ENG_SCOPE(40);
         Vec3 manualDir = ctl.inputDirection;
         QuantizeDirection(manualDir, kQuantizedDirectionBias);
@@ -527,6 +613,9 @@ struct AIBase {
     // from 20 m, fully at 65 m, both nearer when tired), half of it always and half by role (the
     // mindset, inverted as the team holds the ball).
     HD float Laziness() const {
+        World &w = world;
+        Player &ps = w.match.players[p];
+        PlayerControllerState &ctl = controller;
         const float fresh = ps.base.fatigueFactorInverse;
         const float from = 20.0f * (fresh * 0.8f + 0.2f), to = 65.0f * (fresh * 0.5f + 0.5f);
         const float away = (Pos() - Pos(Opp().designatedTeamPossessionPlayer)).Length();
@@ -539,6 +628,7 @@ struct AIBase {
     // player slows (not below dribbling when it asked for that) and, after running a lot in the
     // last 10 s (less with work rate), stays below a share of a sprint.
     HDN float GetLazyVelocity(float desiredVel) const {
+        World &w = world;
         float v = desiredVel;
         if (v > kSprintVelocity) v = kSprintVelocity + (v - kSprintVelocity) * 0.1f;
         const float lazy = Laziness();
@@ -594,7 +684,9 @@ struct AIBase {
     // nearest teammates; with it held better still, the ball's path 200 to 650 ms ahead; and for
     // players other than the carrier, a flock ring around it (attract to 21 m, repel within 12 m).
     // The result stays onside (8 cm) and on the pitch.
-    HDN Vec3 GetSupportPositionForceField(const Vec3 &base, bool makeRun) const {
+    HDN Vec3 GetSupportPositionForceField(Vec3 base, bool makeRun) const {
+        World &w = world;
+        const Ctx &c = context;
         ENG_SCOPE(41);
         const int designated = Own().designatedTeamPossessionPlayer;
         const Vec3 cur = Pos() + Mov() * 0.1f;
@@ -665,6 +757,10 @@ struct AIBase {
     // the line's base less its mindset and the possession; inside the offside trap except for
     // attackers. Its speed is the distance at the AI's distance-to-velocity rate, made lazy.
     HDN void FieldStrategyRequestInput(int kind, Vec3 &dir, float &vel) const {
+        World &w = world;
+        const Ctx &c = context;
+        MatchState &m = w.match;
+        PlayerControllerState &ctl = controller;
         const LineStrategy line = LineStrategyOf(kind);
         const FormationHistory history = FormationHistoryOf(w, p);
         const Vec3 fixed = TeamAdaptedFormationPosition(w, c, p, false, history);
@@ -689,6 +785,7 @@ struct AIBase {
     // within 3.7 m of the centre, widened by the keeper's panic (1.02, up to 1.52 as its
     // defensive positioning and vision fall).
     HDN bool BallBoundForGoal() {
+        AIControllerState *const eliza = elizaState;
         const float panic = 1.02f + (1.0f - (Stat(kStatDefensivePositioning) * 0.6f + Stat(kStatVision) * 0.4f)) * 0.5f;
         bool bound = false;
         float crossY = 0;
@@ -715,6 +812,10 @@ struct AIBase {
     // attacker's shooting point (24 m) is as badly covered. `path` starts where the attack comes
     // from (the opponent 0.32 s ahead, blended with the ball).
     HD float KeeperRush(const Vec3 &ball, const Vec3 &goal, Line &path) const {
+        World &w = world;
+        const Ctx &c = context;
+        MatchState &m = w.match;
+        PlayerControllerState &ctl = controller;
         float rush = 0.3f;
         rush *= NormalizedClamp(ctl.fadingTeamPossessionAmount, 1.0f, 1.5f);
         if (!(ctl.fadingTeamPossessionAmount < 1.0f)) return rush;
@@ -747,6 +848,8 @@ struct AIBase {
     // the rush (at least 0.7 m) toward where the attack comes from; walking once in front of its
     // target near that line.
     HD Vec3 KeeperCover(const Vec3 &ball, const Vec3 &goal, float &maxVel) const {
+        World &w = world;
+        MatchState &m = w.match;
         const Vec3 post1 = Vec3(kPitchHalfLength * side, 3.7f, 0) - ball;
         const Vec3 post2 = Vec3(kPitchHalfLength * side, -3.7f, 0) - ball;
         const Vec3 middle = post1.Rotated2D(post2.Angle2D(post1) * 0.5f).Normalized(Vec3(side, 0, 0));
@@ -769,6 +872,7 @@ struct AIBase {
     // line (0.4 m short), at the point nearest the keeper; at the crossing itself when the ball
     // will pass the keeper above 2.5 m.
     HD Vec3 KeeperSave() const {
+        AIControllerState *const eliza = elizaState;
         Line path;
         path.pts[0] = MentalBall(10).Get2D();
         Vec3 crossing = Vec3(kPitchHalfLength * side, eliza->ballBoundForGoalY, 0);
@@ -788,6 +892,8 @@ struct AIBase {
     // The goalkeeper's movement: 10 m off its goal line by default; with the ball (600 ms plus a
     // fifth of its time to it ahead) in its half, covering the goal or saving a ball bound for it.
     HDN void GoalieRequestInput(Vec3 &dir, float &vel) {
+        World &w = world;
+        Player &ps = w.match.players[p];
         ENG_SCOPE(46);
         const Vec3 ball = MentalBall(TruncToInt32(600 + (float)ps.timeToBallMs * 0.2f)).Get2D();
         const Vec3 goal = Vec3(kPitchHalfLength * side, 0, 0);
@@ -827,7 +933,7 @@ struct AIBase {
     }
     // The odds of a pass (or, with a ball-speed factor, a shot) to `target` from 0.12 s ahead:
     // 1 less the summed threats (a high pass starts at 0.4), clamped.
-    HDN float PassingOdds(const Vec3 &target, int passType, const ImageList &opps, float ballVelMul = 1.0f) const {
+    HDN float PassingOdds(Vec3 target, int passType, const ImageList &opps, float ballVelMul = 1.0f) const {
         ENG_SCOPE(42);
         const float secondScale = 1.0f;
         const Vec3 origin = Pos() + Mov() * 0.12f;
@@ -849,6 +955,8 @@ struct AIBase {
     }
     // A fully automatic pass of `passType` to teammate `target`.
     HDN void AddPass(int target, int passType) {
+        World &w = world;
+        CommandQueue &q = queue;
         PlayerCommand cmd = DefaultPlayerCommand();
         cmd.desiredFunctionType = passType;
         TouchInformation &t = cmd.touchInfo;
@@ -866,6 +974,7 @@ struct AIBase {
     // turned upfield and toward the touchline it faces, lifted 0.3; offered as a high pass (power
     // 0.7), a shot (0.6) and a long pass (0.8), fully manual.
     HDN void AddPanicPass() {
+        CommandQueue &q = queue;
         const int flank = SignSide(Dir().v[1]);
         Vec3 away = ((Dir() * Vec3(0.8f, 1.0f, 0.0f)).Normalized() + Vec3(-side * 0.7f, flank * 0.5f, 0)).Normalized(0) + Vec3(0, 0, 0.3f);
         away.Normalize(Dir());
@@ -892,6 +1001,8 @@ struct AIBase {
     // the dribble setting and the mindset). The speed is the pull at the AI's rate, snapped to a
     // velocity category.
     HDN void BestDribbleMovement(Vec3 &desiredDir, float &desiredVel) const {
+        World &w = world;
+        const Ctx &c = context;
         ENG_SCOPE(43);
         const Vec3 at = Pos(), mov = Mov();
         const float offense = 0.7f + kDribbleOffensiveness * 0.05f + GetMindSet(DynamicRole()) * 0.05f;

@@ -13,7 +13,10 @@ namespace eng {
 struct AIController : AIBase {
     using AIBase::AIBase;
 
-    HD float Random(float lo, float hi) { return RandomInRange(w, lo, hi); }
+    HD float Random(float lo, float hi) {
+        World &w = world;
+        return RandomInRange(w, lo, hi);
+    }
 
     HD float TacticalRating(const Player &pl, float fsw, float sw, float fw, float total) const {
         const auto &t = pl.tactical;
@@ -39,6 +42,9 @@ struct AIController : AIBase {
     // above a threshold and minimum odds that fall as possession lasts. -1 for none.
     HD int BestPassTarget(float mind, const ImageList &opps, float oneTouchIsHard, float longPossession, int &passType,
                           float &passOdds) const {
+        World &w = world;
+        MatchState &m = w.match;
+        Player &ps = w.match.players[p];
         const PassWeights pw = PassWeightsOf(mind);
         const float improvement = 0.06f * (1.0f - mind);
         const float gainWeight = 1.0f + (mind * mind) * 10.0f, oddsWeight = 1.0f;
@@ -83,6 +89,7 @@ struct AIController : AIBase {
     // no pass is good enough for the danger and its possession is shaky; a goalkeeper clears when
     // its possession is below 3.
     HD void ConsiderClearance(float mind, int bestPlayer, float bestOdds) {
+        PlayerControllerState &ctl = controller;
         if (!(mind < 0.25f)) return;
         const float panic = 1.0f - mind * 2.0f;
         const float nearGoal = 1.0f - NormalizedClamp((Pos() - Vec3(kPitchHalfLength * side, 0, 0)).Length(), 2.0f, 16.0f);
@@ -97,6 +104,7 @@ struct AIController : AIBase {
     // pass 0.5: at that point, scattered by a draw (less with the shot statistic), leaning 30%
     // against its running direction by speed, with a drawn power (stronger further out).
     HD void ConsiderShot(const ImageList &opps, float rawVel) {
+        CommandQueue &q = queue;
         const float goalDistance = NormalizedClamp((Vec3(kPitchHalfLength * -side, 0, 0) - Pos()).Length(), 0.0f, 32.0f);
         const float ideal = Curve(1.0f - NormalizedClamp((Vec3((kPitchHalfLength - 7.0f) * -side, 0, 0) - Pos()).Length(), 0.0f, 16.0f), 1.0f);
         if (!(ideal > 0.1f)) return;
@@ -129,6 +137,9 @@ struct AIController : AIBase {
     // The commands of a player on the ball: a panic clearance, a pass to the best-placed teammate,
     // a shot, and a dribble direction from a force field.
     HDN void GetOnTheBallCommands(Vec3 &rawDir, float &rawVel) {
+        World &w = world;
+        MatchState &m = w.match;
+        Player &ps = w.match.players[p];
         ENG_SCOPE(44);
         const float ballGap = NormalizedClamp((m.ball.momentum - Mov()).Length(), 0.0f, 10.0f);
         const float oneTouchIsHard = ballGap - Stat(kStatShortPass) * ballGap * 0.8f;
@@ -156,6 +167,8 @@ struct AIController : AIBase {
         int type, scorer;  // type 1 scored, 2 conceded; scorer 2 for the scorer itself
     };
     HD Celebration CelebrationOf() const {
+        World &w = world;
+        MatchState &m = w.match;
         const int xSide = (BallAt(0).Get2D().v[0] > 0) ? 1 : -1;
         const int last = Own().lastTouchPlayer;
         const int ySide = last >= 0 ? ((Pos(last).v[1] > 0) ? 1 : -1) : side;
@@ -182,6 +195,9 @@ struct AIController : AIBase {
         return c;
     }
     HDN void AddCelebration() {
+        World &w = world;
+        MatchState &m = w.match;
+        CommandQueue &q = queue;
         const Celebration c = CelebrationOf();
         const uint64_t stop = m.referee.buffer.stopTime;
         if (m.actualTimeMs - stop > 2000 && m.actualTimeMs - stop < 4000) {
@@ -206,6 +222,7 @@ struct AIController : AIBase {
     // The penalty taker shoots at a drawn point up to 5 m from the goal's centre with a drawn
     // power. Returns the shot's direction.
     HD Vec3 PenaltyShot() {
+        CommandQueue &q = queue;
         PlayerCommand action = DefaultPlayerCommand();
         action.desiredFunctionType = kFnShot;
         TouchInformation &t = action.touchInfo;
@@ -222,6 +239,10 @@ struct AIController : AIBase {
     // throw-in at the taker; a goalkeeper holding the ball lofts it upfield to a teammate who has
     // 10 m of space (or after 4 s), or waits. Returns false when the keeper waits.
     HD bool RestartPassTarget(int type, PlayerCommand &action, Vec3 &target) {
+        World &w = world;
+        const Ctx &c = context;
+        MatchState &m = w.match;
+        Player &ps = w.match.players[p];
         TouchInformation &t = action.touchInfo;
         switch (type) {
             case kModeGoalKick:
@@ -277,6 +298,10 @@ struct AIController : AIBase {
     // the teammate nearest its target, then a movement: toward the ball at walking pace, or, for
     // the retainer, facing its pass (or the centre) standing.
     HDN void SetPieceCommands() {
+        World &w = world;
+        const Ctx &c = context;
+        MatchState &m = w.match;
+        CommandQueue &q = queue;
         const int type = AI().setPieceType;
         Vec3 passDir;
         if (type == kModePenalty) {
@@ -317,6 +342,9 @@ struct AIController : AIBase {
     // out of play or for a lazy player, drifting toward the centre (60% its own direction) at
     // 95% of its speed less a draw of up to 3.2 m/s, looking at the ball. True when one was given.
     HD bool StoppageCommand(bool lazy) {
+        World &w = world;
+        MatchState &m = w.match;
+        CommandQueue &q = queue;
         const RefereeBuffer &rb = m.referee.buffer;
         if (!m.inPlay && m.goalScored) {
             AddCelebration();
@@ -347,6 +375,10 @@ struct AIController : AIBase {
     // haste, and one of the two nearest to the opponent moves to its defending position when it
     // is out of line.
     HD void PressOpponent(bool &forceMagnet, bool &extraHaste) {
+        World &w = world;
+        const Ctx &c = context;
+        Player &ps = w.match.players[p];
+        PlayerControllerState &ctl = controller;
         const int o = Opp().designatedTeamPossessionPlayer;
         const float mind = GetMindSet(DynamicRole());
         float hunt = 10.0f + (1.0f - mind) * 10.0f;
@@ -382,6 +414,9 @@ struct AIController : AIBase {
     // handled as a restart before.)
     enum OpenPlayPart { kNoPart, kLinePart, kBallPart, kKeeperPart };
     HD int OpenPlayPartOf(int role) const {
+        World &w = world;
+        MatchState &m = w.match;
+        Player &ps = w.match.players[p];
         if (!m.inPlay || m.inSetPiece) return kNoPart;
         if (role == kRoleGoalkeeper) return kKeeperPart;
         if (m.designatedPossessionPlayer != p) return kLinePart;
@@ -404,6 +439,9 @@ struct AIController : AIBase {
     // it holds the ball uniquely with possession 3.4 or more (pickups only when nothing is bound
     // for goal and the possession passes 1.3).
     HD bool KeeperPart(Vec3 &dir, float &vel) {
+        World &w = world;
+        MatchState &m = w.match;
+        PlayerControllerState &ctl = controller;
         const bool bound = BallBoundForGoal();
         GoalieRequestInput(dir, vel);
         if (!ctl.hasUniquePossession || ctl.possessionAmount < 3.4f) KeeperDeflectCommand(!bound && ctl.possessionAmount > 1.3f);
@@ -412,12 +450,16 @@ struct AIController : AIBase {
     // The team's pressure order names this player, still running, while the opponents hold the
     // ball better; never the designated player or the keeper.
     HD bool PressureOrdered(int role) const {
+        World &w = world;
+        MatchState &m = w.match;
+        PlayerControllerState &ctl = controller;
         return m.inPlay && !m.inSetPiece && (AI().endApplyTeamPressureMs > m.actualTimeMs && AI().teamPressurePlayer == p) &&
                !ctl.teamHasBestPossession && m.designatedPossessionPlayer != p && role != kRoleGoalkeeper;
     }
     // Moving by the player's own choice: along `dir` at `vel`, looking 10 m toward the ball 40 ms
     // ahead.
     HD void OwnMovement(const Vec3 &dir, float vel) {
+        CommandQueue &q = queue;
         PlayerCommand cmd = DefaultPlayerCommand();
         cmd.useDesiredMovement = true;
         cmd.desiredDirection = dir;
@@ -433,6 +475,12 @@ struct AIController : AIBase {
     // together), the touch commands, and the movement command (pressing first), or the keeper's
     // own movement.
     HDN bool RequestCommand() {
+        World &w = world;
+        const Ctx &c = context;
+        MatchState &m = w.match;
+        Player &ps = w.match.players[p];
+        PlayerControllerState &ctl = controller;
+        AIControllerState *const eliza = elizaState;
         if (m.designatedPossessionPlayer < 0) return Fail("the AI controller finds no designated possession player");
         if (Own().designatedTeamPossessionPlayer < 0 || Opp().designatedTeamPossessionPlayer < 0)
             return Fail("the AI controller finds no designated team possession player");
@@ -484,7 +532,9 @@ struct AIController : AIBase {
     }
 };
 
-HDN void TeamApplyTeamPressure(World &w, const Ctx &c, int teamID) {
+HDN void TeamApplyTeamPressure(GlobalRef<World> world, LocalRef<const Ctx> context, int teamID) {
+    World &w = world;
+    const Ctx &c = context;
     TeamAI &ai = TeamByID(w, teamID).ai;
     ai.endApplyTeamPressureMs = w.match.actualTimeMs + 500;
     int o = TeamBestPossessionPlayer(w, 1 - teamID);
@@ -631,7 +681,10 @@ HD void GamerTouchCommands(World &w, int p, AIController &ai, HumanControllerSta
 // and the others wait in position; otherwise the touch commands and a movement, forced toward
 // the ball by pressure or an armed pass or shot. Without the magnet the movement follows the
 // stick, facing the ball half a second ahead; dribble with sprint off the ball follows it too.
-HDN bool HumanRequestCommand(World &w, const Ctx &c, int p, CommandQueue &q) {
+HDN bool HumanRequestCommand(GlobalRef<World> world, LocalRef<const Ctx> context, int p, GlobalRef<CommandQueue> queue) {
+    World &w = world;
+    const Ctx &c = context;
+    CommandQueue &q = queue;
     ENG_SCOPE(45);
     HumanControllerState &hc = HumanGamerOf(w, p).controller;
     PlayerControllerState &ctl = hc.base;
@@ -680,7 +733,10 @@ HDN bool HumanRequestCommand(World &w, const Ctx &c, int p, CommandQueue &q) {
     return true;
 }
 
-HDN bool PlayerRequestCommand(World &w, const Ctx &c, int p, CommandQueue &q) {
+HDN bool PlayerRequestCommand(GlobalRef<World> world, LocalRef<const Ctx> context, int p, GlobalRef<CommandQueue> queue) {
+    World &w = world;
+    const Ctx &c = context;
+    CommandQueue &q = queue;
     ENG_SCOPE(13);
     if (ExternalControllerActive(w, p)) return HumanRequestCommand(w, c, p, q);
     AIControllerState &e = w.match.players[p].controller;

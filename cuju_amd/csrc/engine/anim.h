@@ -18,7 +18,8 @@ namespace eng {
 // (both ratios divided in double and rounded to float once); with a key on one side only, that key
 // holds. Also run on the host to fill the interpolation table, so that table reads equal it bit
 // for bit.
-HDN void ComputeInterpolated(const Anim &a, const KeyFrame *keys, int keyCount, int frame, Quat &ori, Vec3 &pos) {
+HDN void ComputeInterpolated(GlobalRef<const Anim> animation, GlobalPointer<const KeyFrame> keys, int keyCount, int frame, Quat &ori, Vec3 &pos) {
+    const Anim &a = animation;
     if (frame >= a.frameCount) {
         ori = Quat::Identity();
         pos = Vec3(0);
@@ -57,12 +58,12 @@ HDN void ComputeInterpolated(const Anim &a, const KeyFrame *keys, int keyCount, 
 
 HD void Interpolated(const Ctx &c, const Anim &a, const NodeAnim &n, int frame, Quat &ori, Vec3 &pos) {
     if (frame < n.interpFrames) {
-        const InterpEntry &e = c.t->interp[n.interpFirst + (frame < 0 ? 0 : frame) * n.interpStride];
+        const InterpEntry &e = c.T().interp[n.interpFirst + (frame < 0 ? 0 : frame) * n.interpStride];
         ori = e.orientation;
         pos = e.position;
         return;
     }
-    ComputeInterpolated(a, c.t->keys + n.keyFirst, n.keyCount, frame, ori, pos);
+    ComputeInterpolated(a, c.T().keys + n.keyFirst, n.keyCount, frame, ori, pos);
 }
 
 HD void BlendFrames(Quat at, const Vec3 &pAt, const Quat &next, const Vec3 &pNext, float bias, Quat &ori, Vec3 &pos) {
@@ -73,13 +74,13 @@ HD void BlendFrames(Quat at, const Vec3 &pAt, const Quat &next, const Vec3 &pNex
 
 HD void InterpolatedZ(const Ctx &c, const Anim &a, const NodeAnim &n, int frame, Quat &ori, Vec3 &pos, float &z) {
     if (frame < n.interpFrames) {
-        const InterpEntry &e = c.t->interp[n.interpFirst + (frame < 0 ? 0 : frame) * n.interpStride];
+        const InterpEntry &e = c.T().interp[n.interpFirst + (frame < 0 ? 0 : frame) * n.interpStride];
         ori = e.orientation;
         pos = e.position;
         z = e.angleZ;
         return;
     }
-    ComputeInterpolated(a, c.t->keys + n.keyFirst, n.keyCount, frame, ori, pos);
+    ComputeInterpolated(a, c.T().keys + n.keyFirst, n.keyCount, frame, ori, pos);
     float x, y;
     ori.Angles(x, y, z);
 }
@@ -89,7 +90,7 @@ HD void InterpolatedZ(const Ctx &c, const Anim &a, const NodeAnim &n, int frame,
 HD void GetKeyFrameZ(const Ctx &c, const Anim &a, int bodyPart, int frame, Quat &ori, Vec3 &pos, float &z) {
     const int i = a.nodeOfBodyPart[bodyPart];
     if (i >= 0) {
-        InterpolatedZ(c, a, c.t->nodes[a.nodeFirst + i], frame, ori, pos, z);
+        InterpolatedZ(c, a, c.T().nodes[a.nodeFirst + i], frame, ori, pos, z);
         return;
     }
     float x, y;
@@ -99,10 +100,10 @@ HD void GetKeyFrameZ(const Ctx &c, const Anim &a, int bodyPart, int frame, Quat 
 HD bool GetKeyFrame(const Ctx &c, const Anim &a, int bodyPart, int frame, Quat &ori, Vec3 &pos) {
     const int i = a.nodeOfBodyPart[bodyPart];
     if (i < 0) return false;
-    const NodeAnim &n = c.t->nodes[a.nodeFirst + i];
+    const NodeAnim &n = c.T().nodes[a.nodeFirst + i];
     Interpolated(c, a, n, frame, ori, pos);
     for (int k = 0; k < n.keyCount; k++)
-        if (c.t->keys[n.keyFirst + k].frame == frame) return true;
+        if (c.T().keys[n.keyFirst + k].frame == frame) return true;
     return false;
 }
 
@@ -115,7 +116,7 @@ struct Transform {
 // A local transform placed under `parent`. A relative one composes with it: the rotations
 // multiplied and renormalized, the scales multiplied, the position scaled and turned by the
 // parent's, then moved by its position. An absolute one, or a root's, stands as it is.
-HDN Transform Placed(const Transform *parent, int localMode, const Vec3 &pos, const Quat &rot, const Vec3 &scale) {
+HDN Transform Placed(const Transform *parent, int localMode, Vec3 pos, const Quat &rot, Vec3 scale) {
     if (localMode != kLocalRelative || !parent) return Transform{pos, scale, rot};
     Transform t;
     t.rotation = (parent->rotation * rot).Normalized();
@@ -182,7 +183,7 @@ HD void ApplyPrepare(const Ctx &c, const Anim &a, Humanoid &h, bool smooth, int 
     }
     int count = entries;
     for (int n = 0; n < a.nodeCount; n++) {
-        int bp = c.t->nodes[a.nodeFirst + n].bodyPart;
+        int bp = c.T().nodes[a.nodeFirst + n].bodyPart;
         int found = last[bp];
         plan.isNew[n] = found < 0;
         if (found < 0) {
@@ -210,7 +211,7 @@ HD const MiddleEntry *NodeFramePose(const Ctx &c, const Anim &a, const NodeAnim 
     const int bp = na.bodyPart;
     const MiddleEntry *middle = nullptr;
     if (frame >= 0 && frame + 1 < na.interpFrames) {
-        middle = &c.t->middle[na.interpFirst + frame * na.interpStride];
+        middle = &c.T().middle[na.interpFirst + frame * na.interpStride];
         ori = middle->orientation;
         pos = middle->position;
     } else {
@@ -292,10 +293,14 @@ HD void SmoothRootHeight(Vec3 &pos, const Vec3 &current, const Vec3 &basePos, fl
 }
 // One node of a humanoid's frame: its pose, smoothed against the movement history (a node new to
 // the history starts it at this pose), then written to the node.
-HDN void ApplyNode(const Ctx &c, const Anim &a, const Skeleton &sk, Humanoid &h, int ni, int frame, bool smooth,
-                   float smoothFactor, const Vec3 &basePos, float baseRot, BiasedOffset *offsets, int dtMs, bool noPos,
+HDN void ApplyNode(LocalRef<const Ctx> context, GlobalRef<const Anim> animation, GlobalRef<const Skeleton> skeleton, GlobalRef<Humanoid> humanoid, int ni, int frame, bool smooth,
+                   float smoothFactor, Vec3 basePos, float baseRot, GlobalPointer<BiasedOffset> offsets, int dtMs, bool noPos,
                    const ApplyPlan &plan) {
-    const NodeAnim &na = c.t->nodes[a.nodeFirst + ni];
+    const Ctx &c = context;
+    const Anim &a = animation;
+    const Skeleton &sk = skeleton;
+    Humanoid &h = humanoid;
+    const NodeAnim &na = c.T().nodes[a.nodeFirst + ni];
     const int bp = na.bodyPart;
     NodeState &node = h.nodes[sk.nodeMap[bp]];
     Quat ori;
@@ -330,7 +335,8 @@ HDN void ApplyNode(const Ctx &c, const Anim &a, const Skeleton &sk, Humanoid &h,
 }
 
 // Applies every humanoid's buffered frame; humanoids are independent.
-HDN void FetchPutBuffers(const Ctx &c, const Skeleton *const *skels, Humanoid *const *hums, int count) {
+HDN void FetchPutBuffers(LocalRef<const Ctx> context, const GlobalPointer<const Skeleton> *skels, const GlobalPointer<Humanoid> *hums, int count) {
+    const Ctx &c = context;
     // A humanoid's pose reads and writes only its own state, so the lanes of the match take the
     // humanoids in turn. A node reads and writes only its own body part's node, offset and history
     // entry, so the humanoids left over after the whole rounds have their nodes split over the lanes
@@ -397,7 +403,7 @@ HD float AllowedBodyDirAngle(int i) {
     return 0.0f;
 }
 constexpr int kNoAllowedBodyDirection = 5;
-HDN int BodyDirectionIndex(const Vec3 &src) {
+HDN int BodyDirectionIndex(Vec3 src) {
     float best = -1.0f;
     int bi = kNoAllowedBodyDirection;
     for (int i = 0; i < 5; i++) {
@@ -412,7 +418,7 @@ HDN int BodyDirectionIndex(const Vec3 &src) {
 HD Vec3 BodyDirectionSnapped(const Vec3 &src) { return AllowedBodyDir(BodyDirectionIndex(src)); }
 
 // Ground-plane movement in m/s at `frame` of a position list of two frames or more.
-HDN Vec3 MovementAtFrame(const Vec3 *pos, int count, uint32_t frame, uint32_t smooth) {
+HDN Vec3 MovementAtFrame(GlobalPointer<const Vec3> pos, int count, uint32_t frame, uint32_t smooth) {
     if (frame == (uint32_t)(count - 1)) return (pos[count - 1] - pos[count - 2]).Get2D() * 100.0f;
     if (frame == 0) return (pos[1] - pos[0]).Get2D() * 100.0f;
     Vec3 total;
@@ -464,7 +470,9 @@ HD Vec3 RelativeBody(const Vec3 &body, float angle, int velocityCat, float &unsn
 // movement, which is the movement); the animation's own movement; velocity and its category;
 // the direction (the movement's, or the body's when idle) and angle; the body direction relative
 // to it, snapped to the allowed directions, and in the world.
-HDN SpatialState NextSpatialState(const Ctx &c, const Humanoid &h) {
+HDN SpatialState NextSpatialState(LocalRef<const Ctx> context, GlobalRef<const Humanoid> humanoid) {
+    const Ctx &c = context;
+    const Humanoid &h = humanoid;
     ENG_SCOPE(29);
     const AnimationState &cur = h.anim;
     const Anim &a = c.A(cur.anim);
@@ -475,7 +483,7 @@ HDN SpatialState NextSpatialState(const Ctx &c, const Humanoid &h) {
     s.physicsMovement = s.actualMovement - (s.actionSmuggleMovement) - (s.movementSmuggleMovement) - (s.positionOffsetMovement * 0.5f);
     s.animationMovement = s.physicsMovement;
     if (cur.positions.count > 0)
-        s.animationMovement = MovementAtFrame(c.t->positions + a.posFirst, a.posCount, cur.frameNum, 1).Rotated2D(h.startAngle.value());
+        s.animationMovement = MovementAtFrame(c.T().positions + a.posFirst, a.posCount, cur.frameNum, 1).Rotated2D(h.startAngle.value());
     s.movement = s.physicsMovement;
     Vec3 bodyPos;
     Quat bodyOri;

@@ -198,7 +198,8 @@ struct BallFlight {
 // whether it is in the goal. When those match the last full prediction bit for bit, its first step
 // lands on entry 1; unless the cached path applies, the full path would write exactly what the
 // arrays already hold, so only its other results are restored.
-HDN BallSpatial BallCalculatePrediction(Ball &ball, bool ballIsInGoal) {
+HDN BallSpatial BallCalculatePrediction(GlobalRef<Ball> matchBall, bool ballIsInGoal) {
+    Ball &ball = matchBall;
     ENG_SCOPE(37);
     if (ball.memoValid && ball.memoInGoal == ballIsInGoal && SameBits(ball.memoPosition, ball.positionBuffer) &&
         SameBits(ball.memoMomentum, ball.momentum) && SameBits(ball.memoOrientation, ball.orientationBuffer) &&
@@ -276,7 +277,8 @@ HD void BallRecalculatePrediction(World &w) {
     BallCalculatePrediction(w.match.ball, w.match.ballIsInGoal);
 }
 
-HDN void BallProcess(Ball &b, bool inGoal) {
+HDN void BallProcess(GlobalRef<Ball> matchBall, bool inGoal) {
+    Ball &b = matchBall;
     ENG_SCOPE(7);
     BallMaterialize(b);
     BallSpatial s = BallCalculatePrediction(b, inGoal);
@@ -384,7 +386,8 @@ HD TimeNeeded GetTimeNeededMs(const Vec3 &pos, const Vec3 &mov, const Vec3 &targ
 // result as GetTimeNeededMs. With `cooperative` the lanes of the match (all running the same
 // sequential code) test consecutive steps of the walk together.
 HD bool TimeWalkApplies(const Vec3 &mov) { return mov.Length() > kIdleDribbleSwitch; }
-HDN void BuildTimeWalk(TimeWalk &wk, const Vec3 &pos, const Vec3 &mov, float maxVel) {
+HDN void BuildTimeWalk(GlobalRef<TimeWalk> timeWalk, Vec3 pos, Vec3 mov, float maxVel) {
+    TimeWalk &wk = timeWalk;
     Vec3 cur = pos, cm = mov;
     cur += cm.Normalized() * 0.1f;
     cur += cm * 0.01f;
@@ -408,8 +411,9 @@ HDN void BuildTimeWalk(TimeWalk &wk, const Vec3 &pos, const Vec3 &mov, float max
         wk.optimisticSquared[k] = optR * optR;
     }
 }
-HDN TimeNeeded WalkTimeNeeded(const TimeWalk &wk, const Vec3 &pos, const Vec3 &mov, const Vec3 &target, float maxVel,
+HDN TimeNeeded WalkTimeNeeded(GlobalRef<const TimeWalk> timeWalk, Vec3 pos, Vec3 mov, Vec3 target, float maxVel,
                               bool precise, uint32_t maxTime, bool cooperative) {
+    const TimeWalk &wk = timeWalk;
     TimeNeeded r;
     if ((pos - target).Length() > (precise ? 48.0f : 16.0f)) {
         r.usual = DirectTimeMs(pos, mov, target, maxVel);
@@ -579,7 +583,7 @@ HD Vec3 PredFlip(const Vec3 *pred, bool flip, int ms) {
 // walk at its own point of a round of `lanes`; the lowest reached point of a round ends the coarse
 // part, and the refinement's 10 ms points are shared the same way. What the scan visits, and so
 // its result, is the same for any number of lanes.
-HDN ScanResult SharedPossessionScan(const Vec3 *pred, bool flip, const Vec3 &pos, const Vec3 &mov, float maxVel,
+HDN ScanResult SharedPossessionScan(GlobalPointer<const Vec3> pred, bool flip, Vec3 pos, Vec3 mov, float maxVel,
                                     bool precise, uint32_t start, int lane, int lanes) {
     ENG_SCOPE(35);
     ScanResult s;
@@ -659,7 +663,7 @@ HDN ScanResult SharedPossessionScan(const Vec3 *pred, bool flip, const Vec3 &pos
 }
 
 // The same scan on one lane, point after point.
-HDN ScanResult PossessionScan(const Vec3 *pred, bool flip, const Vec3 &pos, const Vec3 &mov, float maxVel,
+HDN ScanResult PossessionScan(GlobalPointer<const Vec3> pred, bool flip, Vec3 pos, Vec3 mov, float maxVel,
                               bool precise, uint32_t start) {
     ENG_SCOPE(35);
     ScanResult s;
@@ -703,7 +707,8 @@ HDN ScanResult PossessionScan(const Vec3 *pred, bool flip, const Vec3 &pos, cons
     return s;
 }
 
-HDN bool HasPossession(const World &w, int p) {
+HDN bool HasPossession(GlobalRef<const World> world, int p) {
+    const World &w = world;
     const Ball &b = w.match.ball;
     const SpatialState &s = Sp(w, p);
     if ((double)(s.position - BallPredict(b, 0)).Length() > 5.0) return false;
@@ -719,7 +724,9 @@ HDN bool HasPossession(const World &w, int p) {
 
 HD bool IsPassOrShot(int f) { return f == kFnShortPass || f == kFnLongPass || f == kFnHighPass || f == kFnShot; }
 
-HDN void PlayerUpdatePossessionStatistics(World &w, const StaticData &sd, int p, int lane = 0, int lanes = 1) {
+HDN void PlayerUpdatePossessionStatistics(GlobalRef<World> world, GlobalRef<const StaticData> staticData, int p, int lane = 0, int lanes = 1) {
+    World &w = world;
+    const StaticData &sd = staticData;
     Player &ps = w.match.players[p];
     const Humanoid &h = ps.base.humanoid;
     const Ball &b = w.match.ball;
@@ -765,7 +772,9 @@ HDN void PlayerUpdatePossessionStatistics(World &w, const StaticData &sd, int p,
     w.roster.timeToBallMs[p] = ps.timeToBallMs;
 }
 
-HDN void TeamUpdatePossessionStatistics(World &w, const Ctx &c, int teamID) {
+HDN void TeamUpdatePossessionStatistics(GlobalRef<World> world, LocalRef<const Ctx> context, int teamID) {
+    World &w = world;
+    const Ctx &c = context;
     ENG_SCOPE(16);
     // A player's statistics read only the ball, the opposing team and its own fields, so the lanes
     // of the match take the players in turn, one a lane in whole rounds. The players left after
@@ -793,7 +802,9 @@ HDN void TeamUpdatePossessionStatistics(World &w, const Ctx &c, int teamID) {
     t.timeToBallMs = timeToBall;
 }
 
-HDN void BallTouch(World &w, const Ctx &c, const Vec3 &target) {
+HDN void BallTouch(GlobalRef<World> world, LocalRef<const Ctx> context, const Vec3 &target) {
+    World &w = world;
+    const Ctx &c = context;
     Ball &b = w.match.ball;
     b.validPredictions = 0;
     if (b.positionBuffer.v[2] < 0.11f) b.positionBuffer.v[2] = 0.11f;

@@ -84,7 +84,7 @@ HD void RecordCameraAim(MatchState &m, const Vec3 &aim, const Vec3 &shake) {
 HD Vec3 CameraHistoryMean(const MatchState &m, const Ctx &c) {
     const auto &history = m.cameraPosition;
     const int count = history.count;
-    const float *weights = c.t->cameraWeights + count * (count - 1) / 2;
+    const float *weights = c.T().cameraWeights + count * (count - 1) / 2;
     Vec3 sum;
     float total = 0;
     constexpr int kChunk = 8;
@@ -191,7 +191,9 @@ HD void CameraOnCard(World &w, bool mirrored) {
 }
 
 // The camera's tick, on the unmirrored pitch (team 1 read mirrored in place).
-HDN void UpdateCamera(World &w, const Ctx &c) {
+HDN void UpdateCamera(GlobalRef<World> world, LocalRef<const Ctx> context) {
+    World &w = world;
+    const Ctx &c = context;
     ENG_SCOPE(19);
     MatchState &m = w.match;
     if (m.autoUpdateInGameCamera) {

@@ -70,7 +70,8 @@ HD void BlendAfterSwitch(World &w, int p, PlayerControllerState &base, Vec3 &dir
 }
 // What a gamer's keyboard asks of player `p`: a direction and a velocity. A stick inside the dead
 // zone keeps the player's direction, idle.
-HDN void HumanGetKeyboardInput(World &w, int p, Vec3 &dir, float &vel) {
+HDN void HumanGetKeyboardInput(GlobalRef<World> world, int p, Vec3 &dir, float &vel) {
+    World &w = world;
     HumanControllerState &hc = HumanGamerOf(w, p).controller;
     const SpatialState &s = Sp(w, p);
     dir = StickInsidePitch(KeyboardDirection(hc.keyboard), s.position);
@@ -101,7 +102,8 @@ HD void KeyboardReleaseNonStickyButtons(World &w, int g) {
     ReleaseNonStickyButtons(w.match.secondKeyboardCopies[g]);
 }
 
-HDN void HumanControllerReset(World &w, int g) {
+HDN void HumanControllerReset(GlobalRef<World> world, int g) {
+    World &w = world;
     HumanControllerState &c = GamerByGlobal(w, g).controller;
     c.actionMode = 0;
     c.gaugeMs = 0;
@@ -135,7 +137,8 @@ HD void SetExternalController(World &w, int p, int g) {
         ps.controller.lastDesiredVelocity = 0;
     }
 }
-HDN void HumanGamerSetSelectedPlayer(World &w, int g, int p) {
+HDN void HumanGamerSetSelectedPlayer(GlobalRef<World> world, int g, int p) {
+    World &w = world;
     HumanGamer &gm = GamerByGlobal(w, g);
     if (p >= 0 && w.match.players[p].base.externalController >= 0) return;
     if (gm.selectedPlayer >= 0) {
@@ -158,7 +161,9 @@ HD void RotateSwitchOrder(Team &t) {
 }
 // A selectable player becomes the team's main selection and, when no gamer holds it, the player of
 // the gamer first in the switch order (who then goes to the back); it is the designated player.
-HDN bool TeamSelectPlayer(World &w, const Ctx &c, int teamID, int p) {
+HDN bool TeamSelectPlayer(GlobalRef<World> world, LocalRef<const Ctx> context, int teamID, int p) {
+    World &w = world;
+    const Ctx &c = context;
     Team &t = TeamByID(w, teamID);
     if (Formation(w, c, p).controllable) {
         t.mainSelectedPlayer = p;
@@ -171,8 +176,10 @@ HDN bool TeamSelectPlayer(World &w, const Ctx &c, int teamID, int p) {
     return true;
 }
 // A tie keeps the player first in the state.
-HDN int GetClosestPlayer(const World &w, const Ctx &c, int teamID, const Vec3 &pos, bool onlyAI, int except = -1,
+HDN int GetClosestPlayer(GlobalRef<const World> world, LocalRef<const Ctx> context, int teamID, Vec3 pos, bool onlyAI, int except = -1,
                          bool onlySelectable = false) {
+    const World &w = world;
+    const Ctx &c = context;
     float best = 10000;
     int bp = -1;
     const int players = w.match.playerCount;
@@ -208,7 +215,9 @@ HD int HumanControlledToBallTime(const World &w, int teamID) {
 // front of the switch order; the team's designated outfield player goes to a gamer when it is
 // three times quicker to the ball than every controlled player, or when it alone has the ball (or
 // a set piece is on). Each test reads the designated player anew.
-HDN bool TeamUpdateSwitch(World &w, const Ctx &c, int teamID) {
+HDN bool TeamUpdateSwitch(GlobalRef<World> world, LocalRef<const Ctx> context, int teamID) {
+    World &w = world;
+    const Ctx &c = context;
     ENG_SCOPE(9);
     MatchState &m = w.match;
     Team &t = TeamByID(w, teamID);
@@ -223,7 +232,9 @@ HDN bool TeamUpdateSwitch(World &w, const Ctx &c, int teamID) {
     if (freeOutfield(d) && (m.players[d].hasUniquePossession || m.inSetPiece) && !TeamSelectPlayer(w, c, teamID, d)) return false;
     return true;
 }
-HDN void TeamHumanGamersSelectAnyone(World &w, const Ctx &c, int teamID) {
+HDN void TeamHumanGamersSelectAnyone(GlobalRef<World> world, LocalRef<const Ctx> context, int teamID) {
+    World &w = world;
+    const Ctx &c = context;
     MatchState &m = w.match;
     if (!m.inPlay) return;
     Team &t = TeamByID(w, teamID);

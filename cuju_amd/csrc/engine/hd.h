@@ -66,6 +66,45 @@ HD double DoubleOf(uint64_t b) {
     return v;
 }
 
+// ---- memory spaces ---------------------------------------------------------------------------------
+// Pointers and references that name the memory they point into: the GPU's memory (HBM) or the
+// workgroup's LDS. A plain pointer is generic: the hardware resolves its memory per lane, its loads
+// and stores count as both kinds of memory, and the code after one waits for every outstanding
+// access, stores included. A noinline function knows nothing of what its arguments point to, so the
+// functions of the engine take what lives in HBM as GlobalRef and what lives in LDS as LocalRef, and
+// pointers kept in structures are GlobalPointers. On the host all of them are plain pointers.
+// Measured on gfx950, ms per step against generic pointers (6,111 generic loads in the code, 1,002
+// left): 11-a-side, one environment 16.1 -> 15.3, 4,096 55.0 -> 51.9, 16,384 (11 agents) 143.5 ->
+// 137.8; a masked reset of a tenth of 4,096 15.1 -> 12.9.
+#if ENG_DEVICE
+#define ENG_GLOBAL __attribute__((address_space(1)))
+#define ENG_LOCAL __attribute__((address_space(3)))
+#else
+#define ENG_GLOBAL
+#define ENG_LOCAL
+#endif
+template <class T>
+struct GlobalPointer {
+    ENG_GLOBAL T *p;
+    GlobalPointer() = default;
+    HD GlobalPointer(T *q) : p((ENG_GLOBAL T *)q) {}
+    HD operator T *() const { return (T *)p; }
+    HD T *operator->() const { return (T *)p; }
+    HD T *get() const { return (T *)p; }
+};
+template <class T>
+struct GlobalRef {
+    ENG_GLOBAL T *p;
+    HD GlobalRef(T &r) : p((ENG_GLOBAL T *)&r) {}
+    HD operator T &() const { return *(T *)p; }
+};
+template <class T>
+struct LocalRef {
+    ENG_LOCAL T *p;
+    HD LocalRef(T &r) : p((ENG_LOCAL T *)&r) {}
+    HD operator T &() const { return *(T *)p; }
+};
+
 // Whether `x` holds in any lane of the wavefront that executes the call (the lanes of a wavefront
 // run different matches). The host runs one match at a time, so there it is `x`. Being a
 // wavefront-wide operation, a call is a point where those lanes meet: none passes it before all

@@ -14,7 +14,8 @@ namespace eng {
 // mirrors, so a team that the current frame holds mirrored from the rest frame (`mirrored`, by
 // team ID) stores its direction negated too: a frame change negates a humanoid's position and
 // movement but leaves its direction alone.
-HDN void PushMentalImage(World &w, const bool (&mirrored)[2]) {
+HDN void PushMentalImage(GlobalRef<World> world, const bool (&mirrored)[2]) {
+    World &w = world;
     ENG_SCOPE(8);
     MatchState &m = w.match;
     const int n = m.mentalImages.count < 3 ? m.mentalImages.count + 1 : 3;
@@ -50,7 +51,8 @@ HDN void PushMentalImage(World &w, const bool (&mirrored)[2]) {
     m.mentalImages.count = n;
 }
 
-HDN void CalculateBestPossessionTeamID(World &w) {
+HDN void CalculateBestPossessionTeamID(GlobalRef<World> world) {
+    World &w = world;
     MatchState &m = w.match;
     if (m.ballRetainer != -1) {
         m.bestPossessionTeam = TeamSlot(w, w.playerTeamID[m.ballRetainer]);
@@ -96,7 +98,8 @@ HD bool PathThroughTriangle(const Vec3 (&corner)[3], const Vec3 &normal, const V
 }
 // Whether the ball went into the goal at `side` this tick, from `before`: it must end near the
 // goal line, and a ball that started wide of the posts beyond the line does not count.
-HDN bool BallEnteredGoal(const World &w, int side, const Vec3 &before) {
+HDN bool BallEnteredGoal(GlobalRef<const World> world, int side, Vec3 before) {
+    const World &w = world;
     const Ball &b = w.match.ball;
     if ((double)fabsf(BallPredict(b, 10).v[0]) < (double)kPitchHalfLength - 1.0) return false;
     const Vec3 after = BallPredict(b, 0);
@@ -160,7 +163,9 @@ HD void RecordPossessionSide(World &w) {
 
 // False when the tick ends early: while play waits for a restart (the clock still advances), or
 // on an unsupported path, which also clears `ok`.
-HDN bool MatchProcess(World &w, const Ctx &c, bool &ok) {
+HDN bool MatchProcess(GlobalRef<World> world, LocalRef<const Ctx> context, bool &ok) {
+    World &w = world;
+    const Ctx &c = context;
     ENG_SCOPE(4);
     MatchState &m = w.match;
     ok = true;
@@ -241,7 +246,8 @@ HDN bool MatchProcess(World &w, const Ctx &c, bool &ok) {
     return true;
 }
 
-HDN void PlayerPreparePutBuffers(World &w, int p) {
+HDN void PlayerPreparePutBuffers(GlobalRef<World> world, int p) {
+    World &w = world;
     PoseOffsets(w, p);
     Player &ps = w.match.players[p];
     const Team &t = TeamByID(w, w.playerTeamID[p]);
@@ -262,7 +268,8 @@ HDN void PlayerPreparePutBuffers(World &w, int p) {
     if (ext && gm->controller.actionMode == 2)
         ps.bufferPlayerColor = ps.bufferPlayerColor * (libm::sinf(w.match.actualTimeMs * 0.02f) * 0.3f + 0.7f);
 }
-HDN void MatchPreparePutBuffers(World &w) {
+HDN void MatchPreparePutBuffers(GlobalRef<World> world) {
+    World &w = world;
     ENG_SCOPE(20);
     const int first = w.FirstTeamID(), second = 1 - first;
     // A player's buffers and pose offsets are its own, and the rest of the match is only read, so
@@ -277,11 +284,13 @@ HDN void MatchPreparePutBuffers(World &w) {
     GroupSync();
     MirrorMatch(w, false, false, first == 0);
 }
-HDN void MatchFetchPutBuffers(World &w, const Ctx &c) {
+HDN void MatchFetchPutBuffers(GlobalRef<World> world, LocalRef<const Ctx> context) {
+    World &w = world;
+    const Ctx &c = context;
     ENG_SCOPE(21);
     const int first = w.FirstTeamID();
-    const Skeleton *skels[kPlayers + 3];
-    Humanoid *hums[kPlayers + 3];
+    GlobalPointer<const Skeleton> skels[kPlayers + 3];
+    GlobalPointer<Humanoid> hums[kPlayers + 3];
     int n = 0;
     for (int t = 0; t < 2; t++) {
         PlayerList ps = TeamActivePlayers(w, t == 0 ? first : 1 - first);
@@ -297,7 +306,9 @@ HDN void MatchFetchPutBuffers(World &w, const Ctx &c) {
     FetchPutBuffers(c, skels, hums, n);
 }
 // One 10 ms tick of the game.
-HDN bool GameTick(World &w, const Ctx &c) {
+HDN bool GameTick(GlobalRef<World> world, LocalRef<const Ctx> context) {
+    World &w = world;
+    const Ctx &c = context;
 #if !ENG_DEVICE
     HostTicks()++;
 #endif

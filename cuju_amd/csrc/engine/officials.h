@@ -68,7 +68,8 @@ HD ForceSpot MakeSpot(const Vec3 &origin, int magnet, int decay, float power, fl
 }
 
 // Sums run in spot order.
-HDN Vec3 GetForceFieldMovement(const ForceField &field, const Vec3 &pos, float dampingDistance = 10) {
+HDN Vec3 GetForceFieldMovement(GlobalRef<const ForceField> forces, Vec3 pos, float dampingDistance = 10) {
+    const ForceField &field = forces;
     Vec3 sum;
     float force = 0.0f;
     for (int i = 0; i < field.count; i++) {
@@ -102,7 +103,8 @@ using ImageList = Small<PlayerImagePos, kPlayers>;
 
 // The images of one team in the mental image's order, extrapolated to now and held within the
 // image's deviation limits of the true state.
-HDN void MentalTeamPlayerImages(const World &w, int k, int teamID, ImageList &out) {
+HDN void MentalTeamPlayerImages(GlobalRef<const World> world, int k, int teamID, ImageList &out) {
+    const World &w = world;
     const MentalImage &mi = w.match.mentalImages[k];
     const int age = (int)(w.match.actualTimeMs - (uint64_t)mi.timeStampMs);
     out.clear();
@@ -120,7 +122,7 @@ HDN void MentalTeamPlayerImages(const World &w, int k, int teamID, ImageList &ou
 }
 // Moves the images along x by `futureMs` in place. The deepest image is skipped (the keeper's
 // place), the next deepest or the ball sets the line, which stays in the opponent half.
-HDN float OffsideLineFromImages(ImageList &im, const Vec3 &ball, int side, unsigned futureMs) {
+HDN float OffsideLineFromImages(ImageList &im, Vec3 ball, int side, unsigned futureMs) {
     int ignored = 0;
     for (int i = 0; i < im.count; i++) {
         im[i].position.v[0] += im[i].movement.v[0] * futureMs * 0.001f;
@@ -134,7 +136,8 @@ HDN float OffsideLineFromImages(ImageList &im, const Vec3 &ball, int side, unsig
     if (line * side < 0) line = 0;
     return Clamp(line, -kPitchHalfLength, kPitchHalfLength);
 }
-HDN float GetOffsideLine(const World &w, int k, int teamID, unsigned futureMs = 0) {
+HDN float GetOffsideLine(GlobalRef<const World> world, int k, int teamID, unsigned futureMs = 0) {
+    const World &w = world;
     ImageList im;
     MentalTeamPlayerImages(w, k, teamID, im);
     return OffsideLineFromImages(im, MentalBallPrediction(w, k, 0), TeamDynamicSide(w, teamID), futureMs);
@@ -203,7 +206,8 @@ HD void BallAveragePositions(const World &w, const unsigned (&durationsMs)[N], V
         }
     }
 }
-HDN Vec3 BallAveragePosition(const World &w, unsigned durationMs) {
+HDN Vec3 BallAveragePosition(GlobalRef<const World> world, unsigned durationMs) {
+    const World &w = world;
     const unsigned durations[1] = {durationMs};
     Vec3 avg[1];
     BallAveragePositions(w, durations, avg);
@@ -278,7 +282,10 @@ HD void LinesmanFollowsLine(const World &w, const SpatialState &s, CommandQueue 
     q.push_back(HeadFor(s, target, RangeVelocity((target - pos).Length() * kDistanceToVelocity), Vec3(target.v[0], 0, 0)));
 }
 
-HDN void RefereeRequestCommand(World &w, const Ctx &ctx, int official, CommandQueue &q) {
+HDN void RefereeRequestCommand(GlobalRef<World> world, LocalRef<const Ctx> context, int official, GlobalRef<CommandQueue> queue) {
+    World &w = world;
+    const Ctx &ctx = context;
+    CommandQueue &q = queue;
     const MatchState &m = w.match;
     const SpatialState &s = m.officials[official].humanoid.spatial;
     if (official != 0) {
@@ -294,7 +301,9 @@ HDN void RefereeRequestCommand(World &w, const Ctx &ctx, int official, CommandQu
 
 // An interrupted official takes the first command whose animation it finds, and starts that
 // animation from where it stands, smoothed (less when it merely switches).
-HDN bool OfficialInterrupt(World &w, const Ctx &c, int official) {
+HDN bool OfficialInterrupt(GlobalRef<World> world, LocalRef<const Ctx> context, int official) {
+    World &w = world;
+    const Ctx &c = context;
     const int hi = w.match.playerCount + official;
     Humanoid &h = w.match.officials[official].humanoid;
     CommandQueue &q = c.ws->commands;
@@ -358,7 +367,9 @@ HD void OfficialFillApplyBuffer(const Ctx &c, Humanoid &h) {
 }
 
 // The tick of an official's humanoid: the player's tick without touches, smuggles or requeues.
-HDN bool OfficialHumanoidProcess(World &w, const Ctx &c, int official) {
+HDN bool OfficialHumanoidProcess(GlobalRef<World> world, LocalRef<const Ctx> context, int official) {
+    World &w = world;
+    const Ctx &c = context;
     Humanoid &h = w.match.officials[official].humanoid;
     AnimationState &cur = h.anim;
     // The offset from the last collision and the difficulty of the last animation fade.
@@ -378,7 +389,9 @@ HDN bool OfficialHumanoidProcess(World &w, const Ctx &c, int official) {
     OfficialFillApplyBuffer(c, h);
     return true;
 }
-HDN bool OfficialsProcess(World &w, const Ctx &c) {
+HDN bool OfficialsProcess(GlobalRef<World> world, LocalRef<const Ctx> context) {
+    World &w = world;
+    const Ctx &c = context;
     ENG_SCOPE(15);
     // The three spatial states for the tick at once, as a team's players' are: each reads its own
     // official's animation and last position, which the others' ticks leave alone.

@@ -14,8 +14,8 @@
 namespace eng {
 
 // Defined with the team AI and the player AI.
-HDN void TeamApplyAttackingRun(World &w, const Ctx &c, int teamID, int manualPlayer);
-HDN bool PlayerRequestCommand(World &w, const Ctx &c, int p, CommandQueue &q);
+HDN void TeamApplyAttackingRun(GlobalRef<World> world, LocalRef<const Ctx> context, int teamID, int manualPlayer);
+HDN bool PlayerRequestCommand(GlobalRef<World> world, LocalRef<const Ctx> context, int p, GlobalRef<CommandQueue> queue);
 
 // Reaction times in ms.
 HD int BaseReactionTime(const World &w, const Ctx &c, int p) {
@@ -36,7 +36,8 @@ HD PlayerControllerState &ActiveControllerBase(World &w, int p) {
 }
 
 // 1 for open space around `focus`, falling as opponents can reach it within the time.
-HDN float CalculateFreeSpace(const World &w, int k, int teamID, const Vec3 &focus, float safeDistance, float futureS) {
+HDN float CalculateFreeSpace(GlobalRef<const World> world, int k, int teamID, Vec3 focus, float safeDistance, float futureS) {
+    const World &w = world;
     float situation = 0.0f;
     ImageList opp;
     MentalTeamPlayerImages(w, k, 1 - teamID, opp);
@@ -51,7 +52,8 @@ HDN float CalculateFreeSpace(const World &w, int k, int teamID, const Vec3 &focu
     }
     return 1.0f - NormalizedClamp(situation, 0.0f, 2.5f);
 }
-HDN void CalculateTacticalSituation(World &w, int p) {
+HDN void CalculateTacticalSituation(GlobalRef<World> world, int p) {
+    World &w = world;
     Player &ps = w.match.players[p];
     const SpatialState &s = ps.base.humanoid.spatial;
     const int t = w.playerTeamID[p];
@@ -70,7 +72,9 @@ HDN void CalculateTacticalSituation(World &w, int p) {
 HD bool TeamHasUniquePossession(const World &w, int teamID) {
     return TeamByID(w, teamID).hasPossession && !TeamByID(w, 1 - teamID).hasPossession;
 }
-HDN void ControllerCalculateSituation(World &w, int p, PlayerControllerState &ctl) {
+HDN void ControllerCalculateSituation(GlobalRef<World> world, int p, GlobalRef<PlayerControllerState> controller) {
+    World &w = world;
+    PlayerControllerState &ctl = controller;
     const MatchState &m = w.match;
     const Player &ps = m.players[p];
     const int t = w.playerTeamID[p];
@@ -142,7 +146,9 @@ HD void ArmGamerAction(World &w, int p, HumanControllerState &hc) {
 // difficulty; none right after its own touch), the steady direction, the situation, the armed
 // action and, for a pass or shot, its gauge (10 ms a tick while held, 10 to 1000 ms) or the time
 // since release. The switch button with the ball starts an attacking run.
-HDN bool HumanControllerProcess(World &w, const Ctx &c, int p) {
+HDN bool HumanControllerProcess(GlobalRef<World> world, LocalRef<const Ctx> context, int p) {
+    World &w = world;
+    const Ctx &c = context;
     MatchState &m = w.match;
     HumanControllerState &hc = HumanGamerOf(w, p).controller;
     PlayerControllerState &ctl = hc.base;
@@ -174,7 +180,10 @@ HDN bool HumanControllerProcess(World &w, const Ctx &c, int p) {
 // ---- the humanoid tick of a player ------------------------------------------------------------------
 
 // Whether a player may drop its animation for a fresh command this tick (GRF's requeue).
-HDN bool MayRequeue(World &w, const Ctx &c, int p, const Anim &a, int k) {
+HDN bool MayRequeue(GlobalRef<World> world, LocalRef<const Ctx> context, int p, GlobalRef<const Anim> animation, int k) {
+    World &w = world;
+    const Ctx &c = context;
+    const Anim &a = animation;
     const Player &ps = w.match.players[p];
     const Humanoid &h = ps.base.humanoid;
     const AnimationState &cur = h.anim;
@@ -234,7 +243,10 @@ HD PassAim RefinePassAim(World &w, int p, const AnimationState &cur) {
 // A pass's touch: the refined aim's receiver selected (when there is one), 36 m/s per unit of
 // power plus 0.3, made attainable, and curled away from the body (a fifth as much for a high
 // pass), with the matching z spin.
-HDN bool PassTouch(World &w, const Ctx &c, int p, const AnimationState &cur, Vec3 &touch, float &zRot) {
+HDN bool PassTouch(GlobalRef<World> world, LocalRef<const Ctx> context, int p, GlobalRef<const AnimationState> animationState, Vec3 &touch, float &zRot) {
+    World &w = world;
+    const Ctx &c = context;
+    const AnimationState &cur = animationState;
     const Humanoid &h = Hum(w, p);
     const PassAim aim = RefinePassAim(w, p, cur);
     if (aim.target >= 0 && !TeamSelectPlayer(w, c, w.playerTeamID[p], aim.target)) return false;
@@ -293,7 +305,11 @@ HD void DeflectionOutcome(World &w, const Ctx &c, int p, const AnimDerived &d, T
 // The touch, the spin and the record have one call site each, so that matches of a wavefront
 // touching the ball in different ways run the ball's new prediction together; per environment the
 // calls and their order are GRF's.
-HDN bool AnimationTouch(World &w, const Ctx &c, int p, const Anim &a, const AnimDerived &d, float bumpy) {
+HDN bool AnimationTouch(GlobalRef<World> world, LocalRef<const Ctx> context, int p, GlobalRef<const Anim> animation, GlobalRef<const AnimDerived> derivedTerms, float bumpy) {
+    World &w = world;
+    const Ctx &c = context;
+    const Anim &a = animation;
+    const AnimDerived &d = derivedTerms;
     Player &ps = w.match.players[p];
     Humanoid &h = ps.base.humanoid;
     const AnimationState &cur = h.anim;
@@ -356,7 +372,9 @@ HDN bool AnimationTouch(World &w, const Ctx &c, int p, const Anim &a, const Anim
 // whether the animation is interrupted, the interruption (command request and animation
 // selection, the expensive part), and the rest. Run in that order they are the whole tick; the
 // team loop lets the matches of a wavefront meet at the interruption.
-HDN void HumanoidProcessBegin(World &w, const Ctx &c, int p) {
+HDN void HumanoidProcessBegin(GlobalRef<World> world, LocalRef<const Ctx> context, int p) {
+    World &w = world;
+    const Ctx &c = context;
     ENG_SCOPE(12);
     Player &ps = w.match.players[p];
     Humanoid &h = ps.base.humanoid;
@@ -378,7 +396,9 @@ HDN void HumanoidProcessBegin(World &w, const Ctx &c, int p) {
         if (h.interruptAnim == kIntNone && MayRequeue(w, c, p, a, k)) h.interruptAnim = kIntReQueue;
     }
 }
-HDN bool HumanoidProcessInterrupt(World &w, const Ctx &c, int p) {
+HDN bool HumanoidProcessInterrupt(GlobalRef<World> world, LocalRef<const Ctx> context, int p) {
+    World &w = world;
+    const Ctx &c = context;
     Humanoid &h = w.match.players[p].base.humanoid;
     AnimationState &cur = h.anim;
     {
@@ -469,7 +489,7 @@ HD bool TouchAtTouchFrame(World &w, const Ctx &c, int p, const Anim &a, const An
     const AnimationState &cur = Hum(w, p).anim;
     float animationBallHeight = 0;
     for (int i = 0; i < a.footballCount; i++) {
-        const FootballKey &fk = c.t->football[a.footballFirst + i];
+        const FootballKey &fk = c.T().football[a.footballFirst + i];
         if (fk.frame == cur.touchFrame) animationBallHeight = fk.position.v[2];
     }
     float reach = 0.4f;
@@ -568,7 +588,9 @@ HD void FillApplyBuffer(Humanoid &h) {
 }
 // The rest of a humanoid's tick: controlled collisions, the touch, the retained ball, the
 // smuggles of the frame, the keeper's box and the apply buffer.
-HDN bool HumanoidProcessEnd(World &w, const Ctx &c, int p) {
+HDN bool HumanoidProcessEnd(GlobalRef<World> world, LocalRef<const Ctx> context, int p) {
+    World &w = world;
+    const Ctx &c = context;
     Player &ps = w.match.players[p];
     Humanoid &h = ps.base.humanoid;
     AnimationState &cur = h.anim;

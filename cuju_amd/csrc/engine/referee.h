@@ -12,8 +12,8 @@
 namespace eng {
 
 // Defined with the set pieces.
-HDN bool LeftTeamStartsNearerBall(const World &w);
-HDN bool RefereeRestart(World &w, const Ctx &c, int setPiece);
+HDN bool LeftTeamStartsNearerBall(GlobalRef<const World> world);
+HDN bool RefereeRestart(GlobalRef<World> world, LocalRef<const Ctx> context, int setPiece);
 
 enum MatchPhase { kPreMatch, kFirstHalf, kSecondHalf };
 
@@ -34,7 +34,9 @@ HD Vec3 PitchPosition(const World &w, int p) {
 }
 
 // Advances the clocks by `ms`; the match clock runs at the scenario's pace while in play.
-HDN void BumpActualTime(World &w, const Ctx &c, uint64_t ms) {
+HDN void BumpActualTime(GlobalRef<World> world, LocalRef<const Ctx> context, uint64_t ms) {
+    World &w = world;
+    const Ctx &c = context;
     MatchState &m = w.match;
     if (m.inPlay) m.matchTimeMs = (uint64_t)((float)m.matchTimeMs + ms * (1.0f / c.sd->matchDurationFactor));
     m.actualTimeMs += ms;
@@ -72,7 +74,9 @@ HD void ResetFoul(Foul &f) {
     f.hasBeenProcessed = true;
 }
 // GRF without referee animations: the clock skips the wait of a stoppage at once.
-HDN void RefereeStop(World &w, const Ctx &c, int setPiece, uint64_t extraPrepareMs = 0) {
+HDN void RefereeStop(GlobalRef<World> world, LocalRef<const Ctx> context, int setPiece, uint64_t extraPrepareMs = 0) {
+    World &w = world;
+    const Ctx &c = context;
     MatchState &m = w.match;
     RefereeBuffer &b = m.referee.buffer;
     m.inPlay = false;
@@ -136,7 +140,9 @@ HD void AwardFoul(World &w, const Ctx &c, Foul &f, bool penalty) {
 }
 // The referee's look at the pending foul: the advantage reviewed, then a foul without advantage
 // not yet processed is awarded. True when it stops play.
-HDN bool RefereeCheckFoul(World &w, const Ctx &c) {
+HDN bool RefereeCheckFoul(GlobalRef<World> world, LocalRef<const Ctx> context) {
+    World &w = world;
+    const Ctx &c = context;
     Foul &f = w.match.referee.foul;
     const bool penalty = FoulInPenaltyArea(w, f);
     ReviewAdvantage(w, f, penalty);
@@ -253,7 +259,9 @@ HD bool EndSetPieceWhenTaken(World &w) {
 // During a stoppage: the set piece is prepared at its preparation time (the world RNG reseeded;
 // the first half begins at the match's opening kick-off) and play resumes, as a set piece, at its
 // start time. Then a set piece in progress may end, and the relaxation runs down.
-HDN bool RefereeProcess(World &w, const Ctx &c) {
+HDN bool RefereeProcess(GlobalRef<World> world, LocalRef<const Ctx> context) {
+    World &w = world;
+    const Ctx &c = context;
     ENG_SCOPE(6);
     MatchState &m = w.match;
     Referee &ref = m.referee;
@@ -328,7 +336,9 @@ HD void RecordOffsidePositions(World &w, int attackers) {
 }
 // The referee's part of a touch, with offsides on: punish a touch by a player recorded offside,
 // then record the offside positions at this touch.
-HDN bool RefereeBallTouched(World &w, const Ctx &c) {
+HDN bool RefereeBallTouched(GlobalRef<World> world, LocalRef<const Ctx> context) {
+    World &w = world;
+    const Ctx &c = context;
     if (!w.scenario.offsides) return true;
     const int attackers = w.match.lastTouchTeamID;
     if (attackers == -1) return true;
@@ -416,7 +426,9 @@ HD void DeflectBall(World &w, const Ctx &c, Vec3 bounce, int bounces, float dept
 // the team's designated player, when nobody touched the ball within 200 ms, control it;
 // otherwise it records an accidental touch and adds a bounce (away from the part, blended with
 // the player's movement by how recently the opponents touched) and a contact depth.
-HDN bool CheckBallCollisions(World &w, const Ctx &c) {
+HDN bool CheckBallCollisions(GlobalRef<World> world, LocalRef<const Ctx> context) {
+    World &w = world;
+    const Ctx &c = context;
     ENG_SCOPE(5);
     MatchState &m = w.match;
     if (m.actualTimeMs <= (uint64_t)(uint32_t)(m.lastBodyBallCollisionTimeMs + 150)) return true;
@@ -459,7 +471,8 @@ HDN bool CheckBallCollisions(World &w, const Ctx &c) {
     return true;
 }
 
-HDN void RefereeTripNotice(World &w, int tripped, int tripping, int tackleType) {
+HDN void RefereeTripNotice(GlobalRef<World> world, int tripped, int tripping, int tackleType) {
+    World &w = world;
     MatchState &m = w.match;
     Referee &ref = m.referee;
     if (ref.buffer.active) return;
@@ -508,7 +521,9 @@ HDN void RefereeTripNotice(World &w, int tripped, int tripping, int tackleType) 
     }
 }
 
-HDN void TripMe(World &w, const Ctx &c, int p, const Vec3 &tripVector, int tripType) {
+HDN void TripMe(GlobalRef<World> world, LocalRef<const Ctx> context, int p, Vec3 tripVector, int tripType) {
+    World &w = world;
+    const Ctx &c = context;
     if (w.match.ballRetainer == p) return;
     Humanoid &h = Hum(w, p);
     const Anim &a = c.A(h.anim.anim);
@@ -527,7 +542,10 @@ HD bool BoxesIntersect(const Aabb &a, const Aabb &o) {
     return (o.lo.v[0] < a.hi.v[0] && o.lo.v[1] < a.hi.v[1] && o.lo.v[2] < a.hi.v[2]) &&
            (o.hi.v[0] > a.lo.v[0] && o.hi.v[1] > a.lo.v[1] && o.hi.v[2] > a.lo.v[2]);
 }
-HDN void PlayerGeometries(const World &w, const Ctx &c, int p, PlayerGeometryList &out) {
+HDN void PlayerGeometries(GlobalRef<const World> world, LocalRef<const Ctx> context, int p, GlobalRef<PlayerGeometryList> geometries) {
+    const World &w = world;
+    const Ctx &c = context;
+    PlayerGeometryList &out = geometries;
     const Skeleton &sk = c.skeletons[p];
     Transform der[kHumanoidNodes];
     WorldTransforms(sk, Hum(w, p).nodes, der);
@@ -714,7 +732,11 @@ HD void TackleContact(World &w, const Ctx &c, int p1, int p2, float dist) {
     }
 }
 // One pair's contact, in GRF's order: push apart, drag, trips in the push, then the tackle.
-HDN void CheckHumanoidCollision(World &w, const Ctx &c, int p1, int p2, PlayerBounceList &b1, PlayerBounceList &b2) {
+HDN void CheckHumanoidCollision(GlobalRef<World> world, LocalRef<const Ctx> context, int p1, int p2, GlobalRef<PlayerBounceList> bounces, GlobalRef<PlayerBounceList> b2Ref) {
+    World &w = world;
+    const Ctx &c = context;
+    PlayerBounceList &b1 = bounces;
+    PlayerBounceList &b2 = b2Ref;
     const Contact k = MakeContact(w, p1, p2);
     if (k.dist < kContactBody * 2.0f) PushApart(w, c, k);
     if (k.dist < (kContactBody + kContactShell) * 2.0f) Drag(w, c, k, b1, b2);
@@ -722,7 +744,9 @@ HDN void CheckHumanoidCollision(World &w, const Ctx &c, int p1, int p2, PlayerBo
     TackleContact(w, c, p1, p2, k.dist);
 }
 
-HDN bool CheckHumanoidCollisions(World &w, const Ctx &c) {
+HDN bool CheckHumanoidCollisions(GlobalRef<World> world, LocalRef<const Ctx> context) {
+    World &w = world;
+    const Ctx &c = context;
     ENG_SCOPE(17);
     PlayerList ps = PlayersInProcessingOrder(w);
     PlayerBounceList *const bounces = c.ws->bounces;

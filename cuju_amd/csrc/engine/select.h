@@ -17,7 +17,7 @@ enum SelectResult { kSelectFalse = 0, kSelectTrue = 1, kSelectUnsupported = 2 };
 
 // A candidate list in scratch memory.
 struct AList {
-    int16_t *e;
+    GlobalPointer<int16_t> e;
     int32_t count;
     HD int size() const { return count; }
     HD bool empty() const { return count == 0; }
@@ -30,7 +30,7 @@ struct AList {
 };
 // A planned position list in scratch memory.
 struct PList {
-    Vec3 *e;
+    GlobalPointer<Vec3> e;
     int32_t count;
     HD int size() const { return count; }
     HD Vec3 &operator[](int i) { return e[i]; }
@@ -112,7 +112,7 @@ HD float PreferredAngle(int i) {
     const double f[11] = {0, 0.111, -0.111, 0.25, -0.25, 0.5, -0.5, 0.75, -0.75, 0.999, -0.999};
     return (float)(f[i] * (double)PI);
 }
-HDN Vec3 SnapToPreferredDirection(const Vec3 &src) {
+HDN Vec3 SnapToPreferredDirection(Vec3 src) {
     float best = -1.0f;
     Vec3 bv;
     for (int i = 0; i < 11; i++) {
@@ -176,7 +176,8 @@ HD Vec3 FootReachOffset(float velocity, float bodyAngleRel, float height) {
 // Stable sort of `list` by precomputed keys (doubles hold float and int keys exactly, so `<` on
 // them orders as on the original type). Any stable sort of a strict weak order without NaN gives
 // GRF's std::stable_sort order.
-HDN void StableSortByKeys(const Ctx &c, AList &list) {
+HDN void StableSortByKeys(LocalRef<const Ctx> context, AList &list) {
+    const Ctx &c = context;
     ENG_SCOPE(33);
     const int n = list.count;
     double *keys = c.ws->keys;
@@ -417,11 +418,12 @@ HD bool IncomingBodyPasses(const BodyRule &rule, int entry, const Vec3 &directio
 // body-prefiltered record lists (Tables::crudeBody).
 constexpr int kBodyEntries = 6;
 
-HDN void FilterAnimations(const Ctx &c, const CrudeQuery &query, AList &out) {
+HDN void FilterAnimations(LocalRef<const Ctx> context, const CrudeQuery &query, AList &out) {
+    const Ctx &c = context;
     ENG_SCOPE(28);
     // The query, the tables' bounds and the list held in registers across the list's stores.
     const CrudeQuery q = query;
-    const Tables &T = *c.t;
+    const Tables &T = c.T();
     const float maxIncomingBallDeviation = T.maxIncomingBallDeviation.value();
     const float maxOutgoingBallDeviation = T.maxOutgoingBallDeviation.value();
     int16_t *const kept = out.e;
@@ -525,7 +527,7 @@ HDN void FilterAnimations(const Ctx &c, const CrudeQuery &query, AList &out) {
         }
         return true;
     };
-    const CrudeRecord *records = list ? T.crude + T.fnOffset[q.functionType] : T.crudeByIndex;
+    const CrudeRecord *records = list ? T.crude + T.fnOffset[q.functionType] : T.crudeByIndex.get();
     // A query with its function type's velocity rule reads the animations of that type that pass
     // the velocity test, prefiltered in list order.
     if (list && q.byIncomingVelocity && q.incomingVelocity >= kVelIdle && q.incomingVelocity <= kVelSprint &&
@@ -591,7 +593,8 @@ HD float MovementSimilarityOf(const Vec3 &outDir, const Vec3 &outMov, const Vec3
     return v;
 }
 
-HDN float DirectionSimilarityRating(const Anim &a, const Predicates &p, const Vec3 &relLookAt) {
+HDN float DirectionSimilarityRating(GlobalRef<const Anim> animation, const Predicates &p, Vec3 relLookAt) {
+    const Anim &a = animation;
     Vec3 relBody = (relLookAt - a.translation).Normalized(Vec3(0, -1, 0));
     float maxSmuggle = 0.1f * PI;
     float outAngle = a.outgoingDirection.Rotated2D(Clamp(p.relDesiredDirection.Angle2D(a.outgoingDirection), -maxSmuggle, maxSmuggle))
@@ -619,7 +622,8 @@ HD float KeyIncomingVelocity(const Anim &a, const Predicates &p) {
 }
 
 // The search compares Length; the result is GetDistance.
-HDN float ClosestOpponentDistance(const World &w, int p) {
+HDN float ClosestOpponentDistance(GlobalRef<const World> world, int p) {
+    const World &w = world;
     const int opp = 1 - w.playerTeamID[p];
     const Vec3 pos = Sp(w, p).position;
     float best = 10000;
@@ -792,8 +796,8 @@ struct MovementPlanner {
           playerMaxVel = 0, desiredVel = 0;
     FrameLag lag;
     Vec3 desiredDir, outgoingTurned;
-    const Vec3 *smoothed = nullptr;  // the animation's smoothed movement, when tabulated
-    const Vec3 *positions = nullptr;
+    GlobalPointer<const Vec3> smoothed = nullptr;  // the animation's smoothed movement, when tabulated
+    GlobalPointer<const Vec3> positions = nullptr;
     // What carries from frame to frame.
     Vec3 velocity, position;
 
@@ -1013,7 +1017,7 @@ HD TouchReach KeyReach(int fn, float awkward, bool preferPassAndShot) {
 // What one touch search reads, fixed for its candidates.
 struct TouchSearch {
     MentalBallView mental;
-    const Vec3 *predictions;
+    GlobalPointer<const Vec3> predictions;
     bool flip, retainerIsMe, preferPassAndShot, useDesiredMovement;
     int fn;
     libm::SinCos back;  // turns pitch directions into the body's frame
@@ -1058,8 +1062,8 @@ struct TouchProbe {
 };
 
 struct Selector {
-    World &w;
-    const Ctx &c;
+    GlobalRef<World> world;
+    LocalRef<const Ctx> context;
     int hi;  // humanoid index: a player, or playerCount + official
     Predicates pred;
     struct TurnCache {
@@ -1068,7 +1072,7 @@ struct Selector {
         libm::SinCos t{};
     } fwd, back;
 
-    HD Selector(World &world, const Ctx &ctx, int index) : w(world), c(ctx), hi(index) {}
+    HD Selector(World &w, const Ctx &c, int index) : world(w), context(c), hi(index) {}
 
     HD static libm::SinCos Cached(TurnCache &tc, float angle, float arg) {
         uint32_t b = BitsOf(angle);
@@ -1082,16 +1086,42 @@ struct Selector {
     HD libm::SinCos Turn(float a) { return Cached(fwd, a, a); }
     HD libm::SinCos BackTurn(float a) { return Cached(back, a, -a); }
 
-    HD bool Official() const { return hi >= w.match.playerCount; }
-    HD Player &P() { return w.match.players[hi]; }
-    HD Humanoid &H() { return Official() ? w.match.officials[hi - w.match.playerCount].humanoid : P().base.humanoid; }
+    HD bool Official() const {
+        World &w = world;
+        return hi >= w.match.playerCount;
+    }
+    HD Player &P() {
+        World &w = world;
+        return w.match.players[hi];
+    }
+    HD Humanoid &H() {
+        World &w = world;
+        return Official() ? w.match.officials[hi - w.match.playerCount].humanoid : P().base.humanoid;
+    }
     HD SpatialState &S() { return H().spatial; }
-    HD const Anim &A(int i) const { return c.t->anims[i]; }
-    HD const AnimDerived &D(int i) const { return c.t->derived[i]; }
-    HD int MentalImg() { return MentalImageIndex(w, H().mentalImageTime); }
-    HD Vec3 MentalBallAt(int ms) { return MentalBallPrediction(w, MentalImg(), ms); }
-    HD float Statistic(int s) { return Official() ? c.sd->data[hi].stats[s] : GetStatistic(w, c, hi, s); }
+    HD const Anim &A(int i) const {
+        const Ctx &c = context;
+        return c.T().anims[i];
+    }
+    HD const AnimDerived &D(int i) const {
+        const Ctx &c = context;
+        return c.T().derived[i];
+    }
+    HD int MentalImg() {
+        World &w = world;
+        return MentalImageIndex(w, H().mentalImageTime);
+    }
+    HD Vec3 MentalBallAt(int ms) {
+        World &w = world;
+        return MentalBallPrediction(w, MentalImg(), ms);
+    }
+    HD float Statistic(int s) {
+        World &w = world;
+        const Ctx &c = context;
+        return Official() ? c.sd->data[hi].stats[s] : GetStatistic(w, c, hi, s);
+    }
     HD float BaseLastTouchBias(int decayMs) {
+        World &w = world;
         uint64_t last = Official() ? w.match.officials[hi - w.match.playerCount].lastTouchTimeMs : P().base.lastTouchTimeMs;
         if (decayMs > 0) return 1.0f - Clamp((float)(w.match.actualTimeMs - last) / (float)decayMs, 0.0f, 1.0f);
         return 0.0f;
@@ -1099,23 +1129,32 @@ struct Selector {
     HD Vec3 RelativeLookAt() { return RotatedBy(pred.lookAt - S().position, BackTurn(S().angle.value())); }
 
     HD float MovementSimilarityKey(int i) {
-        const SelectionRecord &r = c.t->selection[i];
+        const Ctx &c = context;
+        const SelectionRecord &r = c.T().selection[i];
         return MovementSimilarityOf(r.preferredOutgoingDirection, r.preferredOutgoingMovement, pred.relDesiredDirection,
                                     pred.desiredVelocity, pred.corneringBias);
     }
     HD int IncomingBodyDirectionQuery() { return BodyDirectionIndex(pred.relIncomingBodyDirection); }
     HD float IncomingBodyDirectionKey(int i, int q) {
-        float r = AllowedBodyDirectionKey(c.t->selection[i].incomingBodyIndex, q);
+        const Ctx &c = context;
+        float r = AllowedBodyDirectionKey(c.T().selection[i].incomingBodyIndex, q);
         if (VelocityCat(A(i).incomingVelocity) == kVelIdle) r = 0;
         return r;
     }
-    HD float PreferredOutgoingAngle(int i) { return c.t->selection[i].preferredOutgoingAngle; }
-    HD float LookAngle(int i) { return c.t->selection[i].lookAngle; }
+    HD float PreferredOutgoingAngle(int i) {
+        const Ctx &c = context;
+        return c.T().selection[i].preferredOutgoingAngle;
+    }
+    HD float LookAngle(int i) {
+        const Ctx &c = context;
+        return c.T().selection[i].lookAngle;
+    }
     HD Vec3 SmoothedMovement(int i, uint32_t frame) {
+        const Ctx &c = context;
         const Anim &a = A(i);
-        int32_t first = c.t->selection[i].smoothedFirst;
-        if (first >= 0 && frame < (uint32_t)a.posCount) return c.t->smoothed[first + frame];
-        return MovementAtFrame(c.t->positions + a.posFirst, a.posCount, frame, 1);
+        int32_t first = c.T().selection[i].smoothedFirst;
+        if (first >= 0 && frame < (uint32_t)a.posCount) return c.T().smoothed[first + frame];
+        return MovementAtFrame(c.T().positions + a.posFirst, a.posCount, frame, 1);
     }
 
     HD void SetMovementSimilarityPredicate(const Vec3 &relDesired, int desiredVel) {
@@ -1128,6 +1167,7 @@ struct Selector {
     // Keys are computed into scratch, then a stable sort permutes the list.
     template <class KeyFn>
     HD void Sort(AList &l, KeyFn key) {
+        const Ctx &c = context;
         if (l.count < 2) return;
         for (int i = GroupRank(); i < l.count; i += kGroupLanes) c.ws->keys[i] = (double)key((int)l[i]);
         GroupSync();
@@ -1237,10 +1277,12 @@ struct Selector {
     }
 
     HD bool AllowLastDitch(bool withPossessionAmount = true) {
+        World &w = world;
         if (withPossessionAmount && TeamOfPlayer(w, hi).teamPossessionAmount < 1.0f) return true;
         return ((int)P().timeToBallOptimisticMs * 1.7f + 800 < (float)(int)P().timeToBallMs);
     }
     HD bool HighOrBouncyBall() {
+        World &w = world;
         const Ball &b = w.match.ball;
         float hn = BallPredict(b, 10).v[2], ht = BallPredict(b, kDefaultTouchOffsetMs).v[2];
         float bounce = fabsf(b.momentum.v[2]);
@@ -1249,16 +1291,18 @@ struct Selector {
         return false;
     }
 
-    HDN void KeepNearestQuadrant(AList &l, const PlayerCommand &cmd, bool strict, float allowedAngle = 0,
+    HDN void KeepNearestQuadrant(AList &l, GlobalRef<const PlayerCommand> command, bool strict, float allowedAngle = 0,
                                          int allowedVelocitySteps = 0, int forcedQuadrant = -1) {
+        const PlayerCommand &cmd = command;
+        const Ctx &c = context;
         ENG_SCOPE(32);
         if (l.empty()) return;
         int bestQ = forcedQuadrant;
         auto keeps = [&](int ai) {
             const Anim &a = A(ai);
             if (strict) return a.quadrantID == bestQ;
-            const Quadrant &bq = c.t->quadrants[bestQ];
-            const Quadrant &qd = c.t->quadrants[a.quadrantID];
+            const Quadrant &bq = c.T().quadrants[bestQ];
+            const Quadrant &qd = c.T().quadrants[a.quadrantID];
             bool keep = true;
             if (!a.lastDitch) {
                 int dv = VelocityRank(qd.velocity, true) - VelocityRank(bq.velocity, true);
@@ -1286,7 +1330,8 @@ struct Selector {
         l.count = kept;
     }
 
-    HDN void KeepNearestLook(AList &l, const PlayerCommand &cmd, bool strict, float allowedAngle = 0) {
+    HDN void KeepNearestLook(AList &l, GlobalRef<const PlayerCommand> command, bool strict, float allowedAngle = 0) {
+        const PlayerCommand &cmd = command;
         ENG_SCOPE(32);
         if (l.empty()) return;
         Vec3 relLookAt;
@@ -1303,8 +1348,9 @@ struct Selector {
     }
 
     HDN int IdleMovementAnimation() {
+        const Ctx &c = context;
         // The crude selection of IdleMovementQuery, made once from the tables; only read here.
-        const AList l{const_cast<int16_t *>(c.t->idleMovement), c.t->idleMovementCount};
+        const AList l{const_cast<int16_t *>(c.T().idleMovement.get()), c.T().idleMovementCount};
         pred.idle = 1;
         pred.relIncomingBodyDirection = Vec3(0, -1, 0);
         pred.incomingVelocity = kVelIdle;
@@ -1329,8 +1375,9 @@ struct Selector {
     // ends with and sets `rotationOffset`, the turn the plan adds to the animation's outgoing angle.
     // `together`: every lane of the match makes this call with the same arguments, and they share
     // the frames' terms; otherwise a lane plans alone.
-    HDN Vec3 PlanMovement(int ai, bool useDesiredMovement, const Vec3 &desiredMovement, const Vec3 &desiredBodyRel, PList &out,
+    HDN Vec3 PlanMovement(int ai, bool useDesiredMovement, Vec3 desiredMovement, Vec3 desiredBodyRel, PList &out,
                           float &rotationOffset, bool together) {
+        const Ctx &c = context;
         ENG_SCOPE(38);
         const Anim &a = A(ai);
         const AnimDerived &d = D(ai);
@@ -1375,9 +1422,9 @@ struct Selector {
         plan.settleFrom = a.frameCount - 2;
         plan.outgoingIdle = VelocityCat(a.outgoingVelocity) == kVelIdle;
         plan.outgoingTurned = RotatedBy(a.outgoingMovement, plan.turn);
-        const int32_t smoothedFirst = c.t->selection[ai].smoothedFirst;
-        plan.smoothed = smoothedFirst >= 0 ? c.t->smoothed + smoothedFirst : nullptr;
-        plan.positions = c.t->positions + a.posFirst;
+        const int32_t smoothedFirst = c.T().selection[ai].smoothedFirst;
+        plan.smoothed = smoothedFirst >= 0 ? c.T().smoothed + smoothedFirst : nullptr;
+        plan.positions = c.T().positions + a.posFirst;
         plan.posCount = a.posCount;
         Vec3 *const frames = out.e;
         const int frameCount = a.frameCount;
@@ -1404,7 +1451,9 @@ struct Selector {
     // the humanoid's movement (its own blended with the animation's) and the ball's (as seen 240
     // to 250 ms ahead) differ by 2 m/s or more, in speed beyond -1.4 to 0.7 m/s, or, for an
     // animation that leaves moving, in direction.
-    HDN bool BallControlNeedsTouch(int ai, const PlayerCommand &cmd) {
+    HDN bool BallControlNeedsTouch(int ai, GlobalRef<const PlayerCommand> command) {
+        const PlayerCommand &cmd = command;
+        World &w = world;
         const Anim &a = A(ai);
         const SpatialState &s = S();
         if (cmd.desiredVelocityFloat > kIdleDribbleSwitch || fabsf(w.match.ball.momentum.Length()) > 2.0f) return true;
@@ -1443,6 +1492,7 @@ struct Selector {
     // the match and of its team, in play, with no set piece, retainer, touch, special state or
     // trip other than of type one.
     HD bool SteersTowardBall() {
+        World &w = world;
         const AnimationState &cur = H().anim;
         const Anim &a = A(cur.anim);
         const MatchState &m = w.match;
@@ -1489,6 +1539,7 @@ struct Selector {
     }
 
     HD float LastTouchBiasAt(int decayMs, uint64_t t) {
+        World &w = world;
         uint64_t at = t;
         if (t == 0) at = w.match.actualTimeMs;
         if (decayMs > 0) return 1.0f - Clamp((float)(at - P().base.lastTouchTimeMs) / (float)decayMs, 0.0f, 1.0f);
@@ -1508,13 +1559,14 @@ struct Selector {
     // the body reaches (TouchProbe).
     HDN bool TryTouchAnimation(const TouchSearch &ts, int ai, PList &plan, float &rotSmuggle, float &predAngle, Vec3 &outMov,
                                Vec3 &smuggle, int &touchFrame) {
+        const Ctx &c = context;
         const Anim &a = A(ai);
         PlanMovement(ai, ts.useDesiredMovement, ts.desiredMovement, ts.desiredBodyRel, plan, rotSmuggle, false);
         predAngle = ModulateIntoRange(-PI, PI, a.outgoingAngle.value() + rotSmuggle);
         outMov = RotatedBy(OutgoingMovementOf(plan), ts.back);
         const int total = a.footballCount, middle = total / 2;
         for (int tn = 0; tn < total; tn++) {
-            const FootballKey &key = c.t->football[a.footballFirst + (tn <= middle ? middle - tn : tn)];
+            const FootballKey &key = c.T().football[a.footballFirst + (tn <= middle ? middle - tn : tn)];
             if (!ts.retainerIsMe && !BallOnPitchAt(ts.predictions, ts.flip, key.frame)) continue;
             const TouchProbe probe = ProbeKey(ts, a, D(ai).touchFrame, key, plan, outMov, predAngle);
             if (probe.reaches) {
@@ -1532,8 +1584,9 @@ struct Selector {
     // must lie within the reach (TouchReach) of the animation's ball (BallWithinReach).
     HD TouchProbe ProbeKey(const TouchSearch &ts, const Anim &a, int defaultTouchFrame, const FootballKey &key, const PList &plan,
                            const Vec3 &outMov, float predAngle) {
+        const Ctx &c = context;
         const int tf = key.frame;
-        const Vec3 touchMov = RotatedBy(MovementAtFrame(plan.e, plan.count, tf, 0), ts.back);
+        const Vec3 touchMov = RotatedBy(MovementAtFrame(plan.e.get(), plan.count, tf, 0), ts.back);
         const Vec3 ballNow = ts.mental.At(tf * 10);
         const Vec3 ballMov = RotatedBy((ts.mental.At(tf * 10 + 10) - ballNow) * 100.0f, ts.back);
         const Vec3 ballAt = RotatedBy(ballNow - ts.position, ts.back);
@@ -1579,9 +1632,11 @@ struct Selector {
     // candidate, in list order, whose plan brings a ball key to the ball. Returns it (-1 for none)
     // with its plan, touch frame and position, the smuggle that moves the body onto the ball and
     // the plan's rotation offset.
-    HDN int FindTouchAnimation(const AList &sorted, bool useDesiredMovement, const Vec3 &desiredDir, float desiredVel,
-                               const Vec3 &desiredBodyRel, PList &positions, int &touchFrameOut, Vec3 &touchPosOut,
+    HDN int FindTouchAnimation(const AList &sorted, bool useDesiredMovement, Vec3 desiredDir, float desiredVel,
+                               Vec3 desiredBodyRel, PList &positions, int &touchFrameOut, Vec3 &touchPosOut,
                                Vec3 &actionSmuggleOut, float &rotationSmuggleOut, bool preferPassAndShot = false) {
+        World &w = world;
+        const Ctx &c = context;
         ENG_SCOPE(31);
         const MatchState &m = w.match;
         const SpatialState &s = S();
@@ -1601,7 +1656,7 @@ struct Selector {
             if (ts.retainerIsMe) return true;
             const Anim &a = A(ai);
             for (int key = 0; key < a.footballCount; key++) {
-                const FootballKey &fk = c.t->football[a.footballFirst + key];
+                const FootballKey &fk = c.T().football[a.footballFirst + key];
                 const int tf = fk.frame;
                 if (!BallOnPitchAt(ts.predictions, ts.flip, tf)) continue;
                 const float m0 = ts.mental.At(tf * 10).v[2], m1 = ts.mental.At(tf * 10 + 10).v[2];
@@ -1673,6 +1728,7 @@ struct Selector {
     // shortens, by at most what a slow, late touch allows; less near an opponent.
     HD Vec3 ShapeActionSmuggle(const TouchSearch &ts, const Vec3 &gap, float ballHeight, float outgoingAngle, float outSpeed,
                                int touchFrame) {
+        World &w = world;
         float keep = 1.0f - 0.4f * (ts.fn != kFnBallControl ? 0.8f : 1.0f) * (ballHeight > 0.5f ? 0.7f : 1.0f) *
                                 (ballHeight > 1.0f ? 0.7f : 1.0f);
         float length = Clamp(gap.Length() - (0.02f + (ts.fn == kFnInterfere ? 0.1f : 0.0f)), 0.0f, (float)100.0);
@@ -1719,7 +1775,7 @@ struct Selector {
         cur.incomingMovement = s.movement;
         cur.outgoingMovement = OutgoingMovementOf(positions);
         // The plan fits the list: both hold kAnimPositions entries.
-        GroupCopy<4>(cur.positions.e, positions.e, positions.count);
+        GroupCopy<4>(cur.positions.e, positions.e.get(), positions.count);
         cur.positions.count = positions.count;
         cur.positionOffset = Vec3(0);
         cur.originatingCommand = cmd;
@@ -1741,6 +1797,7 @@ struct Selector {
 
     // The crude query of an official's command: strict incoming velocity and body direction.
     HD CrudeQuery OfficialQuery(const PlayerCommand &cmd, int fn) {
+        World &w = world;
         const SpatialState &s = S();
         CrudeQuery q;
         q.byFunctionType = true;
@@ -1760,7 +1817,9 @@ struct Selector {
     // An official's animation for a command (GRF's HumanoidBase::SelectAnimation): for movement,
     // trips and specials, the first candidate of the query by the ranking, with its movement plan;
     // other function types select nothing.
-    HDN SelectResult SelectOfficialAnimation(const PlayerCommand &cmd, int interrupt) {
+    HDN SelectResult SelectOfficialAnimation(GlobalRef<const PlayerCommand> command, int interrupt) {
+        const PlayerCommand &cmd = command;
+        const Ctx &c = context;
         AnimationState &cur = H().anim;
         const SpatialState &s = S();
         const int fn = cmd.desiredFunctionType;
@@ -1806,6 +1865,7 @@ struct Selector {
     // further from where the humanoid will be then than it is now; or, for the non-retainer and
     // all but deflections, seen more than 2 m from where it will be a second ahead.
     HD bool BallOutOfTouchRange(int fn, bool retainerIsMe) {
+        World &w = world;
         const SpatialState &s = S();
         const bool needsBall = fn != kFnMovement && fn != kFnTrip && fn != kFnSpecial && fn != kFnSliding;
         if (!needsBall) return false;
@@ -1826,6 +1886,7 @@ struct Selector {
     // command close to what it already plans; movement stays against ball control just after a
     // kick of the player's own ball, unless the velocity changes by 1 m/s or more.
     HD bool RequeueKeepsCurrent(const PlayerCommand &cmd, int fn) {
+        World &w = world;
         const Player &player = P();
         const Humanoid &h = H();
         const AnimationState &cur = h.anim;
@@ -1966,6 +2027,7 @@ struct Selector {
     // The idle level a player's candidates are ranked by: 1 at a set piece or with the ball more
     // than 16 m away in 200 ms, else 2 out of play and 0 in play.
     HD int IdleLevel() {
+        World &w = world;
         const MatchState &m = w.match;
         if (m.inSetPiece) return 1;
         if ((BallPredict(m.ball, 200) - S().position).Length() > 16.0f) return 1;
@@ -2021,7 +2083,10 @@ struct Selector {
     // trip or special takes the first by the ranking, a touch the first whose plan reaches the
     // ball (sliding falls back to its first), then the plan is installed. kSelectFalse when none
     // fits or a requeue keeps what runs.
-    HDN SelectResult SelectPlayerAnimation(const PlayerCommand &cmd, int interrupt, bool preferPassAndShot) {
+    HDN SelectResult SelectPlayerAnimation(GlobalRef<const PlayerCommand> command, int interrupt, bool preferPassAndShot) {
+        const PlayerCommand &cmd = command;
+        World &w = world;
+        const Ctx &c = context;
         ENG_SCOPE(14);
         AnimationState &cur = H().anim;
         const SpatialState &s = S();

@@ -71,7 +71,9 @@ HD Humanoid &HumanoidAt(World &w, int hi) {
 // Puts a humanoid at `pos` facing `focus`, idling at a random frame of the idle animation it
 // selects from there: the stance first, which the selection reads, then the animation, the apply
 // buffer and the nodes.
-HDN bool PlaceHumanoid(World &w, const Ctx &c, int hi, const Vec3 &pos, const Vec3 &focus) {
+HDN bool PlaceHumanoid(GlobalRef<World> world, LocalRef<const Ctx> context, int hi, const Vec3 &pos, const Vec3 &focus) {
+    World &w = world;
+    const Ctx &c = context;
     Humanoid &h = HumanoidAt(w, hi);
     const Stance st = StanceFacing(pos, focus);
     h.startPos = h.nextStartPos = h.prevPosition2D = st.at;
@@ -84,7 +86,7 @@ HDN bool PlaceHumanoid(World &w, const Ctx &c, int hi, const Vec3 &pos, const Ve
     AnimationState &a = h.anim;
     if (ia.posCount > a.positions.kCapacity) Unsupported("a state list outgrows its capacity");
     const int planned = ia.posCount < a.positions.kCapacity ? ia.posCount : a.positions.kCapacity;
-    GroupCopy<4>(a.positions.e, c.t->positions + ia.posFirst, planned);
+    GroupCopy<4>(a.positions.e, c.T().positions + ia.posFirst, planned);
     a.positions.count = planned;
     a.anim = a.id = idle;
     // GRF: the frame draws below the effective frame count, one less than the frame count.
@@ -118,7 +120,9 @@ HDN bool PlaceHumanoid(World &w, const Ctx &c, int hi, const Vec3 &pos, const Ve
 
 // The throw-in taker holds the ball: the idle animation whose start retains it at the right elbow
 // and moves most like standing still, facing the centre spot.
-HDN bool HoldBallForThrowIn(World &w, const Ctx &c, int hi) {
+HDN bool HoldBallForThrowIn(GlobalRef<World> world, LocalRef<const Ctx> context, int hi) {
+    World &w = world;
+    const Ctx &c = context;
     CrudeQuery hold;
     hold.byFunctionType = true;
     hold.functionType = kFnMovement;
@@ -155,7 +159,9 @@ HDN bool HoldBallForThrowIn(World &w, const Ctx &c, int hi) {
 
 // A player or official at a restart: its touch record and history cleared and, when active, placed
 // where it stands facing `focus`; a player's controller forgets its last wish.
-HDN bool RestartPerson(World &w, const Ctx &c, int hi, const Vec3 &focus) {
+HDN bool RestartPerson(GlobalRef<World> world, LocalRef<const Ctx> context, int hi, const Vec3 &focus) {
+    World &w = world;
+    const Ctx &c = context;
     const int players = w.match.playerCount;
     const bool isPlayer = hi < players;
     PersonBase &b = isPlayer ? w.match.players[hi].base : w.match.officials[hi - players];
@@ -179,7 +185,9 @@ HDN bool RestartPerson(World &w, const Ctx &c, int hi, const Vec3 &focus) {
 }
 // A player at a restart: the person's restart, then no possession, a second to the ball and no
 // marking or space ratings (the forward rating stays).
-HDN bool RestartPlayer(World &w, const Ctx &c, int p, const Vec3 &focus) {
+HDN bool RestartPlayer(GlobalRef<World> world, LocalRef<const Ctx> context, int p, const Vec3 &focus) {
+    World &w = world;
+    const Ctx &c = context;
     if (!RestartPerson(w, c, p, focus)) return false;
     Player &ps = w.match.players[p];
     ps.hasPossession = ps.hasBestPossession = ps.hasUniquePossession = false;
@@ -203,7 +211,9 @@ HD void ClearTeamPlan(TeamAI &ai) {
     ai.teamPossessionAmount = ai.fadingTeamPossessionAmount = 1.0f;
     ai.timeNeededToGetToBall = ai.oppTimeNeededToGetToBall = 100;
 }
-HDN bool RestartTeam(World &w, const Ctx &c, int teamID, const Vec3 &focus) {
+HDN bool RestartTeam(GlobalRef<World> world, LocalRef<const Ctx> context, int teamID, const Vec3 &focus) {
+    World &w = world;
+    const Ctx &c = context;
     Team &t = TeamByID(w, teamID);
     t.hasPossession = false;
     t.timeToBallMs = 100;
@@ -234,7 +244,9 @@ HD void RestBall(Ball &b, const Vec3 &focus) {
     b.touchesNet = false;
     b.memoValid = false;
 }
-HDN bool RestartMatch(World &w, const Ctx &c, const Vec3 &focus) {
+HDN bool RestartMatch(GlobalRef<World> world, LocalRef<const Ctx> context, const Vec3 &focus) {
+    World &w = world;
+    const Ctx &c = context;
     MatchState &m = w.match;
     m.ballRetainer = m.lastTouchTeamID = m.lastGoalScorer = m.bestPossessionTeam = -1;
     for (int &t : m.lastTouchTeamIDs) t = -1;
@@ -349,7 +361,9 @@ HD Vec3 KeepOff(const Vec3 &bp, const Vec3 &ball, float gap) { return ball + (bp
 // The kickoff spots: the formation pulled into the team's half, a random sideways step, at least
 // 0.5 m behind the line and outside the centre circle; the taking team's two players nearest the
 // centre spot go onto it again after every placement.
-HDN bool PlaceForKickOff(World &w, const Ctx &c, int teamID, bool taking, const PlayerList &outfield, const Vec3 &ball) {
+HDN bool PlaceForKickOff(GlobalRef<World> world, LocalRef<const Ctx> context, int teamID, bool taking, const PlayerList &outfield, const Vec3 &ball) {
+    World &w = world;
+    const Ctx &c = context;
     const int side = TeamDynamicSide(w, teamID);
     const double ds = side, hl = kPitchHalfLength;
     const Vec3 scale(ToFloat((double)(-side * kPitchHalfLength) * 0.6), ToFloat((double)(-side * kPitchHalfWidth) * 0.6), 0);
@@ -375,7 +389,9 @@ HDN bool PlaceForKickOff(World &w, const Ctx &c, int teamID, bool taking, const 
 // The outfield players by the restart's placement rule, then a defending wall 9.15 m from a free
 // kick (three players between the ball and the goal when it is within 40 m) and, at a penalty,
 // everyone outside the box and 9.65 m from the spot.
-HDN bool PlaceByRule(World &w, const Ctx &c, int teamID, int setPiece, bool taking, const PlayerList &outfield, const Vec3 &ball) {
+HDN bool PlaceByRule(GlobalRef<World> world, LocalRef<const Ctx> context, int teamID, int setPiece, bool taking, const PlayerList &outfield, const Vec3 &ball) {
+    World &w = world;
+    const Ctx &c = context;
     const int side = TeamDynamicSide(w, teamID);
     const Placement r = PlacementRule(setPiece, taking, side, ball);
     const double hl = kPitchHalfLength;
@@ -404,7 +420,9 @@ HDN bool PlaceByRule(World &w, const Ctx &c, int teamID, int setPiece, bool taki
 
 // The taking team's nearest player to the ball takes the restart: it stays put at a kickoff, stands
 // 0.3 m off the ball holding it at a throw-in, 2.3 m behind it otherwise, 3 m behind at a penalty.
-HDN bool PlaceTaker(World &w, const Ctx &c, int teamID, int setPiece, const Vec3 &ball) {
+HDN bool PlaceTaker(GlobalRef<World> world, LocalRef<const Ctx> context, int teamID, int setPiece, const Vec3 &ball) {
+    World &w = world;
+    const Ctx &c = context;
     TeamAI &ai = TeamByID(w, teamID).ai;
     const int side = TeamDynamicSide(w, teamID);
     const PlayerList nearest = GetClosestPlayers(w, c, teamID, ball, false, 2);
@@ -432,7 +450,8 @@ HD float NearestStart(const FormationEntry *team, int size, const Vec3 &ball) {
     for (int i = 0; i < size; i++) nearest = MinF(nearest, (team[i].startPosition - ball).Length());
     return nearest;
 }
-HDN bool LeftTeamStartsNearerBall(const World &w) {
+HDN bool LeftTeamStartsNearerBall(GlobalRef<const World> world) {
+    const World &w = world;
     const Scenario &s = w.scenario;
     return NearestStart(s.leftTeam, s.leftTeamSize, s.ballPosition) < NearestStart(s.rightTeam, s.rightTeamSize, s.ballPosition);
 }
@@ -440,7 +459,9 @@ HDN bool LeftTeamStartsNearerBall(const World &w) {
 // A team's placement for a restart: its goalkeepers on their line, its outfield players by the
 // restart, at a kickoff everyone back to the starting formation (the two teams' swapped when GRF
 // swaps them), then the taker.
-HDN bool PlaceTeam(World &w, const Ctx &c, int teamID, int setPiece, int otherTeamID, int kickoffTeamID, int takerTeamID) {
+HDN bool PlaceTeam(GlobalRef<World> world, LocalRef<const Ctx> context, int teamID, int setPiece, int otherTeamID, int kickoffTeamID, int takerTeamID) {
+    World &w = world;
+    const Ctx &c = context;
     MatchState &m = w.match;
     Team &team = TeamByID(w, teamID);
     team.ai.setPieceType = setPiece;
@@ -503,7 +524,9 @@ HDN bool PlaceTeam(World &w, const Ctx &c, int teamID, int setPiece, int otherTe
 // gamers move to the nearest selectable team mate), restarted again, deactivated and released; the
 // team's designated player is the one nearest the ball, and a keeper's formation entry passes to
 // the team's first remaining player.
-HDN bool SendOff(World &w, const Ctx &c, int p) {
+HDN bool SendOff(GlobalRef<World> world, LocalRef<const Ctx> context, int p) {
+    World &w = world;
+    const Ctx &c = context;
     MatchState &m = w.match;
     Player &ps = m.players[p];
     const int t = w.playerTeamID[p];
@@ -536,7 +559,9 @@ HDN bool SendOff(World &w, const Ctx &c, int p) {
 
 // The referee's restart: a free kick's spot kept inside 95% of the pitch, the match restarted
 // around the spot (in the rest frame), both teams placed in processing order, the taker recorded.
-HDN bool RefereeRestart(World &w, const Ctx &c, int setPiece) {
+HDN bool RefereeRestart(GlobalRef<World> world, LocalRef<const Ctx> context, int setPiece) {
+    World &w = world;
+    const Ctx &c = context;
     Referee &ref = w.match.referee;
     RefereeBuffer &b = ref.buffer;
     if (setPiece == kModeFreeKick) {

@@ -279,36 +279,36 @@ constexpr int kCameraHistory = 150;
 constexpr int kCameraWeights = kCameraHistory * (kCameraHistory + 1) / 2;
 
 struct Tables {
-    const Anim *anims;
+    GlobalPointer<const Anim> anims;
     int32_t animCount;
-    const NodeAnim *nodes;
-    const KeyFrame *keys;
-    const InterpEntry *interp;
-    const MiddleEntry *middle;
-    const FootballKey *football;
-    const Vec3 *positions;
-    const Quadrant *quadrants;
+    GlobalPointer<const NodeAnim> nodes;
+    GlobalPointer<const KeyFrame> keys;
+    GlobalPointer<const InterpEntry> interp;
+    GlobalPointer<const MiddleEntry> middle;
+    GlobalPointer<const FootballKey> football;
+    GlobalPointer<const Vec3> positions;
+    GlobalPointer<const Quadrant> quadrants;
     int32_t quadrantCount;
     Radian maxIncomingBallDeviation, maxOutgoingBallDeviation;
-    const AnimDerived *derived;
-    const SelectionRecord *selection;
-    const Vec3 *smoothed;
-    const int16_t *fnAnims;   // animations accepted per function type, ascending
-    const int32_t *fnOffset;  // kFunctionSlots + 1 entries
-    const CrudeRecord *crude;         // parallel to fnAnims
-    const CrudeRecord *crudeByIndex;  // one per animation
+    GlobalPointer<const AnimDerived> derived;
+    GlobalPointer<const SelectionRecord> selection;
+    GlobalPointer<const Vec3> smoothed;
+    GlobalPointer<const int16_t> fnAnims;   // animations accepted per function type, ascending
+    GlobalPointer<const int32_t> fnOffset;  // kFunctionSlots + 1 entries
+    GlobalPointer<const CrudeRecord> crude;         // parallel to fnAnims
+    GlobalPointer<const CrudeRecord> crudeByIndex;  // one per animation
     // Per function type and incoming velocity (slot fn * 4 + velocity), the records of the type
     // that pass its velocity rule, in list order; kFunctionSlots * 4 + 1 offsets.
-    const CrudeRecord *crudeVelocity;
-    const int32_t *crudeVelocityOffset;
+    GlobalPointer<const CrudeRecord> crudeVelocity;
+    GlobalPointer<const int32_t> crudeVelocityOffset;
     // The same lists prefiltered by the body rule of the function type for each allowed body
     // direction (slot (fn * 4 + velocity) * 6 + entry); kFunctionSlots * 4 * 6 + 1 offsets.
-    const CrudeRecord *crudeBody;
-    const int32_t *crudeBodyOffset;
-    const float *cameraWeights;
+    GlobalPointer<const CrudeRecord> crudeBody;
+    GlobalPointer<const int32_t> crudeBodyOffset;
+    GlobalPointer<const float> cameraWeights;
     // The crude selection of idle movement in and out (IdleMovementAnimation), which reads
     // only the tables: one list for every call.
-    const int16_t *idleMovement;
+    GlobalPointer<const int16_t> idleMovement;
     int32_t idleMovementCount;
 };
 
@@ -373,7 +373,7 @@ struct Aabb {
         b.hi += o;
         return b;
     }
-    HDN bool Intersects(const Vec3 &center, float radius) const {
+    HDN bool Intersects(Vec3 center, float radius) const {
         float d2 = 0;
         for (int k = 0; k < 3; k++) {
             if (center.v[k] < lo.v[k]) {
@@ -462,15 +462,29 @@ struct Scratch {
 };
 
 // Everything a match reads besides its world: the shared tables, its variant's static data and
-// its scratch block.
+// its scratch block. On the device the tables' addresses and each match's context lie in the
+// workgroup's LDS, staged when the kernel starts (StageContext), so that following one costs an LDS
+// read and not a chain of loads from HBM.
 struct Ctx {
-    const Tables *t;
-    const StaticData *sd;
-    const Skeleton *skeletons;  // players then officials
+    GlobalPointer<const Tables> tables;
+    GlobalPointer<const StaticData> sd;
+    GlobalPointer<const Skeleton> skeletons;  // players then officials
     int32_t ticksPerStep;
-    Scratch *ws;
-    HD const Anim &A(int i) const { return t->anims[i]; }
-    HD const AnimDerived &D(int i) const { return t->derived[i]; }
+    GlobalPointer<Scratch> ws;
+    HD const Tables &T() const;
+    HD const Anim &A(int i) const { return T().anims[i]; }
+    HD const AnimDerived &D(int i) const { return T().derived[i]; }
 };
+#if ENG_DEVICE
+__shared__ Tables gLdsTables;
+__shared__ Ctx gLdsContexts[64 / kGroupLanes];
+#endif
+HD const Tables &Ctx::T() const {
+#if ENG_DEVICE
+    return gLdsTables;
+#else
+    return *tables;
+#endif
+}
 
 }  // namespace eng

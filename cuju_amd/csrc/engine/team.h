@@ -11,7 +11,7 @@
 namespace eng {
 
 // Defined with the set pieces.
-HDN bool SendOff(World &w, const Ctx &c, int p);
+HDN bool SendOff(GlobalRef<World> world, LocalRef<const Ctx> context, int p);
 
 // Goals and the possession of the last minute are stored in processing order; these take IDs.
 HD int MatchGoalCount(const World &w, int teamID) { return w.match.goalCount[teamID == w.FirstTeamID() ? 0 : 1]; }
@@ -42,7 +42,8 @@ HD UserTactic UserTacticAt(int i) {
         default: return {kOffenseWidth, 0.74f, 0.1f};
     }
 }
-HDN void TeamUpdateTactics(World &w, int teamID) {
+HDN void TeamUpdateTactics(GlobalRef<World> world, int teamID) {
+    World &w = world;
     TeamAI &ai = TeamByID(w, teamID).ai;
     const MatchState &m = w.match;
     int goals = MatchGoalCount(w, teamID), oppGoals = MatchGoalCount(w, 1 - teamID);
@@ -68,7 +69,9 @@ HD int SelectAttackingRunPlayer(const World &w, const Ctx &c, int teamID) {
     Vec3 focus = Sp(w, pp).position + Vec3(-TeamDynamicSide(w, teamID) * 26.0f, 0, 0);
     return GetClosestPlayer(w, c, teamID, focus, true, pp);
 }
-HDN void TeamApplyAttackingRun(World &w, const Ctx &c, int teamID, int manualPlayer) {
+HDN void TeamApplyAttackingRun(GlobalRef<World> world, LocalRef<const Ctx> context, int teamID, int manualPlayer) {
+    World &w = world;
+    const Ctx &c = context;
     TeamAI &ai = TeamByID(w, teamID).ai;
     ai.endApplyAttackingRunMs = w.match.actualTimeMs + 4000;
     ai.attackingRunPlayer = manualPlayer >= 0 ? manualPlayer : SelectAttackingRunPlayer(w, c, teamID);
@@ -169,7 +172,9 @@ HD void ConsiderAttackingRun(World &w, const Ctx &c, int teamID) {
 // The team AI's tick: tactics each second, the view of the match, the offside trap, the danger
 // ranking, attacking runs and, every 1.5 s, the forward support player (the nearest to a point
 // 1.5 m upfield of the designated player).
-HDN bool TeamAIProcess(World &w, const Ctx &c, int teamID) {
+HDN bool TeamAIProcess(GlobalRef<World> world, LocalRef<const Ctx> context, int teamID) {
+    World &w = world;
+    const Ctx &c = context;
     ENG_SCOPE(10);
     const MatchState &m = w.match;
     TeamAI &ai = TeamByID(w, teamID).ai;
@@ -324,7 +329,9 @@ HDN int HungarianSolve(int *cost, int n, int *colOfRow) {
 
 // Assigns the outfield formation slots to the players nearest them: costs are decimeters, and
 // pairs beyond a growing cutoff cost 50000 until an assignment stays under it.
-HDN bool TeamCalculateDynamicRoles(World &w, const Ctx &c, int teamID) {
+HDN bool TeamCalculateDynamicRoles(GlobalRef<World> world, LocalRef<const Ctx> context, int teamID) {
+    World &w = world;
+    const Ctx &c = context;
     ENG_SCOPE(26);
     PlayerList all = TeamActivePlayers(w, teamID);
     PlayerList ps;
@@ -398,7 +405,8 @@ HDN bool TeamCalculateDynamicRoles(World &w, const Ctx &c, int teamID) {
 // half for distance from the line (to 60 m, to the 0.5) and half for distance from the middle
 // (to the 0.5); an opponent on the near side counts 60%; a fifth is nearness (to the pitch's
 // length).
-HDN float MarkingQuality(const World &w, int teamID, int p, int o) {
+HDN float MarkingQuality(GlobalRef<const World> world, int teamID, int p, int o) {
+    const World &w = world;
     const int side = TeamDynamicSide(w, teamID);
     const SpatialState &ms = Sp(w, p), &os = Sp(w, o);
     const Vec3 opponent = os.position + os.movement * 0.1f, marker = ms.position + ms.movement * 0.1f;
@@ -423,7 +431,9 @@ HDN float MarkingQuality(const World &w, int teamID, int p, int o) {
     return quality * 0.8f + nearness * 0.2f;
 }
 // The three most dangerous opponents get the best-placed outfield marker each, in danger order.
-HDN bool TeamCalculateManMarking(World &w, const Ctx &c, int teamID) {
+HDN bool TeamCalculateManMarking(GlobalRef<World> world, LocalRef<const Ctx> context, int teamID) {
+    World &w = world;
+    const Ctx &c = context;
     ENG_SCOPE(27);
     const int marked = 3;
     const TeamAI &ai = TeamByID(w, teamID).ai;
@@ -456,7 +466,9 @@ HDN bool TeamCalculateManMarking(World &w, const Ctx &c, int teamID) {
 // ---- the tick of a team -----------------------------------------------------------------------------
 // A player's tick (team_process.h, PlayerProcess) around its humanoid's: the part before the
 // humanoid's interruption, which returns the position the fatigue measures from, and the part after.
-HDN bool PlayerProcessBegin(World &w, const Ctx &c, int p, Vec3 &before) {
+HDN bool PlayerProcessBegin(GlobalRef<World> world, LocalRef<const Ctx> context, int p, Vec3 &before) {
+    World &w = world;
+    const Ctx &c = context;
     ENG_SCOPE(11);
     MatchState &m = w.match;
     Player &ps = m.players[p];
@@ -473,7 +485,9 @@ HDN bool PlayerProcessBegin(World &w, const Ctx &c, int p, Vec3 &before) {
     HumanoidProcessBegin(w, c, p);
     return true;
 }
-HDN bool PlayerProcessEnd(World &w, const Ctx &c, int p, const Vec3 &before) {
+HDN bool PlayerProcessEnd(GlobalRef<World> world, LocalRef<const Ctx> context, int p, Vec3 before) {
+    World &w = world;
+    const Ctx &c = context;
     MatchState &m = w.match;
     Player &ps = m.players[p];
     if (!HumanoidProcessEnd(w, c, p)) return false;
@@ -576,13 +590,17 @@ HD void ReconsiderDesignatedPlayer(World &w, int teamID) {
 // Each active player's spatial state for the tick, on the group's lanes at once: it reads the
 // player's own animation and last position only, which no other player's tick changes, so each
 // player's turn takes it from the match's scratch block instead of computing it in order.
-HDN void SpatialStatesAhead(World &w, const Ctx &c, int teamID) {
+HDN void SpatialStatesAhead(GlobalRef<World> world, LocalRef<const Ctx> context, int teamID) {
+    World &w = world;
+    const Ctx &c = context;
     const PlayerList ahead = TeamActivePlayers(w, teamID);
     for (int i = GroupRank(); i < ahead.count; i += kGroupLanes)
         c.ws->spatialAhead[ahead[i]] = NextSpatialState(c, Hum(w, ahead[i]));
     GroupSync();
 }
-HDN bool TeamProcess(World &w, const Ctx &c, int teamID) {
+HDN bool TeamProcess(GlobalRef<World> world, LocalRef<const Ctx> context, int teamID) {
+    World &w = world;
+    const Ctx &c = context;
     ENG_SCOPE(25);
     MatchState &m = w.match;
     UpdatePossessionAmounts(w, teamID);

@@ -97,8 +97,10 @@ HD void PropertiesSet(Tactics &t, int id, float value) {
 // index other tables, run only for the team's active players), and the sort runs in registers: an
 // insertion lands after the last kept entry it is not nearer than, where the shifting scan stops,
 // NaN distances included. A team holds at most kTeamPlayers players.
-HDN PlayerList GetClosestPlayers(const World &w, const Ctx &c, int teamID, const Vec3 &pos, bool onlyAI, unsigned count = 3,
+HDN PlayerList GetClosestPlayers(GlobalRef<const World> world, LocalRef<const Ctx> context, int teamID, Vec3 pos, bool onlyAI, unsigned count = 3,
                                  bool onlySelectable = false) {
+    const World &w = world;
+    const Ctx &c = context;
     float dist[kTeamPlayers];
     int who[kTeamPlayers], n = 0;
     const int players = w.match.playerCount;
@@ -143,7 +145,8 @@ HD int TeamGoalie(const World &w, const Ctx &c, int teamID) {
 }
 // The active player of a team with the least time to the ball, the first in state order on ties.
 // Every player's tests and time load together, without an early exit.
-HDN int TeamBestPossessionPlayer(const World &w, int teamID) {
+HDN int TeamBestPossessionPlayer(GlobalRef<const World> world, int teamID) {
+    const World &w = world;
     int best = 10000000, bp = -1;
     const int players = w.match.playerCount;
 #pragma unroll
@@ -189,7 +192,9 @@ HD float GoalDistanceAhead(const SpatialState &s, const Vec3 &goal) { return (go
 // switch focus, goalkeepers aside, the nearest; while an opponent is the designated player, the
 // first of them that will be at most a metre (plus a tenth of the opponent's distance, up to 3 m)
 // further from the team's goal than the opponent.
-HDN int SwitchTargetPlayer(const World &w, const Ctx &c, int teamID) {
+HDN int SwitchTargetPlayer(GlobalRef<const World> world, LocalRef<const Ctx> context, int teamID) {
+    const World &w = world;
+    const Ctx &c = context;
     const int designated = w.match.designatedPossessionPlayer;
     const PlayerList nearest = GetClosestPlayers(w, c, teamID, SwitchFocus(w, teamID), true, 8);
     PlayerList field;
@@ -291,7 +296,8 @@ HD void FendOff(World &w, Humanoid &h, int p, float influence) {
 }
 // Player p's pose offsets for the tick: cleared, then, in play without holding the ball and
 // moving, the legs, the upper body (off the ball) and the arms.
-HDN void PoseOffsets(World &w, int p) {
+HDN void PoseOffsets(GlobalRef<World> world, int p) {
+    World &w = world;
     Humanoid &h = Hum(w, p);
     const Quat identity(0, 0, 0, 1);
     for (int bp = kBpMiddle; bp <= kBpBody; bp++) SetOffset(h, bp, 0.0, identity);

@@ -34,7 +34,9 @@ struct TouchDifficulty {
 // Player p's touch difficulty: an off-balance body (position offset up to 10 cm), a velocity gap
 // to the ball (10 to 50 m/s), a ball beyond the foot (0.7 to 1.3 m), an opponent's touch just
 // before (recovered from faster with reaction); scaled by ball control and one draw in 0.5..1.
-HDN TouchDifficulty TouchDifficultyOf(World &w, const Ctx &c, int p, const Vec3 &offset) {
+HDN TouchDifficulty TouchDifficultyOf(GlobalRef<World> world, LocalRef<const Ctx> context, int p, Vec3 offset) {
+    World &w = world;
+    const Ctx &c = context;
     const Ball &b = w.match.ball;
     const SpatialState &s = Sp(w, p);
     const float offBalance = NormalizedClamp(offset.Length(), 0.0f, 0.1f) * 2.0f;
@@ -134,8 +136,11 @@ HD void SpinAgainstFoot(Kick &k, const Vec3 &foot) {
 // blended by the physics share, in the time left in the animation plus that delay and the touch
 // offset. Power is the distance over a dribble-scaled time, to the 0.7; the height grows with it;
 // a fast player touches up to 20% harder, less with ball control.
-HDN Kick BallControlKick(World &w, const Ctx &c, int p, const Humanoid &h, float nextBodyAngle, const Vec3 &outMov,
+HDN Kick BallControlKick(GlobalRef<World> world, LocalRef<const Ctx> context, int p, GlobalRef<const Humanoid> humanoid, float nextBodyAngle, Vec3 outMov,
                          float extraFoot = 0.0f) {
+    World &w = world;
+    const Ctx &c = context;
+    const Humanoid &h = humanoid;
     const AnimationState &cur = h.anim;
     const Anim &a = c.A(cur.anim);
     const ControlIntent in = BallControlIntent(w, c, p, h, a, outMov);
@@ -168,7 +173,10 @@ HDN Kick BallControlKick(World &w, const Ctx &c, int p, const Humanoid &h, float
 
 // A trap: a controlled touch with the foot pushed out by the touch's distance difficulty, lifted
 // by its height difficulty (more for a falling ball) and keeping part of the ball's momentum.
-HDN Kick TrapKick(World &w, const Ctx &c, int p, const Humanoid &h, float nextBodyAngle, const Vec3 &outMov) {
+HDN Kick TrapKick(GlobalRef<World> world, LocalRef<const Ctx> context, int p, GlobalRef<const Humanoid> humanoid, float nextBodyAngle, Vec3 outMov) {
+    World &w = world;
+    const Ctx &c = context;
+    const Humanoid &h = humanoid;
     const TouchDifficulty d = TouchDifficultyOf(w, c, p, h.decayingPositionOffset);
     Kick k = BallControlKick(w, c, p, h, nextBodyAngle, outMov, d.distance);
     const Vec3 incoming = w.match.ball.momentum;
@@ -188,7 +196,7 @@ struct ShotTouch {
 HD ShotTouch ShotTouchOf(const Ctx &c, const AnimationState &cur, const SpatialState &s) {
     const Anim &a = c.A(cur.anim);
     ShotTouch t;
-    t.movement = MovementAtFrame(c.t->positions + a.posFirst, a.posCount, cur.frameNum, 0).Rotated2D(s.angle.value());
+    t.movement = MovementAtFrame(c.T().positions + a.posFirst, a.posCount, cur.frameNum, 0).Rotated2D(s.angle.value());
     t.direction = t.movement.Normalized(s.directionVec);
     t.speed = t.movement.Length();
     if (VelocityCat(t.speed) == kVelIdle) t.direction = s.directionVec;
@@ -264,8 +272,12 @@ HD void CurlKick(Vec3 &kick, float amount) { kick.Rotate2D(amount * (0.4f + 0.6f
 
 // A shot's momentum and spin (x and y against the desired direction, z with the curl), with a
 // draw each, the x and y draws scaled up the nearer the shot comes to the worst one.
-HDN Vec3 ShotKick(World &w, const Ctx &c, int p, const AnimationState &cur, const SpatialState &s, const Vec3 &offset,
+HDN Vec3 ShotKick(GlobalRef<World> world, LocalRef<const Ctx> context, int p, GlobalRef<const AnimationState> animationState, GlobalRef<const SpatialState> spatialState, Vec3 offset,
                   float &xRot, float &yRot, float &zRot) {
+    World &w = world;
+    const Ctx &c = context;
+    const AnimationState &cur = animationState;
+    const SpatialState &s = spatialState;
     const PlayerCommand &cmd = cur.originatingCommand;
     const Vec3 desired = cmd.touchInfo.desiredDirection;
     const ShotTouch t = ShotTouchOf(c, cur, s);
@@ -309,7 +321,9 @@ HD Vec3 CapTouchPower(Vec3 r, int fn, const AnimDerived &d, const Vec3 &offset, 
 // up to a quarter turn either way), weakened and lifted by it, keeping some of the ball's
 // momentum, and lifted by one more draw scaled by the pass's own difficulty (less with the pass
 // statistics).
-HDN Vec3 AttainableTouch(World &w, const Ctx &c, int p, const Vec3 &desired, int fn) {
+HDN Vec3 AttainableTouch(GlobalRef<World> world, LocalRef<const Ctx> context, int p, Vec3 desired, int fn) {
+    World &w = world;
+    const Ctx &c = context;
     Humanoid &h = Hum(w, p);
     const AnimationState &cur = h.anim;
     const AnimDerived &d = c.D(cur.anim);
@@ -338,7 +352,7 @@ HDN Vec3 AttainableTouch(World &w, const Ctx &c, int p, const Vec3 &desired, int
 
 // The direction and power of a pass along `v`: lifted 0.11 (a high pass 0.45, less up to 0.15 with
 // distance); power the distance over 60 m to the 1.4, times 1.8 (1.15 for a high pass).
-HDN void PassForVector(int passType, const Vec3 &v, Vec3 &dir, float &power) {
+HDN void PassForVector(int passType, Vec3 v, Vec3 &dir, float &power) {
     const bool high = passType == kFnHighPass;
     const float lift = high ? 0.45f - NormalizedClamp(v.Length(), 0.0f, 60.0f) * 0.15f : 0.11f;
     dir = (v.Normalized(0) + Vec3(0, 0, lift)).Normalized(0);
@@ -386,8 +400,9 @@ HD int PassReceiver(const World &w, int p, const PlayerList &players, const Vec3
 // cut as the two targets part (to 50 m) and, for direction, raised toward 1 near the receiver
 // (within 12 m). A forced receiver or a gamer-controlled passer passes fully automatically; a
 // player without teammates fully manually. Long passes aim 20% of their length further upfield.
-HDN void AimPass(const World &w, int p, int passType, const Vec3 &inDir, float inPower, float autoDirBias, float autoPowerBias,
+HDN void AimPass(GlobalRef<const World> world, int p, int passType, Vec3 inDir, float inPower, float autoDirBias, float autoPowerBias,
                  Vec3 &outDir, float &outPower, int &target, int forcedTarget = -1) {
+    const World &w = world;
     const int teamID = w.playerTeamID[p];
     const Vec3 origin = PassOrigin(w, p);
     const Vec3 manual = origin + inDir * Clamp(inPower * 60.0f, 1.0f, 100.0f);
@@ -429,7 +444,8 @@ HDN void AimPass(const World &w, int p, int passType, const Vec3 &inDir, float i
 // A shot's direction: the input direction blended by the auto bias with a direction at the goal,
 // aimed across its mouth (up to 90% of its half width) as far as the input points away from the
 // goal's centre (a quarter turn reaches the post; the offset to the 0.7).
-HDN Vec3 AimShot(const World &w, int p, const Vec3 &inDir, float autoDirBias) {
+HDN Vec3 AimShot(GlobalRef<const World> world, int p, Vec3 inDir, float autoDirBias) {
+    const World &w = world;
     const SpatialState &s = Sp(w, p);
     const int side = TeamDynamicSide(w, w.playerTeamID[p]);
     const Vec3 from = s.position + s.movement * 0.12f;

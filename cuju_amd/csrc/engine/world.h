@@ -58,7 +58,7 @@ using PlayerList = Small<int, kPlayers>;
 struct Rng {
     static constexpr int kWords = 624, kShift = 397, kIndexAt = 2496, kLowAt = 2504, kHighAt = 2508;
     static constexpr uint32_t kTop = 0x80000000u, kTwist = 0x9908b0dfu;
-    uint8_t *b;
+    GlobalPointer<uint8_t> b;
     template <class T>
     HD T Load(int at) const {
         T v;
@@ -130,7 +130,8 @@ HD float RandomInRange(World &w, float lo, float hi) {
 // ---- mirroring between team frames ----------------------------------------------------------------
 HD void MirrorRadian(Radian &r) { r.rotated = !r.rotated; }
 
-HDN void MirrorHumanoid(Humanoid &h, bool &mirrored) {
+HDN void MirrorHumanoid(GlobalRef<Humanoid> humanoid, bool &mirrored) {
+    Humanoid &h = humanoid;
     NodeState &root = h.nodes[0];
     root.position = root.position * Vec3(-1, -1, 1);
     Quat q = root.rotation;
@@ -232,7 +233,8 @@ HD void MirrorMentalImage(World &w, int k, bool t0, bool t1, bool ball) {
     }
 }
 
-HDN void MirrorMatch(World &w, bool t0, bool t1, bool ball) {
+HDN void MirrorMatch(GlobalRef<World> world, bool t0, bool t1, bool ball) {
+    World &w = world;
     ENG_SCOPE(18);
     if (!t0 && !t1 && !ball) {
         GroupSync();
@@ -249,7 +251,8 @@ HDN void MirrorMatch(World &w, bool t0, bool t1, bool ball) {
 
 // A state stores the ball, last-touch team IDs and referee team/positions in canonical order; the
 // conversion is an involution.
-HDN void CanonicalToRest(World &w) {
+HDN void CanonicalToRest(GlobalRef<World> world) {
+    World &w = world;
     MatchState &m = w.match;
     if (w.FirstTeamID() == 1) {
         for (int i = 0; i < 4; i++)
@@ -454,7 +457,7 @@ HD int MentalImageIndex(const World &w, int historyMs) {
 // one included) reads the last prediction.
 // The fields one image's predictions read, looked up once for the many times a caller asks.
 struct MentalBallView {
-    const Vec3 *image, *ball;
+    GlobalPointer<const Vec3> image, ball;
     uint64_t now;
     uint32_t stamp;
     float maxDeviation;

@@ -86,6 +86,7 @@ __global__ void __launch_bounds__(kWaveLanes, ENG_WAVES_PER_SIMD) ResetKernel(en
                                                                       const int32_t *reverse) {
     const eng::Batch &b = LaunchBatch();
     eng::libm::StageMathTables();
+    eng::StageContext(b);
     const int env = MatchIndex();
     if (env >= b.count) return;
     if (mask && !mask[env]) return;
@@ -95,6 +96,7 @@ __global__ void __launch_bounds__(kWaveLanes, ENG_WAVES_PER_SIMD) ResetKernel(en
 __global__ void __launch_bounds__(kWaveLanes, ENG_WAVES_PER_SIMD) StepKernel(eng::Batch, const int32_t *actions) {
     const eng::Batch &b = LaunchBatch();
     eng::libm::StageMathTables();
+    eng::StageContext(b);
     const int env = MatchIndex();
     if (env >= b.count) return;
     if (!eng::StepEnvironment(b, env, actions)) RecordFault(env);
@@ -103,6 +105,7 @@ __global__ void __launch_bounds__(kWaveLanes, ENG_WAVES_PER_SIMD) StepKernel(eng
 __global__ void __launch_bounds__(kDeviceGroupLanes) OutputKernel(eng::Batch, int env) {
     const eng::Batch &b = LaunchBatch();
     eng::libm::StageMathTables();
+    eng::StageContext(b);
     eng::WriteEnvironmentOutputs(b, env, false);
 }
 

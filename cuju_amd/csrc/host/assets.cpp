@@ -505,12 +505,12 @@ std::unique_ptr<AnimationTables> LoadAnimationTables(const std::string &path) {
         const Tables view = t->View();
         auto scratch = std::make_unique<Scratch>();
         Ctx c{};
-        c.t = &view;
+        c.tables = &view;
         c.ws = scratch.get();
         AList idle{scratch->lists[1], 0};
         FilterAnimations(c, IdleMovementQuery(), idle);
         if (idle.count < 1) throw std::invalid_argument("expected animations of idle movement");
-        t->idleMovement.assign(idle.e, idle.e + idle.count);
+        t->idleMovement.assign(idle.e.get(), idle.e.get() + idle.count);
     }
     return t;
 }

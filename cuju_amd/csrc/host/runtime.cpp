@@ -75,7 +75,7 @@ BatchRuntime::BatchRuntime(const Configuration &cfg, std::unique_ptr<Device> dev
         const Tables *dTables = Upload(&dt, 1);
 
         std::vector<Ctx> contexts;
-        std::vector<const World *> templates;
+        std::vector<GlobalPointer<const World>> templates;
         int agents = 0;
         for (const auto &bundle : bundles_) {
             if (bundle->leftAgents < 0 || bundle->rightAgents < 0 || bundle->leftAgents + bundle->rightAgents > kMaxAgents)
@@ -83,7 +83,7 @@ BatchRuntime::BatchRuntime(const Configuration &cfg, std::unique_ptr<Device> dev
             agents = std::max(agents, bundle->leftAgents + bundle->rightAgents);
             for (const Variant &v : bundle->variants) {
                 Ctx c{};
-                c.t = dTables;
+                c.tables = dTables;
                 c.sd = Upload(&v.staticData, 1);
                 c.skeletons = Upload(v.skeletons);
                 c.ticksPerStep = cfg.ticksPerStep;
@@ -356,7 +356,7 @@ void BatchRuntime::SetDifficulty(const float *difficulty) {
     for (size_t i = 0; i < n; i++)
         if (!(difficulty[i] <= 1)) throw std::invalid_argument("expected a difficulty from 0 to 1, found " + std::to_string(difficulty[i]));
     if (!b_.teamDifficulty) b_.teamDifficulty = Alloc<float>(n);
-    dev_->ToDevice(const_cast<float *>(b_.teamDifficulty), difficulty, n * sizeof(float));
+    dev_->ToDevice(const_cast<float *>(b_.teamDifficulty.get()), difficulty, n * sizeof(float));
     hostDifficulty_.assign(difficulty, difficulty + n);
 }
 
@@ -449,7 +449,7 @@ void BatchRuntime::SetState(int env, const std::string &bytes, int prevScoreDiff
     const Variant &v = VariantAt(variant);
     const Tables hostTables = tables_->View();
     Ctx c{};
-    c.t = &hostTables;
+    c.tables = &hostTables;
     c.sd = &v.staticData;
     c.skeletons = v.skeletons.data();
     c.ticksPerStep = cfg_.ticksPerStep;

@@ -430,7 +430,7 @@ BuiltVariant BuildVariant(const ScenarioDescription &d, bool reverse, const Anim
     const Tables view = tables.View();
     auto scratch = std::make_unique<Scratch>();
     Ctx c{};
-    c.t = &view;
+    c.tables = &view;
     c.sd = &sd;
     c.skeletons = skeletons.data();
     c.ticksPerStep = 10;
