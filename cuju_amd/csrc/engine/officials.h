@@ -101,23 +101,27 @@ struct PlayerImagePos {
 };
 using ImageList = Small<PlayerImagePos, kPlayers>;
 
-// The images of one team in the mental image's order, extrapolated to now and held within the
-// image's deviation limits of the true state.
+// Entry `i` of a mental image, extrapolated to now and held within the image's deviation limits of
+// the true state; false for an inactive player or one of the other team.
+HD bool MentalTeamPlayerImage(const World &w, const MentalImage &mi, int i, int teamID, PlayerImagePos &e) {
+    const int age = (int)(w.match.actualTimeMs - (uint64_t)mi.timeStampMs);
+    const PlayerImage im = MentalImageEntry(w, mi, i);
+    if (!w.roster.active[im.player] || w.playerTeamID[im.player] != teamID) return false;
+    const SpatialState &s = Sp(w, im.player);
+    const Vec3 pos = im.position + im.movement * (float)age * 0.001f;
+    e.position = pos.EnforceMaximumDeviation(s.position, mi.maxDistanceDeviation);
+    e.movement = im.movement.EnforceMaximumDeviation(s.movement, mi.maxMovementDeviation);
+    e.role = im.role;
+    return true;
+}
+// The images of one team in the mental image's order.
 HDN void MentalTeamPlayerImages(GlobalRef<const World> world, int k, int teamID, ImageList &out) {
     const World &w = world;
     const MentalImage &mi = w.match.mentalImages[k];
-    const int age = (int)(w.match.actualTimeMs - (uint64_t)mi.timeStampMs);
     out.clear();
     for (int i = 0; i < mi.players.count; i++) {
-        const PlayerImage im = MentalImageEntry(w, mi, i);
-        if (!w.roster.active[im.player] || w.playerTeamID[im.player] != teamID) continue;
-        const SpatialState &s = Sp(w, im.player);
-        Vec3 pos = im.position + im.movement * (float)age * 0.001f;
         PlayerImagePos e;
-        e.position = pos.EnforceMaximumDeviation(s.position, mi.maxDistanceDeviation);
-        e.movement = im.movement.EnforceMaximumDeviation(s.movement, mi.maxMovementDeviation);
-        e.role = im.role;
-        out.push_back(e);
+        if (MentalTeamPlayerImage(w, mi, i, teamID, e)) out.push_back(e);
     }
 }
 // Moves the images along x by `futureMs` in place. The deepest image is skipped (the keeper's
