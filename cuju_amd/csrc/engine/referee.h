@@ -744,6 +744,15 @@ HDN void CheckHumanoidCollision(GlobalRef<World> world, LocalRef<const Ctx> cont
     TackleContact(w, c, p1, p2, k.dist);
 }
 
+// Pair `q` of the pairs (i, j), i < j, of n players in the order of a loop over i and then j: row i
+// starts at i (2n - 1 - i) / 2.
+HD void PairAt(int q, int n, int &i, int &j) {
+    const int m = 2 * n - 1;
+    i = (int)(((float)m - sqrtf((float)(m * m - 8 * q))) * 0.5f);
+    if (i > 0 && i * (m - i) / 2 > q) i--;
+    if ((i + 1) * (m - i - 1) / 2 <= q) i++;
+    j = q - i * (m - i) / 2 + i + 1;
+}
 HDN bool CheckHumanoidCollisions(GlobalRef<World> world, LocalRef<const Ctx> context) {
     World &w = world;
     const Ctx &c = context;
@@ -752,21 +761,41 @@ HDN bool CheckHumanoidCollisions(GlobalRef<World> world, LocalRef<const Ctx> con
     PlayerBounceList *const bounces = c.ws->bounces;
     for (int i = 0; i < ps.count; i++) bounces[i].clear();
     // A pair at least the tackle reach apart (2 m, beyond both contact radii) changes nothing, so
-    // only nearer pairs make the call; the distance is the one the pair's own check computes.
+    // only nearer pairs make the call; the distance is the one the pair's own check computes. The
+    // lanes of the match test consecutive pairs together, from a copy of the positions gathered
+    // once (one cache line per player otherwise); a call moves only its two players, whose copies
+    // it refreshes, and the search goes on with the pair after it. Each match of a wavefront
+    // searches up to its next near pair before any makes the call, so they make it together.
+    // Against testing the 231 pairs of 22 players one after another: 148 K -> 43 K cycles a tick for one
+    // match of 64 lanes; ms per step, 4,096 matches of 32 lanes 47.7 -> 46.3, 16,384 of 8 lanes 135.8 ->
+    // 134.0.
     static_assert((kContactBody + kContactShell) * 2.0f < kTackleReach, "the tackle reach bounds every contact");
-    // The pairs read the positions from a copy gathered once, not from each player's spatial state
-    // (one cache line per player, read again for every pair); a call moves only its two players,
-    // whose copies it refreshes.
-    Vec3 at[kPlayers];
-    for (int i = 0; i < ps.count; i++) at[i] = Sp(w, ps[i]).position;
-    for (int i = 0; i + 1 < ps.count; i++) {
-        for (int j = i + 1; j < ps.count; j++) {
-            if ((at[i] - at[j]).Length() < kTackleReach) {
-                CheckHumanoidCollision(w, c, ps[i], ps[j], bounces[i], bounces[j]);
-                at[i] = Sp(w, ps[i]).position;
-                at[j] = Sp(w, ps[j]).position;
+    Vec3 *const at = c.ws->contactAt;
+    for (int i = GroupRank(); i < ps.count; i += kGroupLanes) at[i] = Sp(w, ps[i]).position;
+    GroupSync();
+    const int pairs = ps.count * (ps.count - 1) / 2;
+    for (int next = 0; next < pairs;) {
+        int i = 0, j = 0;
+        LaneMask near = 0;
+        while (next < pairs) {
+            bool mine = false;
+            if (next + GroupRank() < pairs) {
+                PairAt(next + GroupRank(), ps.count, i, j);
+                mine = (at[i] - at[j]).LengthBelow(kTackleReach);
             }
+            near = GroupBallot(mine);
+            if (near) break;
+            next += kGroupLanes;
         }
+        if (!near) break;
+        const int hit = LowestBit(near);
+        i = GroupShuffle(i, hit);
+        j = GroupShuffle(j, hit);
+        CheckHumanoidCollision(w, c, ps[i], ps[j], bounces[i], bounces[j]);
+        at[i] = Sp(w, ps[i]).position;
+        at[j] = Sp(w, ps[j]).position;
+        GroupSync();
+        next += hit + 1;
     }
     for (int i = 0; i < ps.count; i++) {
         float total = 0.0f;

@@ -450,6 +450,7 @@ struct Scratch {
     ForceField forceField;
     PlayerBounceList bounces[kPlayers];
     PlayerGeometryList tackleGeometry[2];
+    Vec3 contactAt[kPlayers];
     int16_t lists[3][kMaxAnimations];
     int32_t listCount[3];
     Vec3 plans[2][kAnimPositions];
