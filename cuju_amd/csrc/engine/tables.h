@@ -440,6 +440,14 @@ struct PlanFrame {
     float stretchedSpeed, lean, rc, rs;
 };
 
+// Where a humanoid's frame finds its history: the entry of each of its animation's nodes, whether
+// the frame appended it, and the smoothing's share at the beginning of the animation.
+struct ApplyPlan {
+    int16_t entry[kBodyParts];
+    bool isNew[kBodyParts];
+    float beginBias;
+};
+
 // Per-match working memory: the animation selection's candidate lists, planned positions, sort keys
 // and one candidate plan per lane of the match, and the lists above. One block per environment in
 // HBM, which every lane of the match addresses, in place of large per-lane stack arrays: the lanes
@@ -451,6 +459,7 @@ struct Scratch {
     PlayerBounceList bounces[kPlayers];
     PlayerGeometryList tackleGeometry[2];
     Vec3 contactAt[kPlayers];
+    ApplyPlan applyPlans[kPlayers + 3];
     int16_t lists[3][kMaxAnimations];
     int32_t listCount[3];
     Vec3 plans[2][kAnimPositions];
