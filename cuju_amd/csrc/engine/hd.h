@@ -212,6 +212,14 @@ HD double GroupShuffle(double v, int rank) {
     memcpy(&r, &b, 8);
     return r;
 }
+// Leaves every lane of the group with the first of the lanes' candidates in a total order:
+// `takeIfBefore(r)` compares this lane's candidate with that of the lane of rank r and keeps the
+// earlier. Each round pairs the lanes, so 64 lanes take 6 rounds; taking one lane's candidate after
+// another took 63 (one match of 64 lanes: 13.5 -> 13.3 ms a step). Every lane must make the call.
+template <class TakeFn>
+HD void GroupReduce(TakeFn takeIfBefore) {
+    for (int apart = 1; apart < kGroupLanes; apart <<= 1) takeIfBefore(GroupRank() ^ apart);
+}
 // Orders the group's memory operations: what a lane stored before the call is what every lane of
 // the group loads after it (one wavefront's memory operations complete in order).
 HD void GroupSync() {

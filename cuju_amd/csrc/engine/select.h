@@ -1195,7 +1195,7 @@ struct Selector {
                 bestBase = b;
             }
         }
-        for (int r = 1; r < kGroupLanes; r++) {
+        GroupReduce([&](int r) {
             const int other = GroupShuffle((int32_t)best, r);
             const double ok = GroupShuffle(bestKey, r), ob = GroupShuffle(bestBase, r);
             if (other >= 0 && (best < 0 || ob < bestBase || (ob == bestBase && (ok < bestKey || (ok == bestKey && other < best))))) {
@@ -1203,8 +1203,8 @@ struct Selector {
                 bestKey = ok;
                 bestBase = ob;
             }
-        }
-        // Every lane now holds the group's first; lane 0's combination is taken for all.
+        });
+        // Every lane holds the group's first; lane 0's is taken for all.
         return GroupShuffle((int32_t)best, 0);
     }
     // Keeps, in order, the elements of `l` for which `keep` holds (the lanes of the match test
@@ -1261,19 +1261,16 @@ struct Selector {
             }
             return l[best];
         }
-        int winner = -1;
-        double wk[kMaxChainKeys];
-        for (int r = 0; r < kGroupLanes; r++) {
+        GroupReduce([&](int r) {
             const int e = GroupShuffle((int32_t)best, r);
-            if (e < 0) continue;
             double k[kMaxChainKeys];
             for (int j = 0; j < keyCount; j++) k[j] = GroupShuffle(bk[j], r);
-            if (winner < 0 || ChainPrecedes(k, wk, keyCount) || (!ChainPrecedes(wk, k, keyCount) && e < winner)) {
-                winner = e;
-                for (int j = 0; j < keyCount; j++) wk[j] = k[j];
+            if (e >= 0 && (best < 0 || ChainPrecedes(k, bk, keyCount) || (!ChainPrecedes(bk, k, keyCount) && e < best))) {
+                best = e;
+                for (int j = 0; j < keyCount; j++) bk[j] = k[j];
             }
-        }
-        return l[winner];
+        });
+        return l[best];
     }
 
     HD bool AllowLastDitch(bool withPossessionAmount = true) {
