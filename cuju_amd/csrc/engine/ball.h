@@ -562,6 +562,112 @@ struct TimeNeededScan {
     }
 };
 
+// Whether the walk reaches targets of one player (position, movement and velocity fixed) by given
+// times: the comparisons of GetTimeNeededMs's results with its time limit, for a limit that is the
+// time itself, as the possession scan asks them.
+//
+// After n of the walk's steps its position is from + movement s(n) and its radii 0.28 and 0.9 plus
+// amv b(n), with b and s the sums of the bias and of its rest in closed form, each up to the
+// rounding of 70 additions: 4.2e-6 of the coordinates, under the margin (1 mm and 1e-5 of them). A
+// target nearer than a radius less the margin after some step is reached there; one farther than
+// the radius and the margin after every step is not. Pieces of eight steps are ruled out by the
+// nearest point of their path against the radius at their end, and the steps of the others are
+// looked at one by one. A target within the margin of a radius, which rounding decides, takes
+// GetTimeNeededMs itself (under one in a hundred), so the results are GetTimeNeededMs's, which the host
+// build checks for each. The walk of 70 steps for each target took 13.7 K cycles, two thirds of
+// the scans' time.
+struct ReachScan {
+    static constexpr int kPiece = 8;
+    Vec3 pos, mov, start;
+    float maxVel, amv, perSpeed2;
+    bool moving;
+
+    HD ReachScan(const Vec3 &p, const Vec3 &m, float velocity) : pos(p), mov(m), start(p), maxVel(velocity) {
+        amv = maxVel * 0.94f;
+        moving = mov.Length() > kIdleDribbleSwitch;
+        const float speed2 = mov.v[0] * mov.v[0] + mov.v[1] * mov.v[1];
+        perSpeed2 = speed2 > 0.0f ? 1.0f / speed2 : 0.0f;
+        if (moving) {
+            start += mov.Normalized() * 0.1f;
+            start += mov * 0.01f;
+        }
+    }
+    // The sum of the bias over the first n steps (0, 1/70, ... (n - 1)/70, 10 ms each), and of its rest.
+    HD static float Biases(int n) { return (float)(n * (n - 1)) * (0.01f / 140.0f); }
+    HD static float Rests(int n) { return (float)n * 0.01f - Biases(n); }
+
+    // The squared distance of a target at `v` from the start of the walk after the walk moved for s.
+    HD float SquaredGap(const Vec3 &v, float s) const {
+        const float x = v.v[0] - mov.v[0] * s, y = v.v[1] - mov.v[1] * s;
+        return x * x + y * y + v.v[2] * v.v[2];
+    }
+    // Whether the walk reaches a target within 16 m (48 m with `precise`) by `ms`; false when the
+    // margin cannot tell.
+    HD bool Decide(const Vec3 &target, uint32_t ms, bool &usual, bool &optimistic) const {
+        usual = optimistic = false;
+        if (ms < 10) return false;
+        Vec3 from = start;
+        if (!moving) from += (target - pos).Normalized(0) * 0.1f;
+        const Vec3 v = target - from;
+        const float margin = 0.001f + (fabsf(from.v[0]) + fabsf(from.v[1])) * 1e-5f;
+        const float along = (v.v[0] * mov.v[0] + v.v[1] * mov.v[1]) * perSpeed2;
+        const uint32_t limit = ms / 10 + 1;
+        const int steps = limit < (uint32_t)kTimeWalkSteps ? (int)limit : kTimeWalkSteps;
+        const bool toEnd = ms >= (uint32_t)kTimeWalkSteps * 10;
+        float before = Rests(1);
+        for (int first = 1; first <= steps; first += kPiece) {
+            const int last = first + kPiece - 1 < steps ? first + kPiece - 1 : steps;
+            const float after = Rests(last), grown = amv * Biases(last);
+            const float nearest = SquaredGap(v, Clamp(along, before, after));
+            before = after;
+            const float most = optimistic ? 0.28f + grown + margin : 0.9f + grown + margin;
+            if (nearest > most * most) continue;
+            for (int n = first; n <= last; n++) {
+                const float d2 = SquaredGap(v, Rests(n)), radius = amv * Biases(n);
+                const float u = 0.28f + radius, o = 0.9f + radius;
+                if (!optimistic) {
+                    if (o > margin && d2 < (o - margin) * (o - margin)) optimistic = true;
+                    else if (!(d2 > (o + margin) * (o + margin))) return false;
+                }
+                if (u > margin && d2 < (u - margin) * (u - margin)) {
+                    usual = true;
+                    return true;
+                }
+                if (!(d2 > (u + margin) * (u + margin))) return false;
+            }
+        }
+        if (!toEnd) return true;
+        // Unreached at 700 ms: the rest of the way runs at the top speed.
+        const float d = sqrtf(SquaredGap(v, Rests(kTimeWalkSteps))), grown = amv * Biases(kTimeWalkSteps);
+        // The results are 700 ms and the rest, cut to whole ms.
+        const float left = (float)ms - (float)(kTimeWalkSteps * 10) + 1, slack = margin / amv * 2000 + 0.01f;
+        const float rem = Clamp(d - (0.28f + grown), 0.0f, 100000.0f) / amv * 1000;
+        const float ro = Clamp(d - (0.9f + grown), 0.0f, 100000.0f) / amv * 1000;
+        if (!(fabsf(rem - left) > slack)) return false;
+        usual = rem < left;
+        if (!optimistic) {
+            if (!(fabsf(ro - left) > slack)) return false;
+            optimistic = ro < left;
+        }
+        return true;
+    }
+    HD void Reached(const Vec3 &target, bool precise, uint32_t ms, bool &usual, bool &optimistic) const {
+        if ((pos - target).LengthAbove(precise ? 48.0f : 16.0f)) {
+            const uint32_t direct = DirectTimeMs(pos, mov, target, maxVel);
+            usual = direct <= ms;
+            optimistic = direct - 200 <= ms;
+        } else if (!Decide(target, ms, usual, optimistic)) {
+            const TimeNeeded r = GetTimeNeededMs(pos, mov, target, maxVel, precise, ms);
+            usual = r.usual <= ms;
+            optimistic = r.optimistic <= ms;
+        }
+#if !ENG_DEVICE
+        const TimeNeeded r = GetTimeNeededMs(pos, mov, target, maxVel, precise, ms);
+        if (usual != (r.usual <= ms) || optimistic != (r.optimistic <= ms)) Fatal("a possession scan's reach differs from the walk");
+#endif
+    }
+};
+
 struct ScanResult {
     uint32_t timeToBall, timeToBallOptimistic;
 };
@@ -595,7 +701,7 @@ HDN ScanResult SharedPossessionScan(GlobalPointer<const Vec3> pred, bool flip, V
         s.timeToBall = latest > direct ? latest : direct;
     }
     s.timeToBallOptimistic = s.timeToBall;
-    TimeNeededScan times(pos, mov, maxVel);
+    const ReachScan times(pos, mov, maxVel);
     const int base = GroupRank() - lane;
     const LaneMask mine = lanes >= 64 ? ~(LaneMask)0 : (((LaneMask)1 << lanes) - 1u);
     // This lane's point: whether the walk reaches it usually and optimistically (never above 1.5 m).
@@ -603,9 +709,7 @@ HDN ScanResult SharedPossessionScan(GlobalPointer<const Vec3> pred, bool flip, V
         usual = optimistic = false;
         const Vec3 at = PredFlip(pred, flip, (int)ms);
         if (!(at.v[2] < 1.5f)) return;
-        const TimeNeeded r = times.Get(at.Get2D(), precise, ms);
-        usual = r.usual <= ms;
-        optimistic = r.optimistic <= ms;
+        times.Reached(at.Get2D(), precise, ms, usual, optimistic);
     };
     // The round's lowest usual hit, or -1; the optimistic time takes the lowest optimistic hit up
     // to it (the points of a round rise with the lane).
@@ -677,13 +781,14 @@ HDN ScanResult PossessionScan(GlobalPointer<const Vec3> pred, bool flip, Vec3 po
     s.timeToBallOptimistic = s.timeToBall;
     bool refine = false;
     uint32_t stepMs = 10, prev = 0;
-    TimeNeededScan times(pos, mov, maxVel);
+    const ReachScan times(pos, mov, maxVel);
     for (uint32_t ms = start; ms < kBallPredictionSpanMs; ms += stepMs) {
         if (PredFlip(pred, flip, ms).v[2] < 1.5f) {
             const Vec3 target = PredFlip(pred, flip, ms).Get2D();
-            TimeNeeded r = times.Get(target, precise, ms);
-            if (r.optimistic <= ms && ms < s.timeToBallOptimistic) s.timeToBallOptimistic = ms;
-            if (r.usual <= ms) {
+            bool usual, optimistic;
+            times.Reached(target, precise, ms, usual, optimistic);
+            if (optimistic && ms < s.timeToBallOptimistic) s.timeToBallOptimistic = ms;
+            if (usual) {
                 if (!refine) {
                     ms = prev;
                     stepMs = 10;
@@ -785,9 +890,12 @@ HDN void TeamUpdatePossessionStatistics(GlobalRef<World> world, LocalRef<const C
     const int rest = players.count - whole;
     const int share = rest > 0 && kGroupLanes >= 2 * rest ? kGroupLanes / rest : 1;
     const int single = share == 1 ? players.count : whole;
-    for (int i = GroupRank(); i < single; i += kGroupLanes) PlayerUpdatePossessionStatistics(w, *c.sd, players[i]);
-    if (share > 1 && GroupRank() < share * rest)
-        PlayerUpdatePossessionStatistics(w, *c.sd, players[whole + GroupRank() / share], GroupRank() % share, share);
+    for (int i = GroupRank(); i < single; i += kGroupLanes)
+        PlayerUpdatePossessionStatistics(w, *c.sd, players[i]);
+    if (share > 1 && GroupRank() < share * rest) {
+        const int i = whole + GroupRank() / share;
+        PlayerUpdatePossessionStatistics(w, *c.sd, players[i], GroupRank() % share, share);
+    }
     GroupSync();
     // The team's summary over its active players in state order, kept in registers and stored once.
     bool hasPossession = false;
