@@ -26,16 +26,10 @@ HD double Fma(double a, double b, double c) { return fma(a, b, c); }
 // ---- sinf / cosf: Arm Optimized Routines sinf.c/cosf.c (glibc flt-32 s_sinf.c) -------------------
 // Reference: include/cuju/libm/sincosf.h:61-212.
 
-struct SinCosCoeffs {
-    double sign[4];
-    double hpi_inv, hpi, c0, c1, s1, c2, s2, c3, s3, c4;
-};
-
 // The tables the float routines index with a per-lane value. On the device each workgroup reads
 // them from its LDS, where StageMathTables copies them before any engine code runs; the host
 // reads the constant tables.
 #if ENG_DEVICE
-__shared__ uint64_t gLdsSinCosfCoefficients[28];
 __shared__ uint64_t gLdsPowfLog2Table[32];
 __shared__ uint64_t gLdsExp2fTable[32];
 #endif
@@ -46,57 +40,21 @@ __device__ inline void StageMathTables() {
     for (int i = threadIdx.x; i < 32; i += blockDim.x) {
         gLdsPowfLog2Table[i] = kPowfLog2Table[i];
         gLdsExp2fTable[i] = kExp2fTable[i];
-        if (i < 28) gLdsSinCosfCoefficients[i] = kSinCosfCoefficients[i];
     }
     __syncthreads();
 #endif
 }
 #endif
 #if ENG_DEVICE
-#define LIBM_SINCOSF_TABLE gLdsSinCosfCoefficients
 #define LIBM_POWF_LOG2_TABLE gLdsPowfLog2Table
 #define LIBM_EXP2F_TABLE gLdsExp2fTable
 #else
-#define LIBM_SINCOSF_TABLE kSinCosfCoefficients
 #define LIBM_POWF_LOG2_TABLE kPowfLog2Table
 #define LIBM_EXP2F_TABLE kExp2fTable
 #endif
 
-HD SinCosCoeffs LoadSinCos(int set) {
-    SinCosCoeffs k;
-    const uint64_t *t = LIBM_SINCOSF_TABLE + 14 * set;
-    k.sign[0] = DoubleOf(t[0]);
-    k.sign[1] = DoubleOf(t[1]);
-    k.sign[2] = DoubleOf(t[2]);
-    k.sign[3] = DoubleOf(t[3]);
-    k.hpi_inv = DoubleOf(t[4]);
-    k.hpi = DoubleOf(t[5]);
-    k.c0 = DoubleOf(t[6]);
-    k.c1 = DoubleOf(t[7]);
-    k.s1 = DoubleOf(t[8]);
-    k.c2 = DoubleOf(t[9]);
-    k.s2 = DoubleOf(t[10]);
-    k.c3 = DoubleOf(t[11]);
-    k.s3 = DoubleOf(t[12]);
-    k.c4 = DoubleOf(t[13]);
-    return k;
-}
-
-// sign[j] for j in 0..3, selected rather than indexed.
-HD double SignOf(const SinCosCoeffs &k, int j) {
-    return j == 0 ? k.sign[0] : j == 1 ? k.sign[1] : j == 2 ? k.sign[2] : k.sign[3];
-}
-
 // Exponent and top 3 mantissa bits of |x|.
 HD uint32_t Top12f(float x) { return (BitsOf(x) >> 20) & 0x7ff; }
-
-// |x| < 120: x - n*pi/2 with n = round(x * 2/pi) computed on a 2^24 fixed-point scale.
-HD double ReduceFast(double x, const SinCosCoeffs &k, int *n) {
-    double r = x * k.hpi_inv;
-    int q = ((int32_t)r + 0x800000) >> 24;
-    *n = q;
-    return Fma(-(double)q, k.hpi, x);
-}
 
 // Payne-Hanek reduction of a finite |x| >= 120 with 4/pi held in 32-bit windows.
 HDN double ReduceLarge(uint32_t xi, int *np) {
@@ -114,95 +72,79 @@ HDN double ReduceLarge(uint32_t xi, int *np) {
     return (double)(int64_t)r0 * 0x1.921FB54442D18p-62;
 }
 
-// Sine polynomial for even n, cosine polynomial for odd n, on the reduced argument.
-HD float SinCosPoly(double x, double x2, const SinCosCoeffs &k, int n) {
-    if ((n & 1) == 0) {
-        double x3 = x * x2;
-        double s1 = Fma(x2, k.s3, k.s2);
-        double x7 = x3 * x2;
-        double s = Fma(x3, k.s1, x);
-        return (float)Fma(x7, s1, s);
-    }
-    double x4 = x2 * x2;
-    double c2 = Fma(x2, k.c4, k.c3);
-    double c1 = Fma(x2, k.c1, k.c0);
-    double x6 = x4 * x2;
-    double c = Fma(x4, k.c2, c1);
-    return (float)Fma(x6, c2, c);
-}
-
 struct SinCos {
     float s, c;
 };
 
-// Shared reduction of sinf and cosf: returns false for |x| < pi/4 (no reduction).
-HD bool SinCosReduce(float y, double *xr, double *sgn, int *n, int *set) {
-    uint32_t top = Top12f(y);
-    *set = 0;
-    if (top < Top12f(0x1.921FB6p-1f)) return false;
-    SinCosCoeffs k0 = LoadSinCos(0);
-    if (top < Top12f(120.0f)) {
-        *xr = ReduceFast((double)y, k0, n);
-        *sgn = SignOf(k0, *n & 3);
-        *set = (*n & 2) ? 1 : 0;
-    } else {
-        uint32_t b = BitsOf(y);
-        int s = b >> 31;
-        *xr = ReduceLarge(b, n);
-        *sgn = SignOf(k0, (*n + s) & 3);
-        *set = ((*n + s) & 2) ? 1 : 0;
+// The routines' reduction and polynomials with fewer branches, since the lanes of a wavefront take
+// different ones: the reduction of |y| < 120, n = round(y 2/pi) on a 2^24 fixed-point scale, leaves
+// an argument below pi/4 as it is, and n picks and signs the polynomials' results. The routines'
+// second coefficient set is the first with the cosine's coefficients negated, which negates every
+// step of its polynomial exactly, and the sine's polynomial is odd. The coefficients are constants
+// in the code, not loads. Measured together with atan2f below, ms per step against the routines'
+// branches with the sets in LDS: one match of 64 lanes 13.0 -> 12.7, 16,384 of 8 lanes 122.9 -> 120.7,
+// the mixed 32,768 of 4 lanes 137.8 -> 134.0.
+struct ReducedAngle {
+    double x, x2;
+    int n, turn;  // quarter turns modulo 4, for the choice of the polynomial and for the signs
+    HD explicit ReducedAngle(float y) {
+        x = (double)y;
+        // One match to a wavefront takes one way at a branch, so there it skips the reduction.
+        if (kGroupLanes == kMaxGroupLanes && Top12f(y) < Top12f(0x1.921FB6p-1f)) {
+            n = turn = 0;
+        } else if (Top12f(y) < Top12f(120.0f)) {
+            const int q = (int32_t)(x * DoubleOf(kSinCosfCoefficients[4]));
+            n = turn = (q + 0x800000) >> 24;
+            x = Fma(-(double)n, DoubleOf(kSinCosfCoefficients[5]), x);
+        } else {
+            x = ReduceLarge(BitsOf(y), &n);
+            turn = n + (int)(BitsOf(y) >> 31);
+        }
+        x2 = x * x;
     }
-    return true;
-}
-
+    // The sign of the reduced argument is - for turns 1 and 2 (mod 4), the cosine's for 2 and 3.
+    HD float Sine() const {
+        const double s1 = DoubleOf(kSinCosfCoefficients[8]), s2 = DoubleOf(kSinCosfCoefficients[10]),
+                     s3 = DoubleOf(kSinCosfCoefficients[12]);
+        const double x3 = x * x2;
+        const float sine = (float)Fma(x3 * x2, Fma(x2, s3, s2), Fma(x3, s1, x));
+        return FloatOf(BitsOf(sine) ^ (((uint32_t)(turn + 1) & 2) << 30));
+    }
+    HD float Cosine() const {
+        const double c0 = DoubleOf(kSinCosfCoefficients[6]), c1 = DoubleOf(kSinCosfCoefficients[7]),
+                     c2 = DoubleOf(kSinCosfCoefficients[9]), c3 = DoubleOf(kSinCosfCoefficients[11]),
+                     c4 = DoubleOf(kSinCosfCoefficients[13]);
+        const double x4 = x2 * x2;
+        const float cosine = (float)Fma(x4 * x2, Fma(x2, c4, c3), Fma(x4, c2, Fma(x2, c1, c0)));
+        return FloatOf(BitsOf(cosine) ^ (((uint32_t)turn & 2) << 30));
+    }
+};
+// Arguments below 2^-12 are their own sine, and their cosine is 1.
 HD float sinf(float y) {
-    uint32_t top = Top12f(y);
+    const uint32_t top = Top12f(y);
+    if (top < Top12f(0x1p-12f)) return y;
     if (top >= Top12f(INFINITY)) return (y - y) / (y - y);
-    if (top < Top12f(0x1.921FB6p-1f)) {
-        if (top < Top12f(0x1p-12f)) return y;
-        double x = y;
-        return SinCosPoly(x, x * x, LoadSinCos(0), 0);
-    }
-    double x, s;
-    int n, set;
-    SinCosReduce(y, &x, &s, &n, &set);
-    return SinCosPoly(x * s, x * x, LoadSinCos(set), n);
+    const ReducedAngle a(y);
+    return (a.n & 1) ? a.Cosine() : a.Sine();
 }
-
 HD float cosf(float y) {
-    uint32_t top = Top12f(y);
+    const uint32_t top = Top12f(y);
+    if (top < Top12f(0x1p-12f)) return 1.0f;
     if (top >= Top12f(INFINITY)) return (y - y) / (y - y);
-    if (top < Top12f(0x1.921FB6p-1f)) {
-        if (top < Top12f(0x1p-12f)) return 1.0f;
-        double x = y;
-        return SinCosPoly(x, x * x, LoadSinCos(0), 1);
-    }
-    double x, s;
-    int n, set;
-    SinCosReduce(y, &x, &s, &n, &set);
-    return SinCosPoly(x * s, x * x, LoadSinCos(set), n ^ 1);
+    const ReducedAngle a(y);
+    return (a.n & 1) ? a.Sine() : a.Cosine();
 }
-
 // sinf and cosf of one argument sharing the reduction; each result equals the single function's.
 HD SinCos sincosf(float y) {
-    ENG_SCOPE(50);
-    uint32_t top = Top12f(y);
+    const uint32_t top = Top12f(y);
+    if (top < Top12f(0x1p-12f)) return SinCos{y, 1.0f};
     if (top >= Top12f(INFINITY)) {
-        float v = (y - y) / (y - y);
+        const float v = (y - y) / (y - y);
         return SinCos{v, v};
     }
-    if (top < Top12f(0x1.921FB6p-1f)) {
-        if (top < Top12f(0x1p-12f)) return SinCos{y, 1.0f};
-        double x = y;
-        SinCosCoeffs k = LoadSinCos(0);
-        return SinCos{SinCosPoly(x, x * x, k, 0), SinCosPoly(x, x * x, k, 1)};
-    }
-    double x, s;
-    int n, set;
-    SinCosReduce(y, &x, &s, &n, &set);
-    SinCosCoeffs k = LoadSinCos(set);
-    double xs = x * s, x2 = x * x;
-    return SinCos{SinCosPoly(xs, x2, k, n), SinCosPoly(xs, x2, k, n ^ 1)};
+    const ReducedAngle a(y);
+    const float s = a.Sine(), c = a.Cosine();
+    return SinCos{(a.n & 1) ? c : s, (a.n & 1) ? s : c};
 }
 
 // ---- powf: Arm Optimized Routines powf.c (glibc flt-32 e_powf.c), log2 N=16, exp2 N=32 ----------
@@ -528,87 +470,81 @@ HD float atanf(float x) {
                           -1.1111110449e-01f, 9.0908870101e-02f,  -7.6918758452e-02f,
                           6.6610731184e-02f,  -5.8335702866e-02f, 4.9768779427e-02f,
                           -3.6531571299e-02f, 1.6285819933e-02f};
-    int32_t hx = (int32_t)BitsOf(x), ix = hx & 0x7fffffff;
-    if (ix >= 0x4c000000) {
-        if (ix > 0x7f800000) return x + x;
-        if (hx > 0) return atanhi[3] + atanlo[3];
-        return -atanhi[3] - atanlo[3];
-    }
-    if (ix < 0x31000000 && 1.0e30f + x > 1.0f) return x;
-    // fdlibm's four argument reductions, (2|x| - 1) / (2 + |x|), (|x| - 1) / (|x| + 1),
-    // (|x| - 1.5) / (1 + 1.5|x|) and -1 / |x|, as one selected quotient: the same operations on
-    // each lane, so lanes in different ranges share one division.
+    // Straight-line code on |x|, since the lanes of a wavefront take different ranges: fdlibm's four
+    // argument reductions, (2|x| - 1) / (2 + |x|), (|x| - 1) / (|x| + 1), (|x| - 1.5) / (1 + 1.5|x|)
+    // and -1 / |x|, are one selected quotient. Every step is odd in x, so
+    // the sign goes on last; below 2^-29 the polynomial leaves x as it is.
+    const uint32_t hx = BitsOf(x), ix = hx & 0x7fffffff;
     const bool reduced = ix >= 0x3ee00000;
     const int id = ix < 0x3f300000 ? 0 : ix < 0x3f980000 ? 1 : ix < 0x401c0000 ? 2 : 3;
     const float ax = fabsf(x);
     const float num = id == 0 ? 2.0f * ax - 1.0f : id == 1 ? ax - 1.0f : id == 2 ? ax - 1.5f : -1.0f;
     const float den = id == 0 ? 2.0f + ax : id == 1 ? ax + 1.0f : id == 2 ? 1.0f + 1.5f * ax : ax;
-    if (reduced) x = num / den;
-    float z = x * x;
+    float t = ax;
+    if (reduced) t = num / den;
+    float z = t * t;
     float w = z * z;
     float s1 = z * (aT[0] + w * (aT[2] + w * (aT[4] + w * (aT[6] + w * (aT[8] + w * aT[10])))));
     float s2 = w * (aT[1] + w * (aT[3] + w * (aT[5] + w * (aT[7] + w * aT[9]))));
-    if (!reduced) return x - x * (s1 + s2);
+    if (kGroupLanes == kMaxGroupLanes && !reduced) return x - x * (s1 + s2);
     const float hi = id == 0 ? atanhi[0] : id == 1 ? atanhi[1] : id == 2 ? atanhi[2] : atanhi[3];
     const float lo = id == 0 ? atanlo[0] : id == 1 ? atanlo[1] : id == 2 ? atanlo[2] : atanlo[3];
-    z = hi - ((x * (s1 + s2) - lo) - x);
-    return (hx < 0) ? -z : z;
+    z = reduced ? hi - ((t * (s1 + s2) - lo) - t) : t - t * (s1 + s2);
+    if (ix >= 0x4c000000) z = atanhi[3] + atanlo[3];
+    return ix > 0x7f800000 ? x + x : FloatOf(BitsOf(z) ^ (hx & 0x80000000u));
 }
 
 HD float atan2f(float y, float x) {
-    ENG_SCOPE(51);
     const float tiny = 1.0e-30f, pi_o_4 = 7.8539818525e-01f, pi_o_2 = 1.5707963705e+00f,
                 pi = 3.1415927410e+00f, pi_lo = -8.7422776573e-08f;
     int32_t hx = (int32_t)BitsOf(x), hy = (int32_t)BitsOf(y);
     int32_t ix = hx & 0x7fffffff, iy = hy & 0x7fffffff;
-    if (ix > 0x7f800000 || iy > 0x7f800000) return x + y;
-    if (hx == 0x3f800000) return atanf(y);
-    int m = ((hy >> 31) & 1) | ((hx >> 30) & 2);
-    if (iy == 0) {
-        switch (m) {
-            case 0:
-            case 1:
-                return y;
-            case 2:
-                return pi + tiny;
-            default:
-                return -pi - tiny;
-        }
-    }
-    if (ix == 0) return (hy < 0) ? -pi_o_2 - tiny : pi_o_2 + tiny;
-    if (ix == 0x7f800000) {
-        if (iy == 0x7f800000) {
+    const int m = ((hy >> 31) & 1) | ((hx >> 30) & 2);
+    // Zeros, infinities and NaN.
+    if ((uint32_t)(ix - 1) >= 0x7f7fffffu || (uint32_t)(iy - 1) >= 0x7f7fffffu) {
+        if (ix > 0x7f800000 || iy > 0x7f800000) return x + y;
+        if (iy == 0) {
             switch (m) {
                 case 0:
-                    return pi_o_4 + tiny;
                 case 1:
-                    return -pi_o_4 - tiny;
+                    return y;
                 case 2:
-                    return 3.0f * pi_o_4 + tiny;
+                    return pi + tiny;
                 default:
-                    return -3.0f * pi_o_4 - tiny;
+                    return -pi - tiny;
             }
         }
-        switch (m) {
-            case 0:
-                return 0.0f;
-            case 1:
-                return -0.0f;
-            case 2:
-                return pi + tiny;
-            default:
-                return -pi - tiny;
+        if (ix == 0) return (hy < 0) ? -pi_o_2 - tiny : pi_o_2 + tiny;
+        if (ix == 0x7f800000) {
+            if (iy == 0x7f800000) {
+                switch (m) {
+                    case 0:
+                        return pi_o_4 + tiny;
+                    case 1:
+                        return -pi_o_4 - tiny;
+                    case 2:
+                        return 3.0f * pi_o_4 + tiny;
+                    default:
+                        return -3.0f * pi_o_4 - tiny;
+                }
+            }
+            switch (m) {
+                case 0:
+                    return 0.0f;
+                case 1:
+                    return -0.0f;
+                case 2:
+                    return pi + tiny;
+                default:
+                    return -pi - tiny;
+            }
         }
+        if (iy == 0x7f800000) return (hy < 0) ? -pi_o_2 - tiny : pi_o_2 + tiny;
     }
-    if (iy == 0x7f800000) return (hy < 0) ? -pi_o_2 - tiny : pi_o_2 + tiny;
-    int32_t k = (iy - ix) >> 23;
-    float z;
-    if (k > 60)
-        z = pi_o_2 + 0.5f * pi_lo;
-    else if (hx < 0 && k < -60)
-        z = 0.0f;
-    else
-        z = atanf(fabsf(y / x));
+    const int32_t k = (iy - ix) >> 23;
+    float z = atanf(fabsf(y / x));
+    if (k > 60) z = pi_o_2 + 0.5f * pi_lo;
+    else if (hx < 0 && k < -60) z = 0.0f;
     // The quadrant, selected rather than branched.
     const float zl = z - pi_lo;
     return m == 0 ? z : m == 1 ? FloatOf(BitsOf(z) ^ 0x80000000u) : m == 2 ? pi - zl : zl - pi;
