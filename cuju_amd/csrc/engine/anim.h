@@ -116,7 +116,7 @@ struct Transform {
 // A local transform placed under `parent`. A relative one composes with it: the rotations
 // multiplied and renormalized, the scales multiplied, the position scaled and turned by the
 // parent's, then moved by its position. An absolute one, or a root's, stands as it is.
-HDN Transform Placed(const Transform *parent, int localMode, Vec3 pos, const Quat &rot, Vec3 scale) {
+HD Transform Placed(const Transform *parent, int localMode, const Vec3 &pos, const Quat &rot, const Vec3 &scale) {
     if (localMode != kLocalRelative || !parent) return Transform{pos, scale, rot};
     Transform t;
     t.rotation = (parent->rotation * rot).Normalized();
@@ -137,6 +137,26 @@ HD void WorldTransforms(const Skeleton &sk, const NodeState *nodes, Transform *o
 HD WorldGeometry PlacedGeometry(const SkelGeometry &g, const Transform &node) {
     const Transform at = Placed(&node, g.localMode, g.position, g.rotation, g.scale);
     return WorldGeometry{Aabb{g.boxMin, g.boxMax}.Rotated(at.rotation).Translated(at.position), at.position};
+}
+
+// One of a node's geometries in the world: the transforms down from the root to the node (the path
+// packed root first, four bits a node), then the geometry's.
+static_assert(kHumanoidNodes <= 15, "a node's index and one to spare fit four bits");
+HDN WorldGeometry PlacedPart(GlobalRef<const Skeleton> skeleton, GlobalPointer<const NodeState> nodes, int node, int geometry) {
+    const Skeleton &sk = skeleton;
+    uint64_t path = 0;
+    for (int n = node, up; n >= 0; n = up < n ? up : -1) {
+        path = path << 4 | (uint64_t)(n + 1);
+        up = sk.nodes[n].parent;  // parents come before their children
+    }
+    Transform at;
+    const Transform *parent = nullptr;
+    for (; path; path >>= 4) {
+        const NodeState &s = nodes[(int)(path & 15) - 1];
+        at = Placed(parent, s.localMode, s.position, s.rotation, s.scale);
+        parent = &at;
+    }
+    return PlacedGeometry(sk.nodes[node].geometries[geometry], at);
 }
 
 // ---- applying a frame ------------------------------------------------------------------------------
