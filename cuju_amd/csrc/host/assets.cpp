@@ -650,7 +650,9 @@ void SetupAgents(World &w, const StaticData &sd, int left, int right, const std:
     // GRF: the gamers take the active controllable players closest to the ball (at the origin
     // with the players on their formation spots), the closest as the main selected player, then
     // assigned in stable-ID order.
+    const auto scratch = std::make_unique<Scratch>();
     Ctx c{};
+    c.ws = scratch.get();
     c.sd = &sd;
     for (int t = 0; t < 2; t++) {
         if (agents[t] == 0) continue;
