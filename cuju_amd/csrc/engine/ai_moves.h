@@ -700,7 +700,7 @@ struct AIBase {
         ff.push_back(SupportAnchor(base, mind, cur, carrier));
         if (makeRun) ff.push_back(MakeSpot(Vec3(-side * kPitchHalfLength, cur.v[1] * 0.5f, 0.0f), kAttract, kDecayConstant, 2.0f * runWeight));
         // GRF adds 0.7 to every coordinate of the focus here.
-        const PlayerList opponents = GetClosestPlayers(w, c, oppID, carrier * 0.3f + cur + 0.7f, false, 3);
+        const PlayerRanking opponents = GetClosestPlayers(w, c, oppID, carrier * 0.3f + cur + 0.7f, false, 3);
         for (int i = 0; i < opponents.count; i++) {
             const PlayerImage oi = MentalPlayerImage(w, k, opponents[i]);
             const Vec3 at = oi.position + oi.movement * 0.1f;
@@ -712,7 +712,7 @@ struct AIBase {
             ff.push_back(s);
         }
         if (Own().fadingTeamPossessionAmount >= 1.02f) {
-            const PlayerList mates = GetClosestPlayers(w, c, teamID, cur, false, 6);
+            const PlayerRanking mates = GetClosestPlayers(w, c, teamID, cur, false, 6);
             for (int i = 0; i < mates.count; i++) {
                 if (mates[i] == p) continue;
                 const PlayerImage mi = MentalPlayerImage(w, k, mates[i]);
@@ -1007,7 +1007,7 @@ struct AIBase {
         const Vec3 at = Pos(), mov = Mov();
         const float offense = 0.7f + kDribbleOffensiveness * 0.05f + GetMindSet(DynamicRole()) * 0.05f;
         const float powerMul = 1.0f, futureS = 0.25f;
-        const PlayerList opponents = GetClosestPlayers(w, c, oppID, at, false, 5);
+        const PlayerRanking opponents = GetClosestPlayers(w, c, oppID, at, false, 5);
         ForceField &ff = c.ws->forceField;
         ff.clear();
         const float nearGoalLine = NormalizedClamp(fabsf(at.v[0]) / kPitchHalfLength, 0.0f, 1.0f);

@@ -51,13 +51,12 @@ struct AIController : AIBase {
         const float minimum = 0.2f * (1.0f - mind) - longPossession * 0.1f;
         const float threshold = 0.1f - longPossession * 0.05f;
         const float own = TacticalRating(ps, pw.forwardSpace, pw.space, pw.forward, pw.total);
-        const PlayerList mates = TeamActivePlayers(w, teamID);
+        const PlayerSet mates = TeamActivePlayers(w, teamID);
         float bestTotal = 0.0f;
         int best = -1;
         passType = kFnShortPass;
         passOdds = 0.0f;
-        for (int i = 0; i < mates.count; i++) {
-            const int mate = mates[i];
+        for (const int mate : mates) {
             if (mate == p) continue;
             float rating = TacticalRating(m.players[mate], pw.forwardSpace, pw.space, pw.forward, pw.total);
             if (StaticRole(mate) == kRoleGoalkeeper) rating *= 0.7f;
@@ -397,7 +396,7 @@ struct AIController : AIBase {
             forceMagnet = true;
             extraHaste = true;
         }
-        const PlayerList nearest = GetClosestPlayers(w, c, teamID, Pos(o) + Mov(o) * 0.1f, false, 2);
+        const PlayerRanking nearest = GetClosestPlayers(w, c, teamID, Pos(o) + Mov(o) * 0.1f, false, 2);
         bool near = false;
         for (int i = 0; i < nearest.count && !near; i++) near = nearest[i] == p;
         if (!near) return;

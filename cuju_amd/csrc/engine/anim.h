@@ -349,22 +349,30 @@ HDN void ApplyNode(LocalRef<const Ctx> context, GlobalRef<const Anim> animation,
     }
 }
 
-// Applies every humanoid's buffered frame; humanoids are independent.
-HDN void FetchPutBuffers(LocalRef<const Ctx> context, const GlobalPointer<const Skeleton> *skels, const GlobalPointer<Humanoid> *hums, int count) {
+// Applies the buffered frame of the active players and the officials; humanoids are independent.
+HDN void FetchPutBuffers(GlobalRef<World> world, LocalRef<const Ctx> context, uint32_t active) {
+    World &w = world;
     const Ctx &c = context;
+    const PlayerSet players{active};
+    const int playing = players.size(), count = playing + 3;
+    // Humanoid k's place in the state: the players', then the officials'.
+    auto place = [&](int k) { return k < playing ? players[k] : w.match.playerCount + k - playing; };
+    auto humanoid = [&](int k) -> Humanoid & {
+        return k < playing ? w.match.players[players[k]].base.humanoid : w.match.officials[k - playing].humanoid;
+    };
     // A humanoid's pose reads and writes only its own state, and a node only its own body part's
     // node, offset and history entry.
     ApplyPlan *const plans = c.ws->applyPlans;
     auto applyNode = [&](int k, int n) {
-        Humanoid &h = *hums[k];
+        Humanoid &h = humanoid(k);
         AnimApplyBuffer &buf = h.applyBuf;
         const Anim &a = c.A(buf.anim);
         if (n < a.nodeCount)
-            ApplyNode(c, a, *skels[k], h, n, buf.frameNum, buf.smooth, buf.smoothFactor, buf.position, buf.orientation.value(),
+            ApplyNode(c, a, c.skeletons[place(k)], h, n, buf.frameNum, buf.smooth, buf.smoothFactor, buf.position, buf.orientation.value(),
                       buf.offsets, 10, buf.noPos, plans[k]);
     };
     auto prepare = [&](int k, bool append) {
-        Humanoid &h = *hums[k];
+        Humanoid &h = humanoid(k);
         ApplyPrepare(c, c.A(h.applyBuf.anim), h, h.applyBuf.smooth, h.applyBuf.frameNum, plans[k], append);
     };
     if constexpr (kGroupLanes >= 16) {

@@ -885,11 +885,11 @@ HDN void TeamUpdatePossessionStatistics(GlobalRef<World> world, LocalRef<const C
     // of the match take the players in turn, one a lane in whole rounds. The players left after
     // the whole rounds, when the group has at least two lanes for each, get as many lanes each as
     // the group holds, which share the player's scan (they write the same results).
-    const PlayerList players = TeamActivePlayers(w, teamID);
-    const int whole = players.count - players.count % kGroupLanes;
-    const int rest = players.count - whole;
+    const PlayerSet players = TeamActivePlayers(w, teamID);
+    const int count = players.size(), whole = count - count % kGroupLanes;
+    const int rest = count - whole;
     const int share = rest > 0 && kGroupLanes >= 2 * rest ? kGroupLanes / rest : 1;
-    const int single = share == 1 ? players.count : whole;
+    const int single = share == 1 ? count : whole;
     for (int i = GroupRank(); i < single; i += kGroupLanes)
         PlayerUpdatePossessionStatistics(w, *c.sd, players[i]);
     if (share > 1 && GroupRank() < share * rest) {
@@ -897,14 +897,19 @@ HDN void TeamUpdatePossessionStatistics(GlobalRef<World> world, LocalRef<const C
         PlayerUpdatePossessionStatistics(w, *c.sd, players[i], GroupRank() % share, share);
     }
     GroupSync();
-    // The team's summary over its active players in state order, kept in registers and stored once.
-    bool hasPossession = false;
+    // The team's summary: whether any has the ball, and the shortest time to it.
+    bool holds = false;
     int timeToBall = 100000;
-    for (int i = 0; i < players.count; i++) {
-        if (w.match.players[players[i]].hasPossession) hasPossession = true;
-        const int t = (int)w.roster.timeToBallMs[players[i]];
-        if (t < timeToBall) timeToBall = t;
+    for (int i = GroupRank(); i < count; i += kGroupLanes) {
+        const int p = players[i], t = (int)w.roster.timeToBallMs[p];
+        holds |= w.match.players[p].hasPossession;
+        timeToBall = t < timeToBall ? t : timeToBall;
     }
+    const bool hasPossession = GroupBallot(holds) != 0;
+    GroupReduce([&](int r) {
+        const int other = GroupShuffle((int32_t)timeToBall, r);
+        timeToBall = other < timeToBall ? other : timeToBall;
+    });
     Team &t = TeamByID(w, teamID);
     t.hasPossession = hasPossession;
     t.timeToBallMs = timeToBall;

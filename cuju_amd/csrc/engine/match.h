@@ -29,17 +29,16 @@ HDN void PushMentalImage(GlobalRef<World> world, const bool (&mirrored)[2]) {
     mi.maxDistanceDeviation = 2.5f;
     mi.maxMovementDeviation = kWalkVelocity;
     for (int slot = 0; slot < 2; slot++) {
-        PlayerList ps = TeamActivePlayers(w, slot == 0 ? w.FirstTeamID() : 1 - w.FirstTeamID());
-        for (int i = 0; i < ps.count; i++) {
-            const SpatialState &s = Sp(w, ps[i]);
+        for (const int p : TeamActivePlayers(w, slot == 0 ? w.FirstTeamID() : 1 - w.FirstTeamID())) {
+            const SpatialState &s = Sp(w, p);
             PlayerImage im{};
-            im.player = ps[i];
+            im.player = p;
             im.position = s.position;
             im.directionVector = s.directionVec;
-            if (mirrored[w.playerTeamID[ps[i]]]) im.directionVector.Mirror();
+            if (mirrored[w.playerTeamID[p]]) im.directionVector.Mirror();
             im.velocity = s.velocityCat;
             im.movement = s.movement;
-            im.role = m.players[ps[i]].dynamicFormationEntry.role;
+            im.role = m.players[p].dynamicFormationEntry.role;
             mi.players.push_back(im);
         }
     }
@@ -275,12 +274,12 @@ HDN void MatchPreparePutBuffers(GlobalRef<World> world) {
     // A player's buffers and pose offsets are its own, and the rest of the match is only read, so
     // the lanes of the match take a team's players in turn.
     MirrorMatch(w, false, false, first == 1);
-    PlayerList a = TeamActivePlayers(w, first);
-    for (int i = GroupRank(); i < a.count; i += kGroupLanes) PlayerPreparePutBuffers(w, a[i]);
+    const PlayerSet a = TeamActivePlayers(w, first);
+    for (int i = GroupRank(); i < a.size(); i += kGroupLanes) PlayerPreparePutBuffers(w, a[i]);
     GroupSync();
     MirrorMatch(w, false, false, true);
-    PlayerList b = TeamActivePlayers(w, second);
-    for (int i = GroupRank(); i < b.count; i += kGroupLanes) PlayerPreparePutBuffers(w, b[i]);
+    const PlayerSet b = TeamActivePlayers(w, second);
+    for (int i = GroupRank(); i < b.size(); i += kGroupLanes) PlayerPreparePutBuffers(w, b[i]);
     GroupSync();
     MirrorMatch(w, false, false, first == 0);
 }
@@ -288,22 +287,8 @@ HDN void MatchFetchPutBuffers(GlobalRef<World> world, LocalRef<const Ctx> contex
     World &w = world;
     const Ctx &c = context;
     ENG_SCOPE(21);
-    const int first = w.FirstTeamID();
-    GlobalPointer<const Skeleton> skels[kPlayers + 3];
-    GlobalPointer<Humanoid> hums[kPlayers + 3];
-    int n = 0;
-    for (int t = 0; t < 2; t++) {
-        PlayerList ps = TeamActivePlayers(w, t == 0 ? first : 1 - first);
-        for (int i = 0; i < ps.count; i++) {
-            skels[n] = &c.skeletons[ps[i]];
-            hums[n++] = &w.match.players[ps[i]].base.humanoid;
-        }
-    }
-    for (int o = 0; o < 3; o++) {
-        skels[n] = &c.skeletons[w.match.playerCount + o];
-        hums[n++] = &w.match.officials[o].humanoid;
-    }
-    FetchPutBuffers(c, skels, hums, n);
+    // The humanoids are independent, so the teams' order does not show.
+    FetchPutBuffers(w, c, TeamActivePlayers(w, 0).mask | TeamActivePlayers(w, 1).mask);
 }
 // One 10 ms tick of the game.
 HDN bool GameTick(GlobalRef<World> world, LocalRef<const Ctx> context) {

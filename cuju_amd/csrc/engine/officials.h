@@ -188,7 +188,7 @@ HDN float GetOffsideLine(GlobalRef<const World> world, int k, int teamID, unsign
 // d ms averages the newest min(count, d / 10 + 1) entries of the history, each mirrored when the
 // ball's frame is, summed newest first; an empty history gives the ball's position. Every average
 // is a prefix of the same running sum, so one pass records each at its length. The entries load
-// in batches of 8 (indexes clamped into the history), so a batch waits for memory once; the
+// in batches of 16 (indexes clamped into the history), so a batch waits for memory once; the
 // additions keep their order.
 template <int N>
 HD void BallAveragePositions(const World &w, const unsigned (&durationsMs)[N], Vec3 (&out)[N]) {
@@ -206,20 +206,20 @@ HD void BallAveragePositions(const World &w, const unsigned (&durationsMs)[N], V
         longest = lengths[i] > longest ? lengths[i] : longest;
     }
     Vec3 sum, sums[N];
-    for (int first = 0; first < longest; first += 8) {
-        Vec3 batch[8];
+    for (int first = 0; first < longest; first += 16) {
+        Vec3 batch[16];
 #pragma unroll
-        for (int j = 0; j < 8; j++) {
+        for (int j = 0; j < 16; j++) {
             const int k = first + j < longest ? first + j : longest - 1;
             batch[j] = history[count - 1 - k];
         }
         // Only a batch that holds the end of an average records sums.
         bool records = false;
 #pragma unroll
-        for (int i = 0; i < N; i++) records |= lengths[i] > first && lengths[i] <= first + 8;
+        for (int i = 0; i < N; i++) records |= lengths[i] > first && lengths[i] <= first + 16;
         if (!records) {
 #pragma unroll
-            for (int j = 0; j < 8; j++) {
+            for (int j = 0; j < 16; j++) {
                 Vec3 p = batch[j];
                 if (flip) p.Mirror();
                 sum += p;
@@ -227,7 +227,7 @@ HD void BallAveragePositions(const World &w, const unsigned (&durationsMs)[N], V
             continue;
         }
 #pragma unroll
-        for (int j = 0; j < 8; j++) {
+        for (int j = 0; j < 16; j++) {
             if (first + j >= longest) break;
             Vec3 p = batch[j];
             if (flip) p.Mirror();
@@ -301,9 +301,8 @@ HD void RefereeFollowsPlay(const World &w, const Ctx &ctx, const SpatialState &s
     field.push_back(MakeSpot(BallPredict(m.ball, 200).Get2D(), kRepel, kDecayVariable, 0.5f, 10.0f));
     const int first = w.FirstTeamID();
     for (int k = 0; k < 2; k++) {
-        const PlayerList players = TeamActivePlayers(w, k == 0 ? first : 1 - first);
-        for (int i = 0; i < players.count; i++) {
-            const SpatialState &p = Sp(w, players[i]);
+        for (const int player : TeamActivePlayers(w, k == 0 ? first : 1 - first)) {
+            const SpatialState &p = Sp(w, player);
             field.push_back(MakeSpot(p.position + p.movement * 0.4f, kRepel, kDecayVariable, 0.5f, 10.0f));
         }
     }

@@ -322,17 +322,15 @@ HD void RecordOffsidePositions(World &w, int attackers) {
     ref.offsidePlayers.count = 0;
     if (!(m.inPlay && (!b.active || (b.desiredSetPiece != kModeThrowIn && b.desiredSetPiece != kModeCorner)))) return;
     ImageList defenders;
-    const PlayerList def = TeamActivePlayers(w, 1 - attackers);
-    for (int i = 0; i < def.count; i++) {
-        const SpatialState &s = Sp(w, def[i]);
-        defenders.push_back(PlayerImagePos{s.position, s.movement, m.players[def[i]].dynamicFormationEntry.role});
+    for (const int p : TeamActivePlayers(w, 1 - attackers)) {
+        const SpatialState &s = Sp(w, p);
+        defenders.push_back(PlayerImagePos{s.position, s.movement, m.players[p].dynamicFormationEntry.role});
     }
     const int side = TeamDynamicSide(w, attackers);
     const float line = OffsideLineFromImages(defenders, BallPredict(m.ball, 0), TeamDynamicSide(w, 1 - attackers), 0);
     const int toucher = TeamByID(w, attackers).lastTouchPlayer;
-    const PlayerList att = TeamActivePlayers(w, attackers);
-    for (int i = 0; i < att.count; i++)
-        if (att[i] != toucher && Sp(w, att[i]).position.v[0] * side < line * side) ref.offsidePlayers.push_back(att[i]);
+    for (const int p : TeamActivePlayers(w, attackers))
+        if (p != toucher && Sp(w, p).position.v[0] * side < line * side) ref.offsidePlayers.push_back(p);
 }
 // The referee's part of a touch, with offsides on: punish a touch by a player recorded offside,
 // then record the offside positions at this touch.
@@ -359,11 +357,18 @@ HD bool TeamSetLastTouchPlayer(World &w, const Ctx &c, int p, int touchType) {
 }
 
 // ---- collisions --------------------------------------------------------------------------------------
-HD PlayerList PlayersInProcessingOrder(const World &w) {
-    PlayerList ps = TeamActivePlayers(w, w.FirstTeamID());
-    PlayerList o = TeamActivePlayers(w, 1 - w.FirstTeamID());
-    for (int i = 0; i < o.count; i++) ps.push_back(o[i]);
-    return ps;
+struct ProcessingOrder {
+    PlayerSet first, second;
+    int firstCount, count;
+    HD int operator[](int i) const { return i < firstCount ? first[i] : second[i - firstCount]; }
+};
+HD ProcessingOrder PlayersInProcessingOrder(const World &w) {
+    ProcessingOrder o;
+    o.first = TeamActivePlayers(w, w.FirstTeamID());
+    o.second = TeamActivePlayers(w, 1 - w.FirstTeamID());
+    o.firstCount = o.first.size();
+    o.count = o.firstCount + o.second.size();
+    return o;
 }
 
 // Whether player p's body may deflect the ball this tick: the opponents touched it within 200 ms
@@ -432,7 +437,7 @@ HDN bool CheckBallCollisions(GlobalRef<World> world, LocalRef<const Ctx> context
     ENG_SCOPE(5);
     MatchState &m = w.match;
     if (m.actualTimeMs <= (uint64_t)(uint32_t)(m.lastBodyBallCollisionTimeMs + 150)) return true;
-    const PlayerList ps = PlayersInProcessingOrder(w);
+    const ProcessingOrder ps = PlayersInProcessingOrder(w);
     Vec3 bounce;
     float depth = 0.0;
     int bounces = 0;
@@ -781,7 +786,7 @@ HDN bool CheckHumanoidCollisions(GlobalRef<World> world, LocalRef<const Ctx> con
     World &w = world;
     const Ctx &c = context;
     ENG_SCOPE(17);
-    PlayerList ps = PlayersInProcessingOrder(w);
+    const ProcessingOrder ps = PlayersInProcessingOrder(w);
     PlayerBounceList *const bounces = c.ws->bounces;
     for (int i = 0; i < ps.count; i++) bounces[i].clear();
     // A pair at least the tackle reach apart (2 m, beyond both contact radii) changes nothing, so

@@ -379,7 +379,7 @@ HDN bool PlaceForKickOff(GlobalRef<World> world, LocalRef<const Ctx> context, in
         }
         if (!PlaceHumanoid(w, c, outfield[i], bp, ball)) return false;
         if (!taking) continue;
-        const PlayerList centre = GetClosestPlayers(w, c, teamID, Vec3(0), false, 2);
+        const PlayerRanking centre = GetClosestPlayers(w, c, teamID, Vec3(0), false, 2);
         for (int k = 0; k < centre.count; k++)
             if (!PlaceHumanoid(w, c, centre[k], Vec3(0, ToFloat((double)k * 1.4 * ds), 0), ball)) return false;
     }
@@ -407,7 +407,7 @@ HDN bool PlaceByRule(GlobalRef<World> world, LocalRef<const Ctx> context, int te
     }
     const Vec3 goal(side * kPitchHalfLength, 0, 0);
     if (setPiece == kModeFreeKick && !taking && (double)(ball - goal).Length() < 40.0) {
-        const PlayerList wall = GetClosestPlayers(w, c, teamID, ball, false, 3);
+        const PlayerRanking wall = GetClosestPlayers(w, c, teamID, ball, false, 3);
         for (int k = 0; k < wall.count; k++) {
             Vec3 toGoal = (goal - ball).Normalized(0);
             toGoal += Vec3(0, ToFloat(1.0 - (double)k), 0) * ToFloat(0.07);
@@ -425,7 +425,7 @@ HDN bool PlaceTaker(GlobalRef<World> world, LocalRef<const Ctx> context, int tea
     const Ctx &c = context;
     TeamAI &ai = TeamByID(w, teamID).ai;
     const int side = TeamDynamicSide(w, teamID);
-    const PlayerList nearest = GetClosestPlayers(w, c, teamID, ball, false, 2);
+    const PlayerRanking nearest = GetClosestPlayers(w, c, teamID, ball, false, 2);
     if (nearest.empty()) return Fail("the set piece has no taker");
     const int taker = ai.taker = nearest[0];
     // The direction of the ball from the centre spot (down the touchline's normal at the spot).

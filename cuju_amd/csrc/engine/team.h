@@ -131,32 +131,34 @@ HD void RankOpponentsByDanger(World &w, const Ctx &c, int teamID) {
     const Team &opp = TeamByID(w, 1 - teamID);
     TeamAI &ai = TeamByID(w, teamID).ai;
     const int side = TeamDynamicSide(w, teamID);
-    const PlayerList opponents = TeamActivePlayers(w, 1 - teamID);
+    const PlayerSet opponents = TeamActivePlayers(w, 1 - teamID);
+    const int count = opponents.size();
     Vec3 danger = Vec3((float)(((double)kPitchHalfLength - 2.0) * side), 0, 0);
     danger = danger * 0.8f + BallPredict(m.ball, 100).Get2D() * 0.2f;
     // The lanes of the match take the opponents in turn, first for the factor and then for the place.
     float *const factors = c.ws->teamValues;
     bool unordered = false;
-    for (int i = GroupRank(); i < opponents.count; i += kGroupLanes) {
-        float factor = (1.0f - NormalizedClamp((Sp(w, opponents[i]).position - danger).Length(), 0, kPitchHalfLength * 2));
+    for (int i = GroupRank(); i < count; i += kGroupLanes) {
+        const int o = opponents[i];
+        float factor = (1.0f - NormalizedClamp((Sp(w, o).position - danger).Length(), 0, kPitchHalfLength * 2));
         factor *= 0.95f;
-        if (opponents[i] == opp.designatedTeamPossessionPlayer) factor += 0.05f;
+        if (o == opp.designatedTeamPossessionPlayer) factor += 0.05f;
         factors[i] = factor;
         unordered |= factor != factor;
     }
     GroupSync();
     if (!GroupBallot(unordered)) {
-        for (int i = GroupRank(); i < opponents.count; i += kGroupLanes) {
+        for (int i = GroupRank(); i < count; i += kGroupLanes) {
             int place = 0;
-            for (int j = 0; j < opponents.count; j++) place += (factors[j] > factors[i]) | ((factors[j] == factors[i]) & (j < i));
+            for (int j = 0; j < count; j++) place += (factors[j] > factors[i]) | ((factors[j] == factors[i]) & (j < i));
             ai.tacticalOpponents[place] = TacticalOpponent{opponents[i], factors[i]};
         }
-        ai.tacticalOpponents.count = opponents.count;
+        ai.tacticalOpponents.count = count;
         GroupSync();
         return;
     }
     ai.tacticalOpponents.count = 0;
-    for (int i = 0; i < opponents.count; i++) {
+    for (int i = 0; i < count; i++) {
         const TacticalOpponent e{opponents[i], factors[i]};
         int at = ai.tacticalOpponents.count;
         ai.tacticalOpponents.push_back(e);
@@ -179,7 +181,7 @@ HD void ConsiderAttackingRun(World &w, const Ctx &c, int teamID) {
     const Vec3 at = Sp(w, runner).position;
     const float near = libm::powf(1.0f - NormalizedClamp((at - Sp(w, team.designatedTeamPossessionPlayer).position).Length(), 0, 40), 0.5f);
     const Vec3 spot = at * Vec3(1.0f, 0.8f, 0.0f) + Vec3(TeamDynamicSide(w, teamID) * 10.0f, 0, 0);
-    const PlayerList crowd = GetClosestPlayers(w, c, 1 - teamID, spot, false, 4);
+    const PlayerRanking crowd = GetClosestPlayers(w, c, 1 - teamID, spot, false, 4);
     float space = 1.0f;
     for (int i = 0; i < crowd.count; i++)
         space -= libm::powf(Curve(1.0f - NormalizedClamp((Sp(w, crowd[i]).position - spot).Length(), 0, 15), 1.0f), 0.5f) * 0.3f;
@@ -350,7 +352,7 @@ HDN bool TeamCalculateDynamicRoles(GlobalRef<World> world, LocalRef<const Ctx> c
     World &w = world;
     const Ctx &c = context;
     ENG_SCOPE(26);
-    PlayerList all = TeamActivePlayers(w, teamID);
+    const PlayerList all = TeamActivePlayers(w, teamID);
     PlayerList ps;
     if (!all.empty()) {
         // GRF: removes the first goalkeeper; only one listed first is supported.
@@ -616,9 +618,12 @@ HD void ReconsiderDesignatedPlayer(World &w, int teamID) {
 HDN void SpatialStatesAhead(GlobalRef<World> world, LocalRef<const Ctx> context, int teamID) {
     World &w = world;
     const Ctx &c = context;
-    const PlayerList ahead = TeamActivePlayers(w, teamID);
-    for (int i = GroupRank(); i < ahead.count; i += kGroupLanes)
-        c.ws->spatialAhead[ahead[i]] = NextSpatialState(c, Hum(w, ahead[i]));
+    const PlayerSet ahead = TeamActivePlayers(w, teamID);
+    const int count = ahead.size();
+    for (int i = GroupRank(); i < count; i += kGroupLanes) {
+        const int p = ahead[i];
+        c.ws->spatialAhead[p] = NextSpatialState(c, Hum(w, p));
+    }
     GroupSync();
 }
 HDN bool TeamProcess(GlobalRef<World> world, LocalRef<const Ctx> context, int teamID) {

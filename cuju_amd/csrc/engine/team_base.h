@@ -91,9 +91,19 @@ HD void PropertiesSet(Tactics &t, int id, float value) {
     t.value[id] = RoundTripSixDecimals(value);
 }
 
+// At most kTeamPlayers players in an order, five bits each, so that a call returns them in registers.
+struct PlayerRanking {
+    uint64_t players = 0;
+    int count = 0;
+    HD int size() const { return count; }
+    HD bool empty() const { return count == 0; }
+    HD int operator[](int i) const { return (int)(players >> (5 * i)) & 31; }
+    HD void Set(int i, int p) { players |= (uint64_t)p << (5 * i); }
+};
+static_assert(kPlayers <= 32 && 5 * kTeamPlayers <= 64, "a ranking is a word");
 // The same list by GRF's insertion sort, one player after another, for distances that hold NaN: an
 // insertion lands after the last kept entry it is not nearer than.
-HDN PlayerList ClosestPlayersByInsertion(GlobalRef<const World> world, LocalRef<const Ctx> context, unsigned count, int n) {
+HDN PlayerRanking ClosestPlayersByInsertion(GlobalRef<const World> world, LocalRef<const Ctx> context, unsigned count, int n) {
     const World &w = world;
     const Ctx &c = context;
     const float *const dist = c.ws->teamValues;
@@ -107,8 +117,10 @@ HDN PlayerList ClosestPlayersByInsertion(GlobalRef<const World> world, LocalRef<
         for (int s = order.count - 1; s > at; s--) order[s] = order[s - 1];
         order[at] = p;
     }
-    if ((unsigned)order.count > count) order.count = (int)count;
-    return order;
+    PlayerRanking r;
+    r.count = (unsigned)order.count < count ? order.count : (int)count;
+    for (int i = 0; i < r.count; i++) r.Set(i, order[i]);
+    return r;
 }
 // The closest active players of a team to `pos`, nearest first, ties in state order: the first
 // `count` of a stable sort by distance. The lanes of the match take the players in turn, first for
@@ -116,7 +128,7 @@ HDN PlayerList ClosestPlayersByInsertion(GlobalRef<const World> world, LocalRef<
 // most kTeamPlayers players. Every lane of the match must make the call. One lane's insertions in
 // registers took 20 K cycles a call; ms per step before and after, with GetClosestPlayer: one match of
 // 64 lanes 10.8 -> 10.7, 4,096 of 32 lanes 37.8 -> 37.4, 16,384 of 8 lanes 107.6 -> 106.5.
-HDN PlayerList GetClosestPlayers(GlobalRef<const World> world, LocalRef<const Ctx> context, int teamID, Vec3 pos, bool onlyAI, unsigned count = 3,
+HDN PlayerRanking GetClosestPlayers(GlobalRef<const World> world, LocalRef<const Ctx> context, int teamID, Vec3 pos, bool onlyAI, unsigned count = 3,
                                  bool onlySelectable = false) {
     const World &w = world;
     const Ctx &c = context;
@@ -152,13 +164,13 @@ HDN PlayerList GetClosestPlayers(GlobalRef<const World> world, LocalRef<const Ct
         for (int k = 0; k < kRounds; k++)
             place[k] += (other >= 0) & ((other < dist[k]) | ((other == dist[k]) & (q < k * kGroupLanes + GroupRank())));
     }
-    PlayerList r;
+    PlayerRanking r;
     r.count = (unsigned)n < count ? n : (int)count;
     for (int i = 0; i < r.count; i++) {
 #pragma unroll
         for (int k = 0; k < kRounds; k++) {
             const LaneMask here = GroupBallot(dist[k] >= 0 && place[k] == i);
-            if (here) r[i] = k * kGroupLanes + LowestBit(here);
+            if (here) r.Set(i, k * kGroupLanes + LowestBit(here));
         }
     }
     return r;
@@ -221,7 +233,7 @@ HDN int SwitchTargetPlayer(GlobalRef<const World> world, LocalRef<const Ctx> con
     const World &w = world;
     const Ctx &c = context;
     const int designated = w.match.designatedPossessionPlayer;
-    const PlayerList nearest = GetClosestPlayers(w, c, teamID, SwitchFocus(w, teamID), true, 8);
+    const PlayerRanking nearest = GetClosestPlayers(w, c, teamID, SwitchFocus(w, teamID), true, 8);
     PlayerList field;
     for (int i = 0; i < nearest.count; i++)
         if (Formation(w, c, nearest[i]).role != kRoleGoalkeeper) field.push_back(nearest[i]);

@@ -376,7 +376,7 @@ HD Vec3 LeadPoint(const SpatialState &mate, const Vec3 &origin) {
 // The teammate a pass toward `manual` (input direction `inDir`) goes to, and where: the lowest
 // rating of distance from the manual target (over 70 m, to the 0.8, times 0.8) plus angle off the
 // input direction (in half turns); the passer, at the origin, without teammates.
-HD int PassReceiver(const World &w, int p, const PlayerList &players, const Vec3 &origin, const Vec3 &manual, const Vec3 &inDir,
+HD int PassReceiver(const World &w, int p, const PlayerSet &players, const Vec3 &origin, const Vec3 &manual, const Vec3 &inDir,
                     Vec3 &aim) {
     int best = p;
     float bestRating = 10000;
@@ -406,7 +406,7 @@ HDN void AimPass(GlobalRef<const World> world, int p, int passType, Vec3 inDir, 
     const int teamID = w.playerTeamID[p];
     const Vec3 origin = PassOrigin(w, p);
     const Vec3 manual = origin + inDir * Clamp(inPower * 60.0f, 1.0f, 100.0f);
-    const PlayerList players = TeamActivePlayers(w, teamID);
+    const PlayerSet players = TeamActivePlayers(w, teamID);
     const bool alone = players.size() < 2;
     const bool automatic = ExternalControllerActive(w, p) && !alone;
     float dirBias = alone ? 0.0f : autoDirBias, powerBias = alone ? 0.0f : autoPowerBias;

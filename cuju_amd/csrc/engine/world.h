@@ -336,22 +336,52 @@ HD PlayerList TeamAllPlayers(const World &w, int teamID) {
         if (w.playerTeamID[p] == teamID) l.push_back(p);
     return l;
 }
-// The active players of a team in state order. Every player's two tests load and combine without
-// an early exit (the slots past the match's players are in the arrays), so the scan waits for
-// memory once rather than once a player; each player is written at the list's end, which moves
-// on when the player belongs.
-HD PlayerList TeamActivePlayers(const World &w, int teamID) {
-    PlayerList l;
-    const int players = w.match.playerCount;
-    int count = 0;
+// A set of players, a bit each, read as the list of them in state order: by a loop over the set, or by
+// index. A list of up to 22 entries lies on the lane's stack, behind a store for every player and a
+// load for every use. Measured, ms per step: 4,096 matches of 32 lanes 37.4 -> 36.6, 8,192 of 16 lanes
+// 70.2 -> 68.3, 16,384 of 8 lanes 106.5 -> 104.6.
+struct PlayerSet {
+    uint32_t mask = 0;
+    HD int size() const { return PopCount(mask); }
+    HD bool empty() const { return mask == 0; }
+    // The n-th player: the half that holds its bit, then half of that half.
+    HD int operator[](int n) const {
+        int at = 0;
 #pragma unroll
-    for (int p = 0; p < kPlayers; p++) {
-        const bool in = (p < players) & (w.playerTeamID[p] == teamID) & w.roster.active[p];
-        l.e[count] = p;
-        count += in ? 1 : 0;
+        for (int half = 16; half > 0; half >>= 1) {
+            const int below = PopCount((mask >> at) & ((1u << half) - 1u));
+            const bool above = n >= below;
+            n -= above ? below : 0;
+            at += above ? half : 0;
+        }
+        return at;
     }
-    l.count = count;
-    return l;
+    struct Iterator {
+        uint32_t left;
+        HD int operator*() const { return LowestBit(left); }
+        HD void operator++() { left &= left - 1; }
+        HD bool operator!=(const Iterator &o) const { return left != o.left; }
+    };
+    HD Iterator begin() const { return Iterator{mask}; }
+    HD Iterator end() const { return Iterator{0}; }
+    HD operator PlayerList() const {
+        PlayerList l;
+        for (int p : *this) l.e[l.count++] = p;
+        return l;
+    }
+};
+static_assert(kPlayers <= 32, "a set of players is a word");
+// The active players of a team. The lanes of the match test the players in turn; every lane of the
+// match must make the call.
+HD PlayerSet TeamActivePlayers(const World &w, int teamID) {
+    PlayerSet s;
+    const int players = w.match.playerCount;
+#pragma unroll
+    for (int base = 0; base < kPlayers; base += kGroupLanes) {
+        const int p = base + GroupRank(), at = p < kPlayers ? p : 0;
+        s.mask |= (uint32_t)GroupBallot((p < players) & (w.playerTeamID[at] == teamID) & w.roster.active[at]) << base;
+    }
+    return s;
 }
 HD int TeamDynamicSide(const World &w, int teamID) { return w.flags.teamSide[teamID]; }
 

@@ -657,8 +657,10 @@ void SetupAgents(World &w, const StaticData &sd, int left, int right, const std:
     for (int t = 0; t < 2; t++) {
         if (agents[t] == 0) continue;
         const Vec3 ball = BallPredict(m.ball, 0).Get2D();
-        PlayerList ps = GetClosestPlayers(w, c, t, ball, true, (unsigned)agents[t], true);
-        if (ps.empty()) continue;
+        const PlayerRanking nearest = GetClosestPlayers(w, c, t, ball, true, (unsigned)agents[t], true);
+        if (nearest.empty()) continue;
+        PlayerList ps;
+        for (int i = 0; i < nearest.count; i++) ps.push_back(nearest[i]);
         TeamByID(w, t).mainSelectedPlayer = ps[0];
         for (int i = 1; i < ps.count; i++)
             for (int j = i; j > 0 && sd.stableID[ps[j]] < sd.stableID[ps[j - 1]]; j--) {
