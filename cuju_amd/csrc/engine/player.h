@@ -370,8 +370,10 @@ HDN bool AnimationTouch(GlobalRef<World> world, LocalRef<const Ctx> context, int
         o.ry = o.momentum.Normalized(0).v[0] * (speed * forwardness);
         o.bias = 0.9f * (1.0f - bumpy);
     }
-    if (o.touch) BallTouch(w, c, o.momentum);
-    if (o.rotate) BallSetRotation(w, o.rx, o.ry, o.rz, o.bias);
+    SecondFlight second;
+    if (o.rotate) second.rotation = TurnedRotation(w.match.ball.rotationPerMs, o.rx, o.ry, o.rz, o.bias);
+    if (o.touch) BallTouch(w, c, o.momentum, o.rotate ? &second : nullptr);
+    if (o.rotate) BallSetRotation(w, c, second.rotation, o.touch);
     return TeamSetLastTouchPlayer(w, c, p, o.type);
 }
 
@@ -485,8 +487,7 @@ HD bool ControlledCollision(World &w, const Ctx &c, int p, const Anim &a, const 
     if (cur.originatingCommand.modifier & kModifierKnockOn) momentum *= 1.35f;
     const float bumpy = 0.0f;
     momentum = momentum * (1.0f - bumpy) + incoming * bumpy;
-    BallTouch(w, c, momentum);
-    BallSetRotation(w, k.xRot, k.yRot, 0, 0.2f * (1.0f - bumpy));
+    BallTouchAndTurn(w, c, momentum, k.xRot, k.yRot, 0, 0.2f * (1.0f - bumpy));
     return TeamSetLastTouchPlayer(w, c, p, d.touchType);
 }
 // At the animation's touch frame the ball is touched when it lies within 0.4 m of the planned
@@ -534,11 +535,7 @@ HD bool CarryRetainedBall(World &w, const Ctx &c, int p, const Anim &a, const An
     Transform der[kHumanoidNodes];
     WorldTransforms(sk, h.nodes, der);
     const Transform &node = der[sk.nodeMap[part]];
-    BallTouch(w, c, Vec3(0));
-    // BallSetPosition predicts again from its own position before anything reads the
-    // predictions, so this rotation's prediction is left out.
-    BallSetRotation(w, 0, 0, 0, 1.0f, false);
-    BallSetPosition(w, node.position + node.rotation * Vec3(0, 0, -0.36f));
+    BallCarry(w, c, node.position + node.rotation * Vec3(0, 0, -0.36f));
     return TeamSetLastTouchPlayer(w, c, p, kTouchNonKicked);
 }
 // One frame's share of a smuggle spread over `span` frames, weighted by a raised cosine (0.9 to

@@ -419,11 +419,10 @@ HD void DeflectBall(World &w, const Ctx &c, Vec3 bounce, int bounces, float dept
     Vec3 res = full * bias + cur * (1.0f - bias);
     if (res.Length() > cur.Length()) res = res.Normalized(0) * cur.Length();
     res *= 0.7f;
-    BallTouch(w, c, res);
     const float rz = RandomInRange(w, -30, 30);
     const float ry = RandomInRange(w, -30, 30);
     const float rx = RandomInRange(w, -30, 30);
-    BallSetRotation(w, rx, ry, rz, 0.5f * bias);
+    BallTouchAndTurn(w, c, res, rx, ry, rz, 0.5f * bias);
     m.lastBodyBallCollisionTimeMs = (uint32_t)m.actualTimeMs;
 }
 // The ball against the players' bodies, at most every 150 ms, players in processing order. A

@@ -448,6 +448,20 @@ struct ApplyPlan {
     float beginBias;
 };
 
+// What a flight of the ball starts from, and a flight computed before its turn comes: its start,
+// whether it was flown, its first step's results and its predictions.
+struct FlightStart {
+    Vec3 position, momentum;
+    Quat orientation, rotation;
+};
+struct FlightAhead {
+    FlightStart start;
+    bool flown, touchesNet;
+    Vec3 momentum;
+    Quat rotation, orientation;
+    Vec3 predictions[401];
+};
+
 // Per-match working memory: the animation selection's candidate lists, planned positions, sort keys
 // and one candidate plan per lane of the match, and the lists above. One block per environment in
 // HBM, which every lane of the match addresses, in place of large per-lane stack arrays: the lanes
@@ -475,6 +489,7 @@ struct Scratch {
     int16_t order[2][kMaxAnimations];
     SpatialState spatialAhead[kPlayers + 3];  // spatial states computed ahead: the players', then the officials'
     PlanFrame planFrames[kAnimPositions];     // a movement plan's frame terms, computed ahead
+    FlightAhead flightAhead;                  // a touched ball's second flight, flown with its first
 };
 
 // Everything a match reads besides its world: the shared tables, its variant's static data and
