@@ -48,7 +48,7 @@ struct BallFlight {
 
     HD Vec3 Angles() {
         if (!anglesKnown) {
-            rot.Angles(angles.v[0], angles.v[1], angles.v[2]);
+            angles = EulerAnglesInHalves(rot);
             anglesKnown = true;
         }
         return angles;
@@ -168,8 +168,8 @@ struct BallFlight {
     HD void Roll(const Contact &c) {
         const float spinX = mom.v[1] / kRadius, spinY = mom.v[0] / kRadius;
         Quat rx, ry;
-        rx.SetAngleAxis(Clamp(spinX * 0.001f, -PI * 0.49f, PI * 0.49f), Vec3(-1, 0, 0));
-        ry.SetAngleAxis(Clamp(spinY * 0.001f, -PI * 0.49f, PI * 0.49f), Vec3(0, 1, 0));
+        AxisTurnsInHalves(Clamp(spinX * 0.001f, -PI * 0.49f, PI * 0.49f), Vec3(-1, 0, 0),
+                          Clamp(spinY * 0.001f, -PI * 0.49f, PI * 0.49f), Vec3(0, 1, 0), rx, ry);
         const Quat rolling = rx * ry;
         Quat toRolling = rot.RotationTo(rolling).Normalized();
         // The turn's angle to the identity is the angle of its scalar, whose arc cosine also scales it.

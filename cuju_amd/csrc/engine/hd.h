@@ -212,6 +212,15 @@ HD double GroupShuffle(double v, int rank) {
     memcpy(&r, &b, 8);
     return r;
 }
+// The value of the lane whose rank differs in bit 1, for groups of at least 4 lanes (two lanes of a
+// quad exchange in a register move, without the LDS unit). Both lanes must make the call.
+HD float OppositeOfQuad(float v) {
+#if ENG_DEVICE
+    return FloatOf((uint32_t)__builtin_amdgcn_mov_dpp((int)BitsOf(v), 0x4e, 0xf, 0xf, true));
+#else
+    return v;
+#endif
+}
 // Leaves every lane of the group with the first of the lanes' candidates in a total order:
 // `takeIfBefore(r)` compares this lane's candidate with that of the lane of rank r and keeps the
 // earlier. Each round pairs the lanes, so 64 lanes take 6 rounds; taking one lane's candidate after
