@@ -402,15 +402,10 @@ struct WorldGeometry {
     Aabb box;
     Vec3 position;
 };
-struct PlayerGeometry {
-    bool footOrLowerLeg;
-    WorldGeometry wg;
-};
-using PlayerGeometryList = Small<PlayerGeometry, kHumanoidNodes * 2>;
 
 // Lists that the match's sequential code fills and reads within one call: an interruption's
 // command queue, one force field of the AI or the referee, the bounces of the collision pass and
-// the geometry of a tackler and its victim.
+// the boxes of a tackled player's feet.
 constexpr int kMaxCommands = 16;
 using CommandQueue = Small<PlayerCommand, kMaxCommands>;
 enum MagnetType { kAttract, kRepel };
@@ -471,7 +466,7 @@ struct Scratch {
     CommandQueue commands;
     ForceField forceField;
     PlayerBounceList bounces[kPlayers];
-    PlayerGeometryList tackleGeometry[2];
+    Aabb tackleFeet[2 * kHumanoidNodes];
     Vec3 contactAt[kPlayers];
     ApplyPlan applyPlans[kPlayers + 3];
     // The working lists of team queries that the lanes of the match share: a value and a place per
