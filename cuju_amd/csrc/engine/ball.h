@@ -624,8 +624,9 @@ struct TimeNeededScan {
 // time itself, as the possession scan asks them.
 //
 // After n of the walk's steps its position is from + movement s(n) and its radii 0.28 and 0.9 plus
-// amv b(n), with b and s the sums of the bias and of its rest in closed form, each up to the
-// rounding of 70 additions: 4.2e-6 of the coordinates, under the margin (1 mm and 1e-5 of them). A
+// amv b(n), with b and s the sums of the bias and of its rest in closed form (at most 0.345 and 0.355),
+// each up to the rounding of 70 additions: 4.2e-6 of the largest value they pass through, the start's
+// coordinates plus the way walked or the radii, under the margin (1 mm and 1e-5 of their sum). A
 // target nearer than a radius less the margin after some step is reached there; one farther than
 // the radius and the margin after every step is not. Pieces of eight steps are ruled out by the
 // nearest point of their path against the radius at their end, and the steps of the others are
@@ -636,7 +637,7 @@ struct TimeNeededScan {
 struct ReachScan {
     static constexpr int kPiece = 8;
     Vec3 pos, mov, start;
-    float maxVel, amv, perSpeed2;
+    float maxVel, amv, perSpeed2, walked;  // `walked`: at least the way and the radii's growth
     bool moving;
 
     HD ReachScan(const Vec3 &p, const Vec3 &m, float velocity) : pos(p), mov(m), start(p), maxVel(velocity) {
@@ -644,6 +645,7 @@ struct ReachScan {
         moving = mov.Length() > kIdleDribbleSwitch;
         const float speed2 = mov.v[0] * mov.v[0] + mov.v[1] * mov.v[1];
         perSpeed2 = speed2 > 0.0f ? 1.0f / speed2 : 0.0f;
+        walked = (fabsf(mov.v[0]) + fabsf(mov.v[1])) * 0.36f + amv * 0.35f;
         if (moving) {
             start += mov.Normalized() * 0.1f;
             start += mov * 0.01f;
@@ -666,7 +668,7 @@ struct ReachScan {
         Vec3 from = start;
         if (!moving) from += (target - pos).Normalized(0) * 0.1f;
         const Vec3 v = target - from;
-        const float margin = 0.001f + (fabsf(from.v[0]) + fabsf(from.v[1])) * 1e-5f;
+        const float margin = 0.001f + (fabsf(from.v[0]) + fabsf(from.v[1]) + walked) * 1e-5f;
         const float along = (v.v[0] * mov.v[0] + v.v[1] * mov.v[1]) * perSpeed2;
         const uint32_t limit = ms / 10 + 1;
         const int steps = limit < (uint32_t)kTimeWalkSteps ? (int)limit : kTimeWalkSteps;

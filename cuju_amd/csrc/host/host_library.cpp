@@ -182,6 +182,29 @@ extern "C" __attribute__((visibility("default"))) void cuju_debug_time_needed(co
     }
 }
 
+// Whether a player reaches targets by given times, for `count` cases of the same values as above (the
+// limit is the time): GetTimeNeededMs's answers, then whether the closed form decided and its answers
+// (usual and optimistic, both times); tests compare them. A target beyond the walk's range is not
+// asked of the closed form, as in a possession scan.
+extern "C" __attribute__((visibility("default"))) void cuju_debug_reached(const float *cases, int count, unsigned char *out) {
+    for (int i = 0; i < count; i++) {
+        const float *q = cases + (size_t)i * 12;
+        const eng::Vec3 pos(q[0], q[1], q[2]), mov(q[3], q[4], q[5]), target(q[6], q[7], q[8]);
+        const bool precise = q[10] != 0.0f;
+        const uint32_t ms = (uint32_t)q[11];
+        const eng::TimeNeeded t = eng::GetTimeNeededMs(pos, mov, target, q[9], precise, ms);
+        bool usual = false, optimistic = false;
+        const bool near = !(pos - target).LengthAbove(precise ? 48.0f : 16.0f);
+        const bool decided = near && eng::ReachScan(pos, mov, q[9]).Decide(target, ms, usual, optimistic);
+        unsigned char *const o = out + (size_t)i * 5;
+        o[0] = t.usual <= ms;
+        o[1] = t.optimistic <= ms;
+        o[2] = decided;
+        o[3] = usual;
+        o[4] = optimistic;
+    }
+}
+
 // The bytes of one environment's blocks in device memory: World, EnvCore, EnvSlot and Scratch. The
 // engine's structs have the same layout on the host and the device.
 extern "C" __attribute__((visibility("default"))) void cuju_debug_layout(unsigned long long *out) {

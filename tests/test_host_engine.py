@@ -195,6 +195,49 @@ def test_time_walk_matches_the_direct_estimate(host_library):
     assert walked.sum() > n // 3
 
 
+@pytest.mark.parametrize('slowest,fastest', [(0, 2), (2, 12), (12, 200), (2e3, 2e4), (2e4, 2e6)])
+def test_reach_in_closed_form_is_the_walk(slowest, fastest, host_library):
+    """What the possession scan's closed form decides (ball.h, ReachScan::Decide) equals the walk's
+    answer (ai_time.h:102-409), at every speed of the player, those of a loaded state included: targets
+    within a few mm of both radii at every step of the walk, times at which a target is just reached or
+    just not, and times about the walk's end."""
+    lib = ctypes.CDLL(host_library)
+    rng = np.random.default_rng(17)
+    n = 600_000
+    pos = np.column_stack([rng.uniform(-55, 55, n), rng.uniform(-36, 36, n), np.zeros(n)])
+    speed, angle = rng.uniform(slowest, fastest, n), rng.uniform(-np.pi, np.pi, n)
+    mov = np.column_stack([speed * np.cos(angle), speed * np.sin(angle), np.zeros(n)])
+    velocity = rng.uniform(1, 10, n)
+    # Half of the targets near a radius after a step, the others anywhere within 48 m.
+    k = rng.integers(1, 71, n)
+    growth = k * (k - 1) * 0.01 / 140
+    start = pos[:, :2] + np.where(speed > 1.8, 0.1 / np.maximum(speed, 1e-9) + 0.01, 0.0)[:, None] * mov[:, :2]
+    start += (k * 0.01 - growth)[:, None] * mov[:, :2]
+    radius = rng.choice([0.28, 0.9], n) + velocity * 0.94 * growth + rng.uniform(-0.003, 0.003, n)
+    near, turn = rng.uniform(size=n) < 0.5, rng.uniform(-np.pi, np.pi, n)
+    reach = np.where(near, radius, rng.uniform(0, 48, n))
+    at = np.where(near[:, None], start, pos[:, :2])
+    target = np.column_stack([at[:, 0] + reach * np.cos(turn), at[:, 1] + reach * np.sin(turn), np.zeros(n)])
+    cases = np.column_stack([pos, mov, target, velocity, rng.integers(0, 2, n), np.full(n, -1.0)]).astype(np.float32)
+    times = np.zeros((n, 6), dtype=np.uint32)
+    lib.cuju_debug_time_needed(ctypes.c_void_p(cases.ctypes.data), n, ctypes.c_void_p(times.ctypes.data))
+    needed = np.where(rng.uniform(size=n) < 0.5, times[:, 0], times[:, 1]).astype(float)
+    needed += rng.integers(-2, 3, n)
+    limit = np.where(rng.uniform(size=n) < 0.7, needed, rng.uniform(10, 3000, n))
+    about = rng.uniform(size=n) < 0.1
+    limit[about] = rng.integers(680, 711, about.sum())
+    cases[:, 11] = np.clip(np.round(limit), 0, 1 << 24)
+    out = np.zeros((n, 5), dtype=np.uint8)
+    lib.cuju_debug_reached(ctypes.c_void_p(cases.ctypes.data), n, ctypes.c_void_p(out.ctypes.data))
+    decided = out[:, 2] == 1
+    wrong = np.flatnonzero(decided & ((out[:, 3] != out[:, 0]) | (out[:, 4] != out[:, 1])))
+    assert wrong.size == 0, f'{wrong.size} of {decided.sum()} decisions differ, the first for {cases[wrong[0]]}'
+    # In play the closed form decides most of even these targets.
+    if fastest <= 12:
+        assert decided[np.linalg.norm(target - pos, axis=1) < 16].mean() > 0.5
+        assert (out[decided, 0] == 1).any() and (out[decided, 0] == 0).any()
+
+
 def test_device_time_bias_rounds_as_the_division():
     """The device computes GRF's acceleration bias (10 k) / 700 as a reciprocal product with one
     fused correction (engine/ball.h, TimeNeededBias); for every step index the walks use (k < 200)
