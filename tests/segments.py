@@ -15,7 +15,8 @@ reference library plays the same batch (same environments, states and inputs); e
 environment's digest over its block's steps (the observation after the reset or the state load,
 then every step's observation, reward, done flag and final observation, and the observations of
 its masked resets) and its state at the end must be equal. Block 0 is the start of
-`tests/golden/episodes.json`'s end range, so its digests at step 3,000 are also those goldens.
+`tests/golden/episodes.json`'s end range, so its digests at step 3,000 are also those goldens: where
+the reference library is not built, the device plays block 0 alone against them.
 
 The oracle here is test infrastructure: it supplies the states the blocks start from and the
 digests they must reach.
@@ -231,12 +232,12 @@ def play_oracle(run):
 class DeviceBlocks:
     """The four-block batch on the device, on a stream of its own."""
 
-    def __init__(self, workload, drill_paths, library, matches_per_wavefront, stream=None):
+    def __init__(self, workload, drill_paths, library, matches_per_wavefront, stream=None, blocks=BLOCKS):
         import ctypes
         import cuju_amd
         import lockstep
         self.ctypes = ctypes
-        options = block_options(workload, drill_paths)
+        options = block_options(workload, drill_paths, blocks)
         assets = options.pop('assets')
         with lockstep.matches_per_wavefront(matches_per_wavefront):
             self.batch = cuju_amd.BatchEnvironment(assets, library=library, device='cuda:0',
