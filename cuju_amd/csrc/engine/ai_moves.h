@@ -453,7 +453,7 @@ struct AIBase {
                     GroupSync();
                     built = true;
                 }
-                tn = walks ? WalkTimeNeeded(walk, pp, mov, target, maxVel, true, t, true) : GetTimeNeededMs(pp, mov, target, maxVel, true, t);
+                tn = walks ? WalkTimeNeeded(walk, pp, mov, target, maxVel, true, t) : GetTimeNeededMs(pp, mov, target, maxVel, true, t);
             }
             const unsigned needed = tn.usual;
             int next = TruncToInt32(roundf((float)(int)(needed - t) * 0.05f)) - 5;

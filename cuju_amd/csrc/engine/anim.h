@@ -451,7 +451,6 @@ HDN int BodyDirectionIndex(Vec3 src) {
     }
     return bi;
 }
-HD Vec3 BodyDirectionSnapped(const Vec3 &src) { return AllowedBodyDir(BodyDirectionIndex(src)); }
 
 // Ground-plane movement in m/s at `frame` of a position list of two frames or more.
 HDN Vec3 MovementAtFrame(GlobalPointer<const Vec3> pos, int count, uint32_t frame, uint32_t smooth) {

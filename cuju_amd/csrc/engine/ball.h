@@ -440,8 +440,8 @@ HD TimeNeeded GetTimeNeededMs(const Vec3 &pos, const Vec3 &mov, const Vec3 &targ
 
 // GetTimeNeededMs split in two for a player whose movement exceeds the idle threshold: the walk,
 // which every target shares, and the search along it for one target. The search gives the same
-// result as GetTimeNeededMs. With `cooperative` the lanes of the match (all running the same
-// sequential code) test consecutive steps of the walk together.
+// result as GetTimeNeededMs: the lanes of the match (all running the same sequential code) test
+// consecutive steps of the walk together.
 HD bool TimeWalkApplies(const Vec3 &mov) { return mov.Length() > kIdleDribbleSwitch; }
 HDN void BuildTimeWalk(GlobalRef<TimeWalk> timeWalk, Vec3 pos, Vec3 mov, float maxVel) {
     TimeWalk &wk = timeWalk;
@@ -469,7 +469,7 @@ HDN void BuildTimeWalk(GlobalRef<TimeWalk> timeWalk, Vec3 pos, Vec3 mov, float m
     }
 }
 HDN TimeNeeded WalkTimeNeeded(GlobalRef<const TimeWalk> timeWalk, Vec3 pos, Vec3 mov, Vec3 target, float maxVel,
-                              bool precise, uint32_t maxTime, bool cooperative) {
+                              bool precise, uint32_t maxTime) {
     const TimeWalk &wk = timeWalk;
     TimeNeeded r;
     if ((pos - target).Length() > (precise ? 48.0f : 16.0f)) {
@@ -478,10 +478,9 @@ HDN TimeNeeded WalkTimeNeeded(GlobalRef<const TimeWalk> timeWalk, Vec3 pos, Vec3
         return r;
     }
     const bool limited = maxTime != (uint32_t)-1;
-    const int stride = cooperative ? kGroupLanes : 1, rank = cooperative ? GroupRank() : 0;
     int reach = -1, optimistic = -1;
-    for (int k0 = 0; k0 < kTimeWalkSteps && reach < 0; k0 += stride) {
-        const int k = k0 + rank;
+    for (int k0 = 0; k0 < kTimeWalkSteps && reach < 0; k0 += kGroupLanes) {
+        const int k = k0 + GroupRank();
         bool u = false, o = false;
         if (k < kTimeWalkSteps) {
             const bool late = limited && (uint32_t)(k * 10) > maxTime;
@@ -490,8 +489,8 @@ HDN TimeNeeded WalkTimeNeeded(GlobalRef<const TimeWalk> timeWalk, Vec3 pos, Vec3
             o = d2 < wk.optimisticSquared[k] || late;
             u = d2 < wk.usualSquared[k] || late;
         }
-        const LaneMask um = cooperative ? GroupBallot(u) : (LaneMask)u;
-        LaneMask om = cooperative ? GroupBallot(o) : (LaneMask)o;
+        const LaneMask um = GroupBallot(u);
+        LaneMask om = GroupBallot(o);
         if (um) {
             reach = k0 + LowestBit(um);
             om &= LanesThrough(LowestBit(um));  // the optimistic test comes first within a step
@@ -541,7 +540,7 @@ HDN TimeNeeded WalkTimeNeeded(GlobalRef<const TimeWalk> timeWalk, Vec3 pos, Vec3
 // the walk stops: one step past the time limit, or the end of the bias at 700 ms. The radii there
 // are the same for every target, and so is the position for a moving player; an idle player
 // starts a tenth of a metre towards the target, so its position is walked per target, without
-// the tests. Every other target runs GetTimeNeededMs itself, so the results are GetTimeNeededMs's.
+// the tests.
 struct TimeNeededScan {
     Vec3 pos, mov, start, end;
     float maxVel, amv, reach, endUsual = 0, endOptimistic = 0;
@@ -611,11 +610,6 @@ struct TimeNeededScan {
             r.optimistic = r.usual;
         }
         return true;
-    }
-    HD TimeNeeded Get(const Vec3 &target, bool precise, uint32_t maxTime) {
-        TimeNeeded r;
-        if (Unreachable(target, precise, maxTime, r)) return r;
-        return GetTimeNeededMs(pos, mov, target, maxVel, precise, maxTime);
     }
 };
 

@@ -93,9 +93,9 @@ struct ReducedAngle {
         if (kGroupLanes == kMaxGroupLanes && Top12f(y) < Top12f(0x1.921FB6p-1f)) {
             n = turn = 0;
         } else if (Top12f(y) < Top12f(120.0f)) {
-            const int q = (int32_t)(x * DoubleOf(kSinCosfCoefficients[4]));
+            const int q = (int32_t)(x * DoubleOf(kSinCosfCoefficients[0]));
             n = turn = (q + 0x800000) >> 24;
-            x = Fma(-(double)n, DoubleOf(kSinCosfCoefficients[5]), x);
+            x = Fma(-(double)n, DoubleOf(kSinCosfCoefficients[1]), x);
         } else {
             x = ReduceLarge(BitsOf(y), &n);
             turn = n + (int)(BitsOf(y) >> 31);
@@ -104,16 +104,16 @@ struct ReducedAngle {
     }
     // The sign of the reduced argument is - for turns 1 and 2 (mod 4), the cosine's for 2 and 3.
     HD float Sine() const {
-        const double s1 = DoubleOf(kSinCosfCoefficients[8]), s2 = DoubleOf(kSinCosfCoefficients[10]),
-                     s3 = DoubleOf(kSinCosfCoefficients[12]);
+        const double s1 = DoubleOf(kSinCosfCoefficients[4]), s2 = DoubleOf(kSinCosfCoefficients[6]),
+                     s3 = DoubleOf(kSinCosfCoefficients[8]);
         const double x3 = x * x2;
         const float sine = (float)Fma(x3 * x2, Fma(x2, s3, s2), Fma(x3, s1, x));
         return FloatOf(BitsOf(sine) ^ (((uint32_t)(turn + 1) & 2) << 30));
     }
     HD float Cosine() const {
-        const double c0 = DoubleOf(kSinCosfCoefficients[6]), c1 = DoubleOf(kSinCosfCoefficients[7]),
-                     c2 = DoubleOf(kSinCosfCoefficients[9]), c3 = DoubleOf(kSinCosfCoefficients[11]),
-                     c4 = DoubleOf(kSinCosfCoefficients[13]);
+        const double c0 = DoubleOf(kSinCosfCoefficients[2]), c1 = DoubleOf(kSinCosfCoefficients[3]),
+                     c2 = DoubleOf(kSinCosfCoefficients[5]), c3 = DoubleOf(kSinCosfCoefficients[7]),
+                     c4 = DoubleOf(kSinCosfCoefficients[9]);
         const double x4 = x2 * x2;
         const float cosine = (float)Fma(x4 * x2, Fma(x2, c4, c3), Fma(x4, c2, Fma(x2, c1, c0)));
         return FloatOf(BitsOf(cosine) ^ (((uint32_t)turn & 2) << 30));

@@ -1149,13 +1149,6 @@ struct Selector {
         const Ctx &c = context;
         return c.T().selection[i].lookAngle;
     }
-    HD Vec3 SmoothedMovement(int i, uint32_t frame) {
-        const Ctx &c = context;
-        const Anim &a = A(i);
-        int32_t first = c.T().selection[i].smoothedFirst;
-        if (first >= 0 && frame < (uint32_t)a.posCount) return c.T().smoothed[first + frame];
-        return MovementAtFrame(c.T().positions + a.posFirst, a.posCount, frame, 1);
-    }
 
     HD void SetMovementSimilarityPredicate(const Vec3 &relDesired, int desiredVel) {
         pred.relDesiredDirection = relDesired;

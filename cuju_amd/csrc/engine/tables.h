@@ -469,10 +469,9 @@ struct Scratch {
     Aabb tackleFeet[2 * kHumanoidNodes];
     Vec3 contactAt[kPlayers];
     ApplyPlan applyPlans[kPlayers + 3];
-    // The working lists of team queries that the lanes of the match share: a value and a place per
-    // player, and the dynamic roles' slots and costs.
+    // The working lists of team queries that the lanes of the match share: a value per player, and the
+    // dynamic roles' slots and costs.
     float teamValues[kPlayers];
-    int32_t teamOrder[kPlayers];
     Vec3 roleSlots[kTeamPlayers];
     int32_t roleCosts[kTeamPlayers * kTeamPlayers], roleSorted[kTeamPlayers * kTeamPlayers];
     int16_t lists[3][kMaxAnimations];

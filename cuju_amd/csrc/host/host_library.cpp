@@ -153,7 +153,8 @@ extern "C" __attribute__((visibility("default"))) void cuju_debug_world_rng(unsi
 }
 
 // GRF's time-to-target estimate for `count` cases: directly, along the shared walk, and by the
-// possession scan's shortcut (usual and optimistic times of each, direct first); tests compare them.
+// shortcut of the AI's chase for targets the walk cannot reach, directly for the others (usual and
+// optimistic times of each, direct first); tests compare them.
 extern "C" __attribute__((visibility("default"))) void cuju_debug_time_needed(const float *cases, int count, unsigned int *out) {
     auto walk = std::make_unique<eng::TimeWalk>();
     std::unique_ptr<eng::TimeNeededScan> scan;
@@ -167,12 +168,13 @@ extern "C" __attribute__((visibility("default"))) void cuju_debug_time_needed(co
         eng::TimeNeeded b = a;
         if (eng::TimeWalkApplies(mov)) {
             eng::BuildTimeWalk(*walk, pos, mov, maxVel);
-            b = eng::WalkTimeNeeded(*walk, pos, mov, target, maxVel, precise, maxTime, false);
+            b = eng::WalkTimeNeeded(*walk, pos, mov, target, maxVel, precise, maxTime);
         }
-        // Consecutive cases of one player share a scan, as the targets of a possession scan do.
+        // Consecutive cases of one player share a scan, as the targets of a chase do.
         if (!scan || !(scan->pos == pos) || !(scan->mov == mov) || scan->maxVel != maxVel)
             scan = std::make_unique<eng::TimeNeededScan>(pos, mov, maxVel);
-        const eng::TimeNeeded c = scan->Get(target, precise, maxTime);
+        eng::TimeNeeded c = a;
+        scan->Unreachable(target, precise, maxTime, c);
         out[(size_t)i * 6 + 0] = a.usual;
         out[(size_t)i * 6 + 1] = a.optimistic;
         out[(size_t)i * 6 + 2] = b.usual;

@@ -161,10 +161,10 @@ def test_set_state_refuses_another_scenario(reference_library, host_library):
 
 
 def test_time_walk_matches_the_direct_estimate(host_library):
-    """The time-to-target estimate along the precomputed walk, and the possession scan's shortcut
-    for targets the walk cannot reach, equal GRF's direct loop (ai_time.h:102-409) on random
-    players, movements, targets and time limits, near and far. Each player takes eight targets in
-    a row, as a possession scan does, and a third of the targets sit within a metre of the
+    """The time-to-target estimate along the precomputed walk, and the shortcut for targets the walk
+    cannot reach, both as the AI's chase of the ball asks them, equal GRF's direct loop
+    (ai_time.h:102-409) on random players, movements, targets and time limits, near and far. Each
+    player takes eight targets in a row, as a chase does, and a third of the targets sit within a metre of the
     shortcut's bound."""
     lib = ctypes.CDLL(host_library)
     rng = np.random.default_rng(5)
