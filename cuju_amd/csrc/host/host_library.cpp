@@ -207,6 +207,103 @@ extern "C" __attribute__((visibility("default"))) void cuju_debug_reached(const 
     }
 }
 
+// The predictions of `count` flights, each from a position, a momentum and a rotation per ms (10
+// values): by the engine, then with every stage of every step run; 400 positions each.
+extern "C" __attribute__((visibility("default"))) void cuju_debug_flight(const float *cases, int count, float *out, float *full) {
+    auto ball = std::make_unique<eng::Ball>();
+    for (int i = 0; i < count; i++) {
+        const float *q = cases + (size_t)i * 10;
+        memset(ball.get(), 0, sizeof(*ball));
+        ball->positionBuffer = eng::Vec3(q[0], q[1], q[2]);
+        ball->momentum = eng::Vec3(q[3], q[4], q[5]);
+        ball->rotationPerMs = eng::Quat(q[6], q[7], q[8], q[9]);
+        ball->orientationBuffer = eng::Quat(0, 0, 0, 1);
+        eng::BallFlight f;
+        f.pos = ball->positionBuffer;
+        f.mom = ball->momentum;
+        f.rot = ball->rotationPerMs;
+        eng::BallCalculatePrediction(*ball, false);
+        memcpy(out + (size_t)i * 1200, ball->predictions, 1200 * sizeof(float));
+        for (int k = 0; k < 400; k++) {
+            memcpy(full + (size_t)i * 1200 + 3 * k, &f.pos, sizeof(f.pos));
+            eng::BallFlight::Contact contact = f.Land();
+            contact.grass = eng::libm::PowfPos(contact.depth, 0.7f);
+            if (f.InGrass()) f.RubGrass(contact);
+            if (k == 0) f.HitFrame();
+            if (f.InGrass()) f.Roll(contact);
+            f.Swerve();
+            f.pos += f.mom * eng::BallFlight::kDt;
+        }
+    }
+}
+
+// The pairs of `n` players in the order of the contact search: i and j of each.
+extern "C" __attribute__((visibility("default"))) void cuju_debug_pairs(int n, int *out) {
+    for (int q = 0; q < n * (n - 1) / 2; q++) eng::PairAt(q, n, out[2 * q], out[2 * q + 1]);
+}
+
+// Team queries on a state with the players put at `positions`: the `count` active players of `team`
+// closest to `at` (its first 11 entries of `out`), then the opponents by danger (11 entries) with
+// their factors. Returns their numbers, closest + 100 * opponents, or -1; `team` of each player is
+// left in `teams` (-1 for one that is not active).
+extern "C" __attribute__((visibility("default"))) int cuju_debug_team_queries(const char *bytes, unsigned long long size,
+                                                                                const float *positions, int team, const float *at, int count,
+                                                                                int *out, float *factors, int *teams) {
+    try {
+        auto w = std::make_unique<eng::World>();
+        auto scratch = std::make_unique<eng::Scratch>();
+        eng::host::StateCodec codec;
+        if (!codec.Load(std::string(bytes, size), *w)) return -1;
+        eng::InitializePlayerTeams(*w);
+        eng::Ctx c{};
+        c.ws = scratch.get();
+        for (int p = 0; p < eng::kPlayers; p++) teams[p] = -1;
+        for (int p = 0; p < w->match.playerCount; p++) {
+            eng::Sp(*w, p).position = eng::Vec3(positions[3 * p], positions[3 * p + 1], positions[3 * p + 2]);
+            if (w->roster.active[p]) teams[p] = w->playerTeamID[p];
+        }
+        const eng::PlayerRanking closest =
+            eng::GetClosestPlayers(*w, c, team, eng::Vec3(at[0], at[1], at[2]), false, (unsigned)count, false);
+        for (int i = 0; i < closest.count; i++) out[i] = closest[i];
+        eng::RankOpponentsByDanger(*w, c, team);
+        const auto &ranked = eng::TeamByID(*w, team).ai.tacticalOpponents;
+        for (int i = 0; i < ranked.count; i++) {
+            out[11 + i] = ranked[i].player;
+            factors[i] = ranked[i].dangerFactor;
+        }
+        return closest.count + 100 * ranked.count;
+    } catch (...) {
+        return -1;
+    }
+}
+
+// The body parts of every person of a bundle's template, each placed down its own path and in a walk
+// over the whole body: the numbers of parts compared and of those that differ in a bit.
+extern "C" __attribute__((visibility("default"))) int cuju_debug_placed_parts(const char *path, int *different) {
+    try {
+        const auto bundle = eng::host::LoadBundle(path);
+        const eng::host::Variant &v = bundle->variants[0];
+        int compared = 0;
+        *different = 0;
+        for (int person = 0; person < (int)v.skeletons.size(); person++) {
+            const eng::Skeleton &sk = v.skeletons[person];
+            const eng::NodeState *nodes = eng::HumanoidAt(*v.world, person).nodes;
+            eng::Transform placed[eng::kHumanoidNodes];
+            eng::WorldTransforms(sk, nodes, placed);
+            for (int n = 0; n < sk.nodeCount; n++)
+                for (int g = 0; g < sk.nodes[n].geometryCount; g++) {
+                    const eng::WorldGeometry a = eng::PlacedPart(sk, nodes, n, g);
+                    const eng::WorldGeometry b = eng::PlacedGeometry(sk.nodes[n].geometries[g], placed[n]);
+                    *different += memcmp(&a, &b, sizeof(a)) != 0;
+                    compared++;
+                }
+        }
+        return compared;
+    } catch (...) {
+        return -1;
+    }
+}
+
 // The bytes of one environment's blocks in device memory: World, EnvCore, EnvSlot and Scratch. The
 // engine's structs have the same layout on the host and the device.
 extern "C" __attribute__((visibility("default"))) void cuju_debug_layout(unsigned long long *out) {

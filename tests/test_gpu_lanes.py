@@ -24,7 +24,7 @@ def host(x):
 @pytest.mark.parametrize('matches,lanes', [(32, 2), (16, 4), (8, 8), (3, 16), (2, 32), (1, 64)])
 def test_every_width_plays_as_one_lane(assets, agents, steps, matches, lanes, host_library, monkeypatch):
     import cuju_amd
-    environments = 33  # a last wavefront that is not full, at every width but 64
+    environments = 35  # a last wavefront that is not full, at every width but 64 (one match fills one)
     theirs = ref.ReferenceBatch(assets, environment_count=environments, seed=9, threads=0, library_path=host_library)
     monkeypatch.setenv('CUJU_AMD_MATCHES', str(matches))
     monkeypatch.setenv('CUJU_AMD_LANES', str(lanes))

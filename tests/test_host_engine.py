@@ -11,7 +11,7 @@ import numpy as np
 import pytest
 
 import libm_cases
-from conftest import ROOT, digest_actions, play, short_cases
+from conftest import DATA, ROOT, digest_actions, play, short_cases
 from oracle import ref
 from oracle.ref import ReferenceBatch
 
@@ -236,6 +236,100 @@ def test_reach_in_closed_form_is_the_walk(slowest, fastest, host_library):
     if fastest <= 12:
         assert decided[np.linalg.norm(target - pos, axis=1) < 16].mean() > 0.5
         assert (out[decided, 0] == 1).any() and (out[decided, 0] == 0).any()
+
+
+def test_flight_steps_that_move_the_height_alone_are_the_full_steps(host_library):
+    """A flight without horizontal momentum and rotation steps its height alone (ball.h, OnlyHeight):
+    every prediction equals, bit for bit, the flight in which each step runs every stage
+    (ball.h:23-348). Drops, lofts and balls at rest, with zeros of either sign in every place, on the
+    centre lines too, and flights that do move, which must not take the short way."""
+    lib = ctypes.CDLL(host_library)
+    rng = np.random.default_rng(23)
+    n = 4000
+    signed = lambda size: np.where(rng.uniform(size=size) < 0.5, 0.0, -0.0)  # noqa: E731
+    cases = np.zeros((n, 10), dtype=np.float32)
+    cases[:, 0] = np.where(rng.uniform(size=n) < 0.2, signed(n), rng.uniform(-60, 60, n))
+    cases[:, 1] = np.where(rng.uniform(size=n) < 0.2, signed(n), rng.uniform(-40, 40, n))
+    cases[:, 2] = rng.choice([0.0, 0.1, 0.11, 0.12, 0.134, 0.135, 0.2, 1.0, 2.5, 12.0], n) + rng.choice([0.0, 1e-3], n)
+    cases[:, 3], cases[:, 4] = signed(n), signed(n)
+    cases[:, 5] = np.where(rng.uniform(size=n) < 0.3, signed(n), rng.uniform(-30, 30, n))
+    for k in range(3):
+        cases[:, 6 + k] = signed(n)
+    cases[:, 9] = 1.0
+    moves = rng.uniform(size=n) < 0.25
+    cases[moves, 3:5] = rng.uniform(-8, 8, (moves.sum(), 2))
+    spins = rng.uniform(size=n) < 0.25
+    half = rng.uniform(-0.03, 0.03, spins.sum())
+    axis = rng.normal(size=(spins.sum(), 3))
+    axis /= np.linalg.norm(axis, axis=1, keepdims=True)
+    cases[spins, 6:9], cases[spins, 9] = np.sin(half)[:, None] * axis, np.cos(half)
+    out, full = (np.zeros((n, 400, 3), dtype=np.float32) for _ in range(2))
+    lib.cuju_debug_flight(ctypes.c_void_p(cases.ctypes.data), n, ctypes.c_void_p(out.ctypes.data),
+                          ctypes.c_void_p(full.ctypes.data))
+    wrong = np.flatnonzero((out.view(np.uint32) != full.view(np.uint32)).any(axis=(1, 2)))
+    assert wrong.size == 0, f'{wrong.size} flights differ, the first from {cases[wrong[0]]}'
+    assert (out[:, -1, :2] == out[:, 0, :2]).all(axis=1).sum() > n // 2
+
+
+def test_contact_pairs_are_those_of_the_double_loop(host_library):
+    lib = ctypes.CDLL(host_library)
+    for n in range(23):
+        want = [(i, j) for i in range(n) for j in range(i + 1, n)]
+        out = np.zeros((max(1, len(want)), 2), dtype=np.int32)
+        lib.cuju_debug_pairs(n, ctypes.c_void_p(out.ctypes.data))
+        assert [tuple(pair) for pair in out[:len(want)].tolist()] == want
+
+
+def test_body_parts_placed_alone_are_those_of_the_whole_body(host_library):
+    lib = ctypes.CDLL(host_library)
+    different = ctypes.c_int()
+    path = os.path.join(DATA, 'assets', '11_vs_11_hard_stochastic_l0_r0.cjb')
+    compared = lib.cuju_debug_placed_parts(path.encode(), ctypes.byref(different))
+    assert compared > 25 * 10 and different.value == 0
+
+
+def _inserted(items, before):
+    """GRF's insertion sort: an item moves down while it comes before the one under it."""
+    order = []
+    for item in items:
+        at = len(order)
+        while at > 0 and before(item, order[at - 1]):
+            at -= 1
+        order.insert(at, item)
+    return order
+
+
+@pytest.mark.parametrize('spoiled', [0, 1, 3, 11])
+def test_team_queries_order_as_grf_with_nan_and_ties(spoiled, host_library):
+    """The closest players of a team and its opponents by danger, in the order GRF's insertion sorts
+    give (team_process.h:20-130, team_ai.h:15-533): ties in state order, and a distance that is NaN, before
+    which nothing moves, where the insertions leave it."""
+    lib = ctypes.CDLL(host_library)
+    batch = ReferenceBatch('11_vs_11_stochastic_l1_r0', environment_count=1, seed=3, library_path=host_library)
+    batch.reset()
+    state = batch.raw_state(0)[0]
+    batch.close()
+    rng = np.random.default_rng(spoiled)
+    for trial in range(60):
+        positions = rng.integers(-6, 7, (22, 3)).astype(np.float32)  # whole metres: many ties
+        positions[:, 2] = 0
+        positions[rng.permutation(22)[:spoiled], rng.integers(0, 3)] = np.nan
+        at = np.array([0.0, 0.0, 0.0], dtype=np.float32)
+        team, count = trial % 2, int(rng.integers(1, 12))
+        out, teams = np.full(22, -1, dtype=np.int32), np.zeros(22, dtype=np.int32)
+        factors = np.zeros(11, dtype=np.float32)
+        got = lib.cuju_debug_team_queries(state, ctypes.c_ulonglong(len(state)), ctypes.c_void_p(positions.ctypes.data), team,
+                                          ctypes.c_void_p(at.ctypes.data), count, ctypes.c_void_p(out.ctypes.data),
+                                          ctypes.c_void_p(factors.ctypes.data), ctypes.c_void_p(teams.ctypes.data))
+        assert got == count + 1100
+        d = np.linalg.norm(positions.astype(np.float64), axis=1).astype(np.float32)
+        own = [p for p in range(22) if teams[p] == team]
+        assert out[:count].tolist() == _inserted(own, lambda a, b: d[a] < d[b])[:count]
+        factor = dict(zip(out[11:].tolist(), factors.tolist()))
+        opponents = [p for p in range(22) if teams[p] == 1 - team]
+        assert sorted(factor) == opponents
+        assert out[11:].tolist() == _inserted(opponents, lambda a, b: factor[a] > factor[b])
+        assert [bool(np.isnan(factor[p])) for p in opponents] == [bool(np.isnan(positions[p]).any()) for p in opponents]
 
 
 def test_device_time_bias_rounds_as_the_division():
