@@ -56,16 +56,16 @@ CPU_SAMPLE = 2048
 # (each scaled by what the counter reads for a 1 GiB device copy), keyed by (workload,
 # environments, warm-up steps, timed steps, rounds): the window of launches the profile averaged.
 MEASURED_TRAFFIC = {
-    (1, 64, 5, 20, 3): (75848861, 'profiles/step_kernel_5v5_64_driver_window.md'),
-    (2, 4096, 5, 20, 3): (65277143487, 'profiles/step_kernel_11v11_4096_driver_window.md'),
-    (3, 16384, 5, 20, 3): (191055945597, 'profiles/step_kernel_11v11_hard_16384_driver_window.md'),
-    (4, 8192, 5, 20, 3): (109599148534, 'profiles/step_kernel_11v11_selfplay_stacked_8192_driver_window.md'),
-    (5, 32768, 5, 20, 3): (185300503006, 'profiles/step_kernel_mixed_32768_driver_window.md'),
-    (1, 64, 100, 30, 3): (77848709, 'profiles/step_kernel_5v5_64.md'),
-    (2, 4096, 100, 30, 3): (65060719838, 'profiles/step_kernel_11v11_4096.md'),
-    (3, 16384, 100, 30, 3): (193424500413, 'profiles/step_kernel_11v11_hard_16384.md'),
-    (4, 8192, 100, 30, 3): (110546197410, 'profiles/step_kernel_11v11_selfplay_stacked_8192.md'),
-    (5, 32768, 100, 30, 3): (192416493757, 'profiles/step_kernel_mixed_32768.md'),
+    (1, 64, 5, 20, 3): (58486271, 'profiles/step_kernel_5v5_64_driver_window.md'),
+    (2, 4096, 5, 20, 3): (40378637207, 'profiles/step_kernel_11v11_4096_driver_window.md'),
+    (3, 16384, 5, 20, 3): (161496415820, 'profiles/step_kernel_11v11_hard_16384_driver_window.md'),
+    (4, 8192, 5, 20, 3): (78816826397, 'profiles/step_kernel_11v11_selfplay_stacked_8192_driver_window.md'),
+    (5, 32768, 5, 20, 3): (160893387506, 'profiles/step_kernel_mixed_32768_driver_window.md'),
+    (1, 64, 100, 30, 3): (63559722, 'profiles/step_kernel_5v5_64.md'),
+    (2, 4096, 100, 30, 3): (41516407262, 'profiles/step_kernel_11v11_4096.md'),
+    (3, 16384, 100, 30, 3): (166952332485, 'profiles/step_kernel_11v11_hard_16384.md'),
+    (4, 8192, 100, 30, 3): (81099801649, 'profiles/step_kernel_11v11_selfplay_stacked_8192.md'),
+    (5, 32768, 100, 30, 3): (167028365294, 'profiles/step_kernel_mixed_32768.md'),
 }
 
 
