@@ -82,8 +82,8 @@ struct SinCos {
 // second coefficient set is the first with the cosine's coefficients negated, which negates every
 // step of its polynomial exactly, and the sine's polynomial is odd. The coefficients are constants
 // in the code, not loads. Measured together with atan2f below, ms per step against the routines'
-// branches with the sets in LDS: one match of 64 lanes 13.0 -> 12.7, 16,384 of 8 lanes 122.9 -> 120.7,
-// the mixed 32,768 of 4 lanes 137.8 -> 134.0.
+// branches with the sets in LDS: one match of 64 lanes 12.2 -> 12.0, 16,384 of 8 lanes 116.3 -> 112.8,
+// the mixed 32,768 of 4 lanes 127.1 -> 123.1.
 struct ReducedAngle {
     double x, x2;
     int n, turn;  // quarter turns modulo 4, for the choice of the polynomial and for the signs

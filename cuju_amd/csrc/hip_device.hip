@@ -268,11 +268,16 @@ std::unique_ptr<Device> MakeHipDevice32(int matches);
 std::unique_ptr<Device> MakeHipDevice64(int matches);
 
 // Two wavefronts for each SIMD where the batch allows it: the matches of a wavefront are the
-// environments over the wavefront slots, 1 to 32, and the group is the widest of 64, 32, 16, 8, 4
-// or 2 lanes that those matches leave room for in 64 (measured on an MI355X: one match of 64 lanes
-// steps 64 environments of 5-a-side in 17.7 ms at the median against 18.5 at 16 lanes; two of 32
-// step 4,096 of 11-a-side in 88.5 ms against 90.4 at 2 x 16). CUJU_AMD_MATCHES sets the matches of
-// a wavefront instead.
+// environments over the wavefront slots, 1 to 32, and the group is the widest of 64, 32, 16, 8, 4 or 2
+// lanes that those matches leave room for in 64. Measured on an MI355X, ms per step after 40 steps, two
+// seeds (one from 16,384 on): 64 environments of 5-a-side 8.3 and 9.6 with one match of 64 lanes, 8.9
+// and 10.5 of 32, 9.7 and 11.3 of 16; 4,096 of 11-a-side 37.2 and 38.3 with two of 32, 41.0 and 42.6
+// with two of 16, 40.5 and 40.7 with one of 64 in two rounds; 8,192 58.6 and 58.9 with four of 16, 63.2
+// and 63.0 with two of 32; 16,384 103.1 with eight of 8, 111.2 with four of 16; the mixed 32,768 126.5
+// with sixteen of 4, 134.0 with eight of 8. Just past the 2,048 slots single matches in two rounds
+// would be quicker (2,100: 27.7 and 25.6 against 30.9 and 30.1; 2,500: 31.8 and 30.5 against 32.0 and
+// 31.9; 3,000: 35.2 and 35.6 against 34.3 and 34.0). CUJU_AMD_MATCHES sets the matches of a wavefront
+// instead.
 std::unique_ptr<Device> MakeLibraryDevice(int, int environments) {
     int device = 0, units = 0;
     Check(hipGetDevice(&device), "hipGetDevice");
