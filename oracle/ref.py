@@ -5,7 +5,7 @@ This module is the oracle's entry point for the whole GRF step. It loads
 (`src/cuju_cpu.cpp`, `src/environment_state.cpp`), and drives it through the reference C ABI
 (`src/environment_api.h:47-95` for the configuration, `:252-317` for reset and step, `:367-388` for
 `get_state`). Only tests, the smoke check and the CPU-baseline leg of the benchmark may import it,
-and only as the checker or the timed baseline; the product never loads it.
+and only as the oracle or the timed baseline; the product never loads it.
 
 The digest follows the reference self-check (`tests/conftest.py:60-98`): SHA-256 over every
 observation, reward and done flag of every step, then every environment's `get_state` bytes, which
